@@ -30,13 +30,9 @@ static __device__ __align__(256) unsigned char scratch[SPK_NOALLOC_SCRATCH_BYTES
 
 namespace spk {
 template <typename T, int R, int V>
-__global__ void k_solve(const Inst<T> *, Out *, int, double, int, int);
+__global__ void k_solve(const Inst<T> *, Out *, int, int);
 template <typename T, int R, int V>
-__global__ void k_debug(const Inst<T> *, Out *, int, int, int, int);
-__global__ void k_f32_to_f64(const float *, double *, long);
-__global__ void k_f64_to_f32(const double *, float *, long);
-template <typename T>
-__global__ void k_fill(T *, T, long);
+__global__ void k_debug(const Inst<T> *, Out *, int, int, int);
 template <typename T>
 __global__ void k_lane_solve(const LaneInst<T> *, Out *);
 template <typename T>
@@ -65,6 +61,20 @@ template <typename S, typename D>
 __global__ void k_interleave(const S *, long, D *, long, int, long);
 template <typename S, typename D>
 __global__ void k_deinterleave(const S *, long, D *, long, long, int);
+
+// Elementwise conversions used by the FP32-bulk / FP64-polish path.
+__global__ void k_f32_to_f64(const float *in, double *out, long n) {
+    for (long k = blockIdx.x * (long) blockDim.x + threadIdx.x; k < n; k += (long) gridDim.x * blockDim.x) out[k] = in[k];
+}
+
+__global__ void k_f64_to_f32(const double *in, float *out, long n) {
+    for (long k = blockIdx.x * (long) blockDim.x + threadIdx.x; k < n; k += (long) gridDim.x * blockDim.x) out[k] = (float) in[k];
+}
+
+template <typename T>
+__global__ void k_fill(T *p, T v, long n) {
+    for (long k = blockIdx.x * (long) blockDim.x + threadIdx.x; k < n; k += (long) gridDim.x * blockDim.x) p[k] = v;
+}
 
 // One instance's column of a block-interleaved region (`rows` rows, blocks of w instances) copied
 // to a contiguous row (toRow 1) or back from one (toRow 0).
@@ -409,23 +419,10 @@ int chunkClass(const spk_batch *b) {
     return mx <= 64 ? 1 : 4;
 }
 
-// Ints of per-node index and tree arrays staged in LDS by the kernels (0 when they do not
-// fit in the budget, then the kernels read them from global memory).
-int ldsPoolInts(const spk_batch *b) {
-    int mx = 0;
-    for (auto *p : b->probs) {
-        const HostProblem &h = p->hp;
-        const int need = 12 * h.N + 15 * h.nl + 7 * h.nlf + 2 * h.S;
-        mx = std::max(mx, need);
-    }
-    const int budget = 48 * 1024 / 4;
-    return mx <= budget ? mx : 0;
-}
-
 // Workgroups that cooperate on one instance: 1 for a batch of several instances and by default;
 // for a single instance the count set by spk_batch_set_workgroups.  Bounded by what can be
 // co-resident, which a cooperative launch requires.
-int gridWorkgroups(spk_batch *b, const void *kernel, int bs, size_t shm) {
+int gridWorkgroups(spk_batch *b, const void *kernel, int bs) {
     if (b->count != 1 || b->wgs <= 1) return 1;
     const int dev = b->ctx->device;
     int coop = 0, cus = 0, perCU = 0;
@@ -435,7 +432,7 @@ int gridWorkgroups(spk_batch *b, const void *kernel, int bs, size_t shm) {
         return 1;
     }
     check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "device attribute");
-    check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, kernel, bs, shm), "occupancy");
+    check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, kernel, bs, 0), "occupancy");
     const int most = std::min(spk::GRID_MAXWG, cus * perCU);
     if (most < 1) throw std::runtime_error("the solve kernel does not fit on a compute unit");
     if (b->wgs > most)
@@ -445,16 +442,16 @@ int gridWorkgroups(spk_batch *b, const void *kernel, int bs, size_t shm) {
 }
 
 template <typename K, typename... A>
-void launchMaybeGrid(spk_batch *b, K kernel, int bs, size_t shm, A... args) {
+void launchMaybeGrid(spk_batch *b, K kernel, int bs, A... args) {
     const void *fn = reinterpret_cast<const void *>(kernel);
-    const int g = gridWorkgroups(b, fn, bs, shm);
+    const int g = gridWorkgroups(b, fn, bs);
     int grid = g > 1 ? 1 : 0;
     if (!grid) {
-        hipLaunchKernelGGL(kernel, dim3(b->count), dim3(bs), shm, b->ctx->stream, args..., grid);
+        hipLaunchKernelGGL(kernel, dim3(b->count), dim3(bs), 0, b->ctx->stream, args..., grid);
         return;
     }
     void *argv[] = {static_cast<void *>(&args)..., static_cast<void *>(&grid)};
-    const hipError_t e = hipLaunchCooperativeKernel(fn, dim3(g), dim3(bs), argv, (unsigned) shm, b->ctx->stream);
+    const hipError_t e = hipLaunchCooperativeKernel(fn, dim3(g), dim3(bs), argv, 0, b->ctx->stream);
     // a refused launch queues nothing: read the error back so a later launch check does not see it
     if (e != hipSuccess) {
         (void) hipGetLastError();
@@ -466,18 +463,15 @@ void launchMaybeGrid(spk_batch *b, K kernel, int bs, size_t shm, A... args) {
 template <typename T>
 void launchKernel(spk_batch *b, int bs, bool debug, int op, const void *insDev = nullptr) {
     const int cls = chunkClass(b);
-    const int pool = ldsPoolInts(b);
-    const size_t shm = (size_t) pool * sizeof(int);
     auto *ins = static_cast<const spk::Inst<T> *>(insDev ? insDev : b->dInst.p);
     auto *outs = static_cast<spk::Out *>(b->dOut.p);
     const int count = b->count;
-    const double tick = b->ctx->tickRateHz;
     if (!debug) {
-        if (cls == 1) launchMaybeGrid(b, spk::k_solve<T, 1, 1>, bs, shm, ins, outs, count, tick, pool);
-        else launchMaybeGrid(b, spk::k_solve<T, 4, 4>, bs, shm, ins, outs, count, tick, pool);
+        if (cls == 1) launchMaybeGrid(b, spk::k_solve<T, 1, 1>, bs, ins, outs, count);
+        else launchMaybeGrid(b, spk::k_solve<T, 4, 4>, bs, ins, outs, count);
     } else {
-        if (cls == 1) launchMaybeGrid(b, spk::k_debug<T, 1, 1>, bs, shm, ins, outs, count, op, pool);
-        else launchMaybeGrid(b, spk::k_debug<T, 4, 4>, bs, shm, ins, outs, count, op, pool);
+        if (cls == 1) launchMaybeGrid(b, spk::k_debug<T, 1, 1>, bs, ins, outs, count, op);
+        else launchMaybeGrid(b, spk::k_debug<T, 4, 4>, bs, ins, outs, count, op);
     }
 }
 

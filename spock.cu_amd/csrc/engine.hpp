@@ -4,14 +4,44 @@
 
 namespace spk {
 
-// Per-node factor table on the device: entry for node n starts at data + idx[n] * rows * cols.
+// Per-node factor table on the device: entry for node n starts at data + idx[n] * rows * cols (tab()).
 template <typename T>
 struct DTab {
     const T *data = nullptr;
     const int *idx = nullptr;
     int rows = 0, cols = 0;
-    __device__ __forceinline__ const T *at(int n) const { return data + (size_t) idx[n] * rows * cols; }
 };
+
+// A pointer every lane holds the same value of, moved to scalar registers: loads through it
+// become scalar loads (needed inside non-inlined functions, whose arguments arrive per lane).
+template <typename T>
+__device__ __forceinline__ T *uniformPtr(T *p) {
+    const unsigned long long v = reinterpret_cast<unsigned long long>(p);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned) v);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned) (v >> 32));
+    return reinterpret_cast<T *>(((unsigned long long) hi << 32) | lo);
+}
+
+// Constant address space: the descriptor, the tree arrays and the factor tables are never written
+// while a solve runs, and wave-uniform reads through such pointers become scalar loads.
+#define SPK_CONST __attribute__((address_space(4)))
+#define SPK_GLOBAL __attribute__((address_space(1)))
+#define SPK_LDS __attribute__((address_space(3)))
+template <typename T>
+using CP = const SPK_CONST T *;
+template <typename T>
+using GP = SPK_GLOBAL T *;
+
+template <typename T>
+__device__ __forceinline__ CP<T> cst(const T *p) {
+    return (CP<T>) p;
+}
+
+// Node n's entry of a per-node table, as a constant-space pointer.
+template <typename T>
+__device__ __forceinline__ CP<T> tab(const SPK_CONST DTab<T> &t, int n) {
+    return cst(t.data) + (size_t) cst(t.idx)[n] * t.rows * t.cols;
+}
 
 // One solve instance: problem sizes, device tables, state buffers and options.
 template <typename T>

@@ -51,28 +51,40 @@ __device__ __forceinline__ T waveMax(T v) {
     return v;
 }
 
+// The descriptor is read through the constant address space (scalar loads, kept in scalar
+// registers), the state through the global one: with the descriptor in LDS behind generic pointers
+// every field was a flat load per lane, waited for on its own, and every branch on one an exec mask.
+// Together with the unconditional loads and the shared code of mvChunk: 0.85 -> 0.33 ms per
+// application of T on the 229-node FP64 instance with 32 workgroups, 0.25 -> 0.08 ms on the 31-node one.
+template <typename T>
+using IP = const SPK_CONST Inst<T> &;
+
+template <typename T>
+__device__ __forceinline__ GP<T> glb(T *p) {
+    return (GP<T>) uniformPtr(p);
+}
+
 // Work distribution of a thread: tid/nt and wave/nw index the threads and waves that share one
 // instance (the workgroup, or the whole grid in grid mode); ltid/lw/lnw are workgroup-local.
 struct Tc {
-    int lane, wave, nw, tid, nt;
+    unsigned lane;
+    int wave, nw, tid, nt;
     int ltid, lw, lnw;
     int grid;
-    void *gpart;      // grid mode: two buffers of GRID_MAXK x GRID_MAXWG reduction partials
-    mutable int seq;  // reductions done so far; selects the partials buffer
+    void *gpart;  // grid mode: two buffers of GRID_MAXK x GRID_MAXWG reduction partials
 };
 
 __device__ __forceinline__ Tc threadCtx(int grid = 0, void *gpart = nullptr) {
     Tc c;
     c.ltid = threadIdx.x;
-    c.lw = c.ltid >> 6;
+    c.lw = __builtin_amdgcn_readfirstlane(c.ltid >> 6);
     c.lnw = blockDim.x >> 6;
-    c.grid = grid;
+    c.grid = __builtin_amdgcn_readfirstlane(grid);
     c.gpart = gpart;
-    c.seq = 0;
-    c.tid = grid ? (int) (blockIdx.x * blockDim.x + threadIdx.x) : c.ltid;
-    c.nt = grid ? (int) (gridDim.x * blockDim.x) : (int) blockDim.x;
-    c.lane = c.tid & 63;
-    c.wave = c.tid >> 6;
+    c.tid = c.grid ? (int) (blockIdx.x * blockDim.x + threadIdx.x) : c.ltid;
+    c.nt = c.grid ? (int) (gridDim.x * blockDim.x) : (int) blockDim.x;
+    c.lane = threadIdx.x & 63;
+    c.wave = c.grid ? (int) blockIdx.x * c.lnw + c.lw : c.lw;
     c.nw = c.nt >> 6;
     return c;
 }
@@ -83,6 +95,12 @@ __device__ __forceinline__ void sync(const Tc &c) {
     else __syncthreads();
 }
 
+// Grid reductions done so far by this workgroup; selects the partials buffer.
+__device__ __forceinline__ SPK_LDS int *gridSeq() {
+    __shared__ int seq;
+    return (SPK_LDS int *) &seq;
+}
+
 // Grid mode: combine the workgroup values v[0..K) of every workgroup.  Each workgroup publishes its
 // values, then every wave reads all partials lane-strided and reduces them with the same shuffle
 // tree, so all threads of the grid hold bitwise identical results.  Two partial buffers alternate:
@@ -91,12 +109,13 @@ __device__ __forceinline__ void sync(const Tc &c) {
 template <typename T, int K, bool MAX>
 __device__ __forceinline__ void gridCombine(T (&v)[K], const Tc &c) {
     static_assert(K <= GRID_MAXK, "too many values per grid reduction");
-    T *part = static_cast<T *>(c.gpart) + (size_t) (c.seq & 1) * GRID_MAXK * GRID_MAXWG;
-    c.seq++;
+    const int seq = *gridSeq();  // advanced below, behind the grid barrier; read again behind a block barrier
+    T *part = static_cast<T *>(c.gpart) + (size_t) (seq & 1) * GRID_MAXK * GRID_MAXWG;
     if (c.ltid == 0)
 #pragma unroll
         for (int i = 0; i < K; i++) part[i * GRID_MAXWG + blockIdx.x] = v[i];
     cooperative_groups::this_grid().sync();
+    if (c.ltid == 0) *gridSeq() = seq + 1;
     const int nb = gridDim.x;
 #pragma unroll
     for (int i = 0; i < K; i++) {
@@ -133,54 +152,104 @@ __device__ __forceinline__ void zero(T (&a)[K]) {
 
 // v[c] holds element lane + 64 c of a vector of length len (0 beyond)
 template <typename T, int V, typename F>
-__device__ __forceinline__ void loadV(T (&v)[V], int len, int lane, F f) {
+__device__ __forceinline__ void loadV(T (&v)[V], int len, unsigned lane, F f) {
 #pragma unroll
     for (int c = 0; c < V; c++) {
-        const int k = lane + 64 * c;
-        v[c] = (k < len) ? f(k) : T(0);
+        const unsigned k = lane + 64 * c;
+        v[c] = T(0);
+        if (64 * c < len && k < (unsigned) len) v[c] = f(k);
     }
 }
 
-template <typename T, int V>
-__device__ __forceinline__ void loadPtr(T (&v)[V], const T *p, int len, int lane) {
-    loadV(v, len, lane, [&](int k) { return p[k]; });
+template <typename T, int V, typename P>
+__device__ __forceinline__ void loadPtr(T (&v)[V], P p, int len, unsigned lane) {
+    loadV(v, len, lane, [&](unsigned k) -> T { return p[k]; });
 }
 
-// acc[rc] (row lane + 64 rc) += sum_{c < cols} M[row + c * ld] * v(c).
-// All columns of a 64-column chunk (32 per block in FP64) are requested before any is
-// consumed, so a matvec costs one or two memory round trips instead of one per column;
-// out-of-range columns load 0 and v holds 0 beyond its length.
-template <typename T, int R, int V>
-__device__ __forceinline__ void mvAcc(T (&acc)[R], const T *M, int rows, int ld, int cols, const T (&v)[V], int lane) {
-    constexpr int U = (sizeof(T) == 8 ? 32 : 64) / R;
+// acc[rc] (row lane + 64 rc) += sum_{c < n} M[row + c * ld] * v(c) in column order, n <= U columns,
+// RR row chunks.  All columns are requested before any is consumed, so this costs one memory round
+// trip.  Loads are unconditional: rows past the end repeat the last row (outputs nobody reads),
+// columns past the end repeat the last column against v = 0, and whole blocks of 8 columns past the
+// end are skipped by scalar branches.
+template <typename T, int RR, int U, int R>
+__device__ __forceinline__ void mvBlock(T (&acc)[R], CP<T> M, const unsigned (&row)[RR], int ld, int n, T v, int v0) {
+    T m[U][RR];
 #pragma unroll
-    for (int vc = 0; vc < V; vc++) {
-        if (64 * vc >= cols) break;
-        const int cend = min(64, cols - 64 * vc);
-        const T *base = M + (size_t) (64 * vc) * ld;
-#pragma unroll 1
-        for (int c0 = 0; c0 < cend; c0 += U) {
-            T m[U][R];
+    for (int b = 0; b < U; b += 8) {
+        if (b < n) {
+            CP<T> col = M + (size_t) b * ld;
 #pragma unroll
-            for (int u = 0; u < U; u++)
+            for (int u = b; u < b + 8; u++) {
 #pragma unroll
-                for (int rc = 0; rc < R; rc++) {
-                    const int r = lane + 64 * rc;
-                    m[u][rc] = (c0 + u < cend && r < rows) ? base[(size_t) (c0 + u) * ld + r] : T(0);
-                }
+                for (int rc = 0; rc < RR; rc++) m[u][rc] = col[row[rc]];
+                col += u + 1 < n ? ld : 0;
+            }
+        }
+    }
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                const T xc = bcastLane(v[vc], (c0 + u) & 63);
+    for (int b = 0; b < U; b += 8) {
+        if (b < n) {
 #pragma unroll
-                for (int rc = 0; rc < R; rc++) acc[rc] += m[u][rc] * xc;
+            for (int u = b; u < b + 8; u++) {
+                const T xc = bcastLane(v, v0 + u);
+#pragma unroll
+                for (int rc = 0; rc < RR; rc++) acc[rc] += m[u][rc] * xc;
             }
         }
     }
 }
 
+// One 64-column chunk (cols <= 64) of RR row chunks.  Never inlined: a product is a few KB of
+// straight-line code, and with a copy at each of its call sites the phases of a solve missed the
+// instruction cache all the time (229-node FP64 instance, 32 workgroups: 1.6 ms of tree sweeps per
+// application of T inlined, 0.28 ms called).
+template <typename T, int RR>
+struct RowVals {
+    T a[RR];
+};
+
+template <typename T, int RR>
+__device__ __noinline__ RowVals<T, RR> mvChunk(RowVals<T, RR> acc, const T *Mp, int rows, int ldIn, int colsIn, T v) {
+    constexpr int U = RR == 1 ? 64 : 64 / RR;  // up to 128 registers of matrix entries in FP64
+    CP<T> M = cst(uniformPtr(Mp));
+    const int ld = __builtin_amdgcn_readfirstlane(ldIn), cols = __builtin_amdgcn_readfirstlane(colsIn);
+    unsigned row[RR];
+#pragma unroll
+    for (int rc = 0; rc < RR; rc++) row[rc] = min((threadIdx.x & 63) + 64 * rc, (unsigned) rows - 1);
+#pragma unroll 1
+    for (int c0 = 0; c0 < cols; c0 += U) mvBlock<T, RR, U>(acc.a, M + (size_t) c0 * ld, row, ld, cols - c0, v, c0);
+    return acc;
+}
+
+template <typename T, int RR, int R, int V>
+__device__ __forceinline__ void mvRows(T (&acc)[R], CP<T> M, int rows, int ld, int cols, const T (&v)[V]) {
+    RowVals<T, RR> a;
+#pragma unroll
+    for (int rc = 0; rc < RR; rc++) a.a[rc] = acc[rc];
+#pragma unroll
+    for (int vc = 0; vc < V; vc++)
+        if (64 * vc < cols)
+            a = mvChunk<T, RR>(a, (const T *) (M + (size_t) (64 * vc) * ld), rows, ld, min(64, cols - 64 * vc), v[vc]);
+#pragma unroll
+    for (int rc = 0; rc < RR; rc++) acc[rc] = a.a[rc];
+}
+
+// acc[rc] (row lane + 64 rc) += sum_{c < cols} M[row + c * ld] * v(c), M column major, v 0 beyond
+// its length.
+template <typename T, int R, int V>
+__device__ __forceinline__ void mvAcc(T (&acc)[R], CP<T> M, int rows, int ld, int cols, const T (&v)[V], unsigned) {
+    if constexpr (R == 1) {
+        mvRows<T, 1>(acc, M, rows, ld, cols, v);
+    } else {
+        if (rows <= 64) mvRows<T, 1>(acc, M, rows, ld, cols, v);
+        else if (rows <= 128) mvRows<T, 2>(acc, M, rows, ld, cols, v);
+        else mvRows<T, 4>(acc, M, rows, ld, cols, v);
+    }
+}
+
 // Sum of K per-thread values over the workgroup, identical result in every thread.
 template <typename T, int K>
-__device__ __forceinline__ void blockSum(T (&v)[K], T *lds, const Tc &c) {
+__device__ __forceinline__ void blockSum(T (&v)[K], SPK_LDS T *lds, const Tc &c) {
 #pragma unroll
     for (int i = 0; i < K; i++) v[i] = waveSum(v[i]);
     if (c.lane == 0)
@@ -198,7 +267,7 @@ __device__ __forceinline__ void blockSum(T (&v)[K], T *lds, const Tc &c) {
 }
 
 template <typename T>
-__device__ __forceinline__ T blockMax(T v, T *lds, const Tc &c) {
+__device__ __forceinline__ T blockMax(T v, SPK_LDS T *lds, const Tc &c) {
     v = waveMax(v);
     if (c.lane == 0) lds[c.lw] = v;
     __syncthreads();
@@ -223,6 +292,16 @@ __device__ __forceinline__ T projBox(T v, T lb, T ub) {
     return v * T(1 - lower) * T(1 - upper) + lbi + ubi;
 }
 
+// f(rc, r) for every row r = lane + 64 rc < rows of this lane.
+template <int R, typename F>
+__device__ __forceinline__ void eachRow(int rows, unsigned lane, F f) {
+#pragma unroll
+    for (int rc = 0; rc < R; rc++) {
+        const unsigned r = lane + 64 * rc;
+        if (64 * rc < rows && r < (unsigned) rows) f(rc, r);
+    }
+}
+
 // ------------------------------------------------------------------ L* per node
 // src/operator.cuh:63-82; src/costs.cuh:162-195 (quadratic), :418-458 (quadratic+linear);
 // src/constraints.cuh:171-191 (rectangle), :265-286 (polyhedron).
@@ -235,7 +314,7 @@ struct AdjOut {
 };
 
 template <typename T, int R, int V>
-__device__ __forceinline__ void adjNode(const Inst<T> &P, const T *dual, int n, int lane, AdjOut<T, R> &o) {
+__device__ __forceinline__ void adjNode(IP<T> P, GP<T> dual, int n, unsigned lane, AdjOut<T, R> &o) {
     const int nx = P.nx, nu = P.nu, nxu = nx + nu, d4 = nxu + 2;
     zero(o.x);
     zero(o.u);
@@ -246,101 +325,76 @@ __device__ __forceinline__ void adjNode(const Inst<T> &P, const T *dual, int n, 
     if (n < P.nl) {
         const T II = dual[P.oII + n];
         o.s = II;
-        if (lane < P.yD) o.y = dual[P.oI + (long) n * P.yD + lane] - P.b.at(n)[lane] * II;
-        const long b3 = P.oIII + (long) n * P.con3;
+        if (lane < (unsigned) P.yD) o.y = (dual + (P.oI + (long) n * P.yD))[lane] - tab(P.b, n)[lane] * II;
+        GP<T> d3 = dual + (P.oIII + (long) n * P.con3);
         if (P.ncon == CON_RECT_DEV) {
-#pragma unroll
-            for (int rc = 0; rc < R; rc++) {
-                const int r = lane + 64 * rc;
-                if (r < nx) o.x[rc] = dual[b3 + r];
-                if (r < nu) o.u[rc] = dual[b3 + nx + r];
-            }
+            eachRow<R>(nx, lane, [&](int rc, unsigned r) { o.x[rc] = d3[r]; });
+            GP<T> d3u = d3 + nx;
+            eachRow<R>(nu, lane, [&](int rc, unsigned r) { o.u[rc] = d3u[r]; });
         } else if (P.ncon == CON_POLY_DEV) {
-            loadPtr(v, dual + b3, P.con3, lane);
-            const T *GT = P.nGT.at(n);
+            loadPtr(v, d3, P.con3, lane);
+            CP<T> GT = tab(P.nGT, n);
             mvAcc(o.x, GT, nx, nxu, P.con3, v, lane);
             mvAcc(o.u, GT + nx, nu, nxu, P.con3, v, lane);
         }
-        const int c0 = P.chFrom[n], nc = P.numCh[n];
+        const int c0 = cst(P.chFrom)[n], nc = cst(P.numCh)[n];
+#pragma unroll 1
         for (int ci = 0; ci < nc; ci++) {  // children accumulate in order (src/costs.cuh:172-177)
             const int j = c0 + ci;
             if (P.ncost == COST_LIN_DEV) {  // x_i += q_j sum_j, u_i += r_j sum_j (src/costs.cuh:274-285)
                 const T sj = dual[P.oIV + j];
-                const T *qj = P.q.at(j), *rj = P.r.at(j);
-#pragma unroll
-                for (int rc = 0; rc < R; rc++) {
-                    const int r = lane + 64 * rc;
-                    if (r < nx) o.x[rc] += qj[r] * sj;
-                    if (r < nu) o.u[rc] += rj[r] * sj;
-                }
+                CP<T> qj = tab(P.q, j), rj = tab(P.r, j);
+                eachRow<R>(nx, lane, [&](int rc, unsigned r) { o.x[rc] += qj[r] * sj; });
+                eachRow<R>(nu, lane, [&](int rc, unsigned r) { o.u[rc] += rj[r] * sj; });
                 continue;
             }
-            const T *iv = dual + P.oIV + (long) j * d4;
+            GP<T> iv = dual + (P.oIV + (long) j * d4);
             const T a = iv[nxu], bb = iv[nxu + 1];
             loadPtr(v, iv, nx, lane);
             zero(w);
-            mvAcc(w, P.sQ.at(j), nx, nx, nx, v, lane);
+            mvAcc(w, tab(P.sQ, j), nx, nx, nx, v, lane);
             if (P.ncost == COST_QUADLIN_DEV) {
-                const T *qj = P.q.at(j);
-#pragma unroll
-                for (int rc = 0; rc < R; rc++) {
-                    const int r = lane + 64 * rc;
-                    if (r < nx) w[rc] = w[rc] - T(0.5) * qj[r] * a - T(0.5) * qj[r] * bb;
-                }
+                CP<T> qj = tab(P.q, j);
+                eachRow<R>(nx, lane, [&](int rc, unsigned r) { w[rc] = w[rc] - T(0.5) * qj[r] * a - T(0.5) * qj[r] * bb; });
             }
 #pragma unroll
             for (int rc = 0; rc < R; rc++) o.x[rc] += w[rc];
             loadPtr(v, iv + nx, nu, lane);
             zero(w);
-            mvAcc(w, P.sR.at(j), nu, nu, nu, v, lane);
+            mvAcc(w, tab(P.sR, j), nu, nu, nu, v, lane);
             if (P.ncost == COST_QUADLIN_DEV) {
-                const T *rj = P.r.at(j);
-#pragma unroll
-                for (int rc = 0; rc < R; rc++) {
-                    const int r = lane + 64 * rc;
-                    if (r < nu) w[rc] = w[rc] - T(0.5) * rj[r] * a - T(0.5) * rj[r] * bb;
-                }
+                CP<T> rj = tab(P.r, j);
+                eachRow<R>(nu, lane, [&](int rc, unsigned r) { w[rc] = w[rc] - T(0.5) * rj[r] * a - T(0.5) * rj[r] * bb; });
             }
 #pragma unroll
             for (int rc = 0; rc < R; rc++) o.u[rc] += w[rc];
         }
     } else {
         const int l = n - P.nl;
-        const long b5 = P.oV + (long) l * P.con5;
+        GP<T> d5 = dual + (P.oV + (long) l * P.con5);
         if (P.lcon == CON_RECT_DEV) {
-#pragma unroll
-            for (int rc = 0; rc < R; rc++) {
-                const int r = lane + 64 * rc;
-                if (r < nx) o.x[rc] = dual[b5 + r];
-            }
+            eachRow<R>(nx, lane, [&](int rc, unsigned r) { o.x[rc] = d5[r]; });
         } else if (P.lcon == CON_POLY_DEV) {
-            loadPtr(v, dual + b5, P.con5, lane);
-            mvAcc(o.x, P.lGT.at(l), nx, nx, P.con5, v, lane);
+            loadPtr(v, d5, P.con5, lane);
+            mvAcc(o.x, tab(P.lGT, l), nx, nx, P.con5, v, lane);
         }
         if (P.lcost == COST_LIN_DEV) {  // x_l += q sum_l, s_l = set_l (src/costs.cuh:289-292)
             const T sl = dual[P.oVI + l];
-            const T *lq = P.lq.at(l);
-#pragma unroll
-            for (int rc = 0; rc < R; rc++) {
-                const int r = lane + 64 * rc;
-                if (r < nx) o.x[rc] += lq[r] * sl;
-            }
+            CP<T> lq = tab(P.lq, l);
+            eachRow<R>(nx, lane, [&](int rc, unsigned r) { o.x[rc] += lq[r] * sl; });
             o.s = dual[P.oVI + P.nlf + l];
         } else {
-            const T *vi = dual + P.oVI + (long) l * (nx + 2);
+            GP<T> vi = dual + (P.oVI + (long) l * (nx + 2));
             const T a = vi[nx], bb = vi[nx + 1];
             loadPtr(v, vi, nx, lane);
             zero(w);
-            mvAcc(w, P.lsQ.at(l), nx, nx, nx, v, lane);
+            mvAcc(w, tab(P.lsQ, l), nx, nx, nx, v, lane);
 #pragma unroll
             for (int rc = 0; rc < R; rc++) o.x[rc] += w[rc];
             if (P.lcost == COST_QUADLIN_DEV) {
-                const T *lq = P.lq.at(l);
-#pragma unroll
-                for (int rc = 0; rc < R; rc++) {
-                    const int r = lane + 64 * rc;
-                    if (r < nx) o.x[rc] = o.x[rc] - T(0.5) * lq[r] * a - T(0.5) * lq[r] * bb;
-                }
+                CP<T> lq = tab(P.lq, l);
+                eachRow<R>(nx, lane,
+                           [&](int rc, unsigned r) { o.x[rc] = o.x[rc] - T(0.5) * lq[r] * a - T(0.5) * lq[r] * bb; });
             }
             o.s = (a + bb) * T(0.5);
         }
@@ -348,7 +402,7 @@ __device__ __forceinline__ void adjNode(const Inst<T> &P, const T *dual, int n, 
     if (P.ncost == COST_LIN_DEV) {
         o.t = dual[P.oIV + P.N + n];  // t <- set, every node (src/costs.cuh:286)
     } else if (n >= 1) {
-        const T *iv = dual + P.oIV + (long) n * d4;
+        GP<T> iv = dual + (P.oIV + (long) n * d4);
         o.t = (iv[nxu] + iv[nxu + 1]) * T(0.5);
     }
 }
@@ -356,130 +410,108 @@ __device__ __forceinline__ void adjNode(const Inst<T> &P, const T *dual, int n, 
 // ------------------------------------------------------------------ L per node
 // src/operator.cuh:41-60; src/costs.cuh:126-160 (quadratic), :379-416 (quadratic+linear);
 // src/constraints.cuh:158-169 (rectangle), :251-263 (polyhedron).
+// pv(base, k): element base + k of the primal vector, base wave-uniform.
 // The handler H receives each dual block of node n as register values:
 //   blockI(n, yk (lane < yD), IIval)
 //   blockElem(dualIndexBase, vals, rows, lb table entry, ub table entry)  [III and V]
 //   blockSoc(dualIndexBase, xs (rows nx), us (rows nu, may be 0 rows), h, transEntry)  [IV and VI]
 template <typename T, int R, int V, typename PV, typename H>
-__device__ __forceinline__ void opNode(const Inst<T> &P, int n, int lane, PV pv, H &h) {
+__device__ __forceinline__ void opNode(IP<T> P, int n, unsigned lane, PV pv, H &h) {
     const int nx = P.nx, nu = P.nu, nxu = nx + nu;
     T v[V], v2[V], acc[R], acc2[R];
     if (n < P.nl) {
+        const long xn = P.oX + (long) n * nx, un = P.oU + (long) n * nu;
         // I and II
-        const T yk = (lane < P.yD) ? pv(P.oY + (long) n * P.yD + lane) : T(0);
-        const T bk = (lane < P.yD) ? P.b.at(n)[lane] : T(0);
+        const T yk = (lane < (unsigned) P.yD) ? pv(P.oY + (long) n * P.yD, lane) : T(0);
+        const T bk = (lane < (unsigned) P.yD) ? tab(P.b, n)[lane] : T(0);
         const T by = waveSum(bk * yk);
-        const T IIval = pv(P.oS + n) - by;
+        const T IIval = pv(P.oS + n, 0) - by;
         h.blockI(n, yk, IIval);
         // III
         if (P.ncon == CON_RECT_DEV) {
             zero(acc);
             zero(acc2);
-#pragma unroll
-            for (int rc = 0; rc < R; rc++) {
-                const int r = lane + 64 * rc;
-                if (r < nx) acc[rc] = pv(P.oX + (long) n * nx + r);
-                if (r < nu) acc2[rc] = pv(P.oU + (long) n * nu + r);
-            }
+            eachRow<R>(nx, lane, [&](int rc, unsigned r) { acc[rc] = pv(xn, r); });
+            eachRow<R>(nu, lane, [&](int rc, unsigned r) { acc2[rc] = pv(un, r); });
             const long base = P.oIII + (long) n * P.con3;
-            h.blockElem(base, acc, nx, P.nLB.at(n), P.nUB.at(n));
-            h.blockElem(base + nx, acc2, nu, P.nLB.at(n) + nx, P.nUB.at(n) + nx);
+            h.blockElem(base, acc, nx, tab(P.nLB, n), tab(P.nUB, n));
+            h.blockElem(base + nx, acc2, nu, tab(P.nLB, n) + nx, tab(P.nUB, n) + nx);
         } else if (P.ncon == CON_POLY_DEV) {
-            loadV(v, nx, lane, [&](int k) { return pv(P.oX + (long) n * nx + k); });
-            loadV(v2, nu, lane, [&](int k) { return pv(P.oU + (long) n * nu + k); });
+            loadV(v, nx, lane, [&](unsigned k) { return pv(xn, k); });
+            loadV(v2, nu, lane, [&](unsigned k) { return pv(un, k); });
             zero(acc);
-            const T *G = P.nG.at(n);
+            CP<T> G = tab(P.nG, n);
             mvAcc(acc, G, P.con3, P.con3, nx, v, lane);
             mvAcc(acc, G + (size_t) P.con3 * nx, P.con3, P.con3, nu, v2, lane);
-            h.blockElem(P.oIII + (long) n * P.con3, acc, P.con3, P.nLB.at(n), P.nUB.at(n));
+            h.blockElem(P.oIII + (long) n * P.con3, acc, P.con3, tab(P.nLB, n), tab(P.nUB, n));
         }
     }
     // IV
     if (P.ncost == COST_LIN_DEV) {  // (sum_n, set_n) = (q_n' x_anc + r_n' u_anc, t_n), node 0: (0, t_0)
         T sum = T(0);              // (src/costs.cuh:261-267)
         if (n >= 1) {
-            const int a = P.anc[n];
-            const T *qn = P.q.at(n), *rn = P.r.at(n);
+            const int a = cst(P.anc)[n];
+            CP<T> qn = tab(P.q, n), rn = tab(P.r, n);
             T pq = T(0), pr = T(0);
-#pragma unroll
-            for (int c = 0; c < V; c++) {
-                const int k = lane + 64 * c;
-                if (k < nx) pq += qn[k] * pv(P.oX + (long) a * nx + k);
-                if (k < nu) pr += rn[k] * pv(P.oU + (long) a * nu + k);
-            }
+            eachRow<V>(nx, lane, [&](int, unsigned k) { pq += qn[k] * pv(P.oX + (long) a * nx, k); });
+            eachRow<V>(nu, lane, [&](int, unsigned k) { pr += rn[k] * pv(P.oU + (long) a * nu, k); });
             sum = waveSum(pq) + waveSum(pr);
         }
-        h.blockLin(P.oIV + n, P.oIV + P.N + n, sum, pv(P.oT + n));
+        h.blockLin(P.oIV + n, P.oIV + P.N + n, sum, pv(P.oT + n, 0));
     } else {
         zero(acc);
         zero(acc2);
         T hv = T(0);
         if (n >= 1) {
-            const int a = P.anc[n];
-            loadV(v, nx, lane, [&](int k) { return pv(P.oX + (long) a * nx + k); });
-            loadV(v2, nu, lane, [&](int k) { return pv(P.oU + (long) a * nu + k); });
-            mvAcc(acc, P.sQ.at(n), nx, nx, nx, v, lane);
-            mvAcc(acc2, P.sR.at(n), nu, nu, nu, v2, lane);
-            hv = pv(P.oT + n) * T(0.5);
+            const int a = cst(P.anc)[n];
+            loadV(v, nx, lane, [&](unsigned k) { return pv(P.oX + (long) a * nx, k); });
+            loadV(v2, nu, lane, [&](unsigned k) { return pv(P.oU + (long) a * nu, k); });
+            mvAcc(acc, tab(P.sQ, n), nx, nx, nx, v, lane);
+            mvAcc(acc2, tab(P.sR, n), nu, nu, nu, v2, lane);
+            hv = pv(P.oT + n, 0) * T(0.5);
             if (P.ncost == COST_QUADLIN_DEV) {
-                const T *qn = P.q.at(n);
-                const T *rn = P.r.at(n);
+                CP<T> qn = tab(P.q, n), rn = tab(P.r, n);
                 T pq = T(0), pr = T(0);
-#pragma unroll
-                for (int c = 0; c < V; c++) {
-                    const int k = lane + 64 * c;
-                    if (k < nx) pq += qn[k] * v[c];
-                    if (k < nu) pr += rn[k] * v2[c];
-                }
+                eachRow<V>(nx, lane, [&](int c, unsigned k) { pq += qn[k] * v[c]; });
+                eachRow<V>(nu, lane, [&](int c, unsigned k) { pr += rn[k] * v2[c]; });
                 hv = hv + T(-0.5) * waveSum(pq);
                 hv = hv + T(-0.5) * waveSum(pr);
             }
         }
-        h.blockSoc(P.oIV + (long) n * (nxu + 2), acc, nx, acc2, nu, hv, P.trans.at(n));
+        h.blockSoc(P.oIV + (long) n * (nxu + 2), acc, nx, acc2, nu, hv, tab(P.trans, n));
     }
     // V and VI
     if (n >= P.nl) {
         const int l = n - P.nl;
-        loadV(v, nx, lane, [&](int k) { return pv(P.oX + (long) n * nx + k); });
+        const long xn = P.oX + (long) n * nx;
+        loadV(v, nx, lane, [&](unsigned k) { return pv(xn, k); });
         if (P.lcon == CON_RECT_DEV) {
             zero(acc);
-#pragma unroll
-            for (int rc = 0; rc < R; rc++) {
-                const int r = lane + 64 * rc;
-                if (r < nx) acc[rc] = pv(P.oX + (long) n * nx + r);
-            }
-            h.blockElem(P.oV + (long) l * P.con5, acc, nx, P.lLB.at(l), P.lUB.at(l));
+            eachRow<R>(nx, lane, [&](int rc, unsigned) { acc[rc] = v[rc]; });
+            h.blockElem(P.oV + (long) l * P.con5, acc, nx, tab(P.lLB, l), tab(P.lUB, l));
         } else if (P.lcon == CON_POLY_DEV) {
             zero(acc);
-            mvAcc(acc, P.lG.at(l), P.con5, P.con5, nx, v, lane);
-            h.blockElem(P.oV + (long) l * P.con5, acc, P.con5, P.lLB.at(l), P.lUB.at(l));
+            mvAcc(acc, tab(P.lG, l), P.con5, P.con5, nx, v, lane);
+            h.blockElem(P.oV + (long) l * P.con5, acc, P.con5, tab(P.lLB, l), tab(P.lUB, l));
         }
         if (P.lcost == COST_LIN_DEV) {  // (q' x_l, s_l) (src/costs.cuh:269-272)
-            const T *lq = P.lq.at(l);
+            CP<T> lq = tab(P.lq, l);
             T pq = T(0);
-#pragma unroll
-            for (int c = 0; c < V; c++) {
-                const int k = lane + 64 * c;
-                if (k < nx) pq += lq[k] * v[c];
-            }
-            h.blockLin(P.oVI + l, P.oVI + P.nlf + l, waveSum(pq), pv(P.oS + n));
+            eachRow<V>(nx, lane, [&](int c, unsigned k) { pq += lq[k] * v[c]; });
+            h.blockLin(P.oVI + l, P.oVI + P.nlf + l, waveSum(pq), pv(P.oS + n, 0));
             return;
         }
         zero(acc);
         zero(acc2);
-        mvAcc(acc, P.lsQ.at(l), nx, nx, nx, v, lane);
-        T hs = pv(P.oS + n) * T(0.5);
+        mvAcc(acc, tab(P.lsQ, l), nx, nx, nx, v, lane);
+        T hs = pv(P.oS + n, 0) * T(0.5);
         if (P.lcost == COST_QUADLIN_DEV) {
-            const T *lq = P.lq.at(l);
+            CP<T> lq = tab(P.lq, l);
             T pq = T(0);
-#pragma unroll
-            for (int c = 0; c < V; c++) {
-                const int k = lane + 64 * c;
-                if (k < nx) pq += lq[k] * v[c];
-            }
+            eachRow<V>(nx, lane, [&](int c, unsigned k) { pq += lq[k] * v[c]; });
             hs = hs + T(-0.5) * waveSum(pq);
         }
-        h.blockSoc(P.oVI + (long) l * (nx + 2), acc, nx, acc2, 0, hs, P.ltrans.at(l));
+        h.blockSoc(P.oVI + (long) l * (nx + 2), acc, nx, acc2, 0, hs, tab(P.ltrans, l));
     }
 }
 
@@ -487,33 +519,27 @@ __device__ __forceinline__ void opNode(const Inst<T> &P, int n, int lane, PV pv,
 // Raw store of L values into out (dual-local indices).
 template <typename T, int R>
 struct StoreL {
-    const Inst<T> &P;
-    T *out;
-    int lane;
-    __device__ void blockI(int n, T yk, T IIval) {
-        if (lane < P.yD) out[P.oI + (long) n * P.yD + lane] = yk;
+    IP<T> P;
+    GP<T> out;
+    unsigned lane;
+    __device__ __forceinline__ void blockI(int n, T yk, T IIval) {
+        if (lane < (unsigned) P.yD) (out + (P.oI + (long) n * P.yD))[lane] = yk;
         if (lane == 0) out[P.oII + n] = IIval;
     }
-    __device__ void blockElem(long base, const T (&a)[R], int rows, const T *, const T *) {
-#pragma unroll
-        for (int rc = 0; rc < R; rc++) {
-            const int r = lane + 64 * rc;
-            if (r < rows) out[base + r] = a[rc];
-        }
+    __device__ __forceinline__ void blockElem(long base, const T (&a)[R], int rows, CP<T>, CP<T>) {
+        GP<T> ob = out + base;
+        eachRow<R>(rows, lane, [&](int rc, unsigned r) { ob[r] = a[rc]; });
     }
-    __device__ void blockSoc(long base, const T (&xs)[R], int nxr, const T (&us)[R], int nur, T hv, const T *) {
-#pragma unroll
-        for (int rc = 0; rc < R; rc++) {
-            const int r = lane + 64 * rc;
-            if (r < nxr) out[base + r] = xs[rc];
-            if (r < nur) out[base + nxr + r] = us[rc];
-        }
+    __device__ __forceinline__ void blockSoc(long base, const T (&xs)[R], int nxr, const T (&us)[R], int nur, T hv, CP<T>) {
+        GP<T> ob = out + base;
+        eachRow<R>(nxr, lane, [&](int rc, unsigned r) { ob[r] = xs[rc]; });
+        eachRow<R>(nur, lane, [&](int rc, unsigned r) { (ob + nxr)[r] = us[rc]; });
         if (lane == 0) {
-            out[base + nxr + nur] = hv;
-            out[base + nxr + nur + 1] = hv;
+            ob[nxr + nur] = hv;
+            ob[nxr + nur + 1] = hv;
         }
     }
-    __device__ void blockLin(long eSum, long eSet, T sum, T set) {
+    __device__ __forceinline__ void blockLin(long eSum, long eSet, T sum, T set) {
         if (lane == 0) {
             out[eSum] = sum;
             out[eSet] = set;
@@ -526,59 +552,55 @@ struct StoreL {
 // NNOC (src/cones.cuh:134-137), box (src/constraints.cuh:70-74), SOC (src/projections.cuh:102-128).
 template <typename T, int R>
 struct ProxL {
-    const Inst<T> &P;
-    const T *zd;
-    T *cd;
-    int lane;
-    __device__ __forceinline__ T wOf(T Lv, long k, T trans) const { return (Lv * P.gamma + zd[k]) * P.gammaRecip + trans; }
-    __device__ void blockI(int n, T yk, T IIval) {
-        if (lane < P.yD) {
-            const long k = P.oI + (long) n * P.yD + lane;
-            const T w = wOf(yk, k, T(0));
-            const int idx = (lane < 2 * P.numCh[n]) && (w < T(0));
+    IP<T> P;
+    GP<T> zd, cd;
+    unsigned lane;
+    __device__ __forceinline__ T wOf(T Lv, T z, T trans) const { return (Lv * P.gamma + z) * P.gammaRecip + trans; }
+    __device__ __forceinline__ void blockI(int n, T yk, T IIval) {
+        if (lane < (unsigned) P.yD) {
+            const long base = P.oI + (long) n * P.yD;
+            const T w = wOf(yk, (zd + base)[lane], T(0));
+            const int idx = ((int) lane < 2 * cst(P.numCh)[n]) && (w < T(0));
             const T p = T(1 - idx) * w;
-            cd[k] = (w - p) * P.gamma;
+            (cd + base)[lane] = (w - p) * P.gamma;
         }
         if (lane == 0) {
             const long k = P.oII + n;
-            const T w = wOf(IIval, k, T(0));
+            const T w = wOf(IIval, zd[k], T(0));
             const T p = fmax(T(0), w);
             cd[k] = (w - p) * P.gamma;
         }
     }
-    __device__ void blockElem(long base, const T (&a)[R], int rows, const T *lb, const T *ub) {
-#pragma unroll
-        for (int rc = 0; rc < R; rc++) {
-            const int r = lane + 64 * rc;
-            if (r < rows) {
-                const long k = base + r;
-                const T w = wOf(a[rc], k, T(0));
-                const T p = projBox(w, lb[r], ub[r]);
-                cd[k] = (w - p) * P.gamma;
-            }
-        }
+    __device__ __forceinline__ void blockElem(long base, const T (&a)[R], int rows, CP<T> lb, CP<T> ub) {
+        GP<T> zb = zd + base, cb = cd + base;
+        eachRow<R>(rows, lane, [&](int rc, unsigned r) {
+            const T w = wOf(a[rc], zb[r], T(0));
+            const T p = projBox(w, lb[r], ub[r]);
+            cb[r] = (w - p) * P.gamma;
+        });
     }
-    __device__ void blockSoc(long base, const T (&xs)[R], int nxr, const T (&us)[R], int nur, T hv,
-                             const T *tr) {
+    __device__ __forceinline__ void blockSoc(long base, const T (&xs)[R], int nxr, const T (&us)[R], int nur, T hv,
+                                             CP<T> tr) {
         T wx[R], wu[R];
         T ss = T(0);
+        GP<T> zx = zd + base, zu = zx + nxr, zh = zu + nur, cx = cd + base, cu = cx + nxr, ch = cu + nur;
+        CP<T> tu = tr + nxr, th = tu + nur;
 #pragma unroll
         for (int rc = 0; rc < R; rc++) {
-            const int r = lane + 64 * rc;
+            const unsigned r = lane + 64 * rc;
             wx[rc] = T(0);
             wu[rc] = T(0);
-            if (r < nxr) {
-                wx[rc] = wOf(xs[rc], base + r, tr[r]);
+            if (64 * rc < nxr && r < (unsigned) nxr) {
+                wx[rc] = wOf(xs[rc], zx[r], tr[r]);
                 ss += wx[rc] * wx[rc];
             }
-            if (r < nur) {
-                wu[rc] = wOf(us[rc], base + nxr + r, tr[nxr + r]);
+            if (64 * rc < nur && r < (unsigned) nur) {
+                wu[rc] = wOf(us[rc], zu[r], tu[r]);
                 ss += wu[rc] * wu[rc];
             }
         }
-        const long kh = base + nxr + nur;
-        const T w1 = wOf(hv, kh, tr[nxr + nur]);
-        const T w2 = wOf(hv, kh + 1, tr[nxr + nur + 1]);
+        const T w1 = wOf(hv, zh[0], th[0]);
+        const T w2 = wOf(hv, zh[1], th[1]);
         ss = waveSum(ss) + w1 * w1;
         const T nrm = sqrt(ss), tl = w2;
         const int i1 = nrm <= tl;
@@ -586,25 +608,21 @@ struct ProxL {
         const int i3 = !i1 && !i2;
         const T sc = (nrm + tl) / (T(2) * nrm + T(1 - i3));
         const T mult = T(1 - i2) * (T(i3) * sc + T(1 - i3));
-#pragma unroll
-        for (int rc = 0; rc < R; rc++) {
-            const int r = lane + 64 * rc;
-            if (r < nxr) cd[base + r] = (wx[rc] - wx[rc] * mult) * P.gamma;
-            if (r < nur) cd[base + nxr + r] = (wu[rc] - wu[rc] * mult) * P.gamma;
-        }
+        eachRow<R>(nxr, lane, [&](int rc, unsigned r) { cx[r] = (wx[rc] - wx[rc] * mult) * P.gamma; });
+        eachRow<R>(nur, lane, [&](int rc, unsigned r) { cu[r] = (wu[rc] - wu[rc] * mult) * P.gamma; });
         if (lane == 0) {
             const T p1 = w1 * mult;
             const int i1b = (1 - i2) * (1 - i3);
             const T p2 = T(i1b) * (w2 * T(1 - i2)) + T((1 - i1b) * (1 - i2)) * (T(i3) * (sc * nrm - T(1)) + T(1));
-            cd[kh] = (w1 - p1) * P.gamma;
-            cd[kh + 1] = (w2 - p2) * P.gamma;
+            ch[0] = (w1 - p1) * P.gamma;
+            ch[1] = (w2 - p2) * P.gamma;
         }
     }
     // linear cost: the cost entry clamped to at most the epigraph entry, which is kept
     // (src/costs.cuh:296-301 with k_projectRectangle, lower bound -inf)
-    __device__ void blockLin(long eSum, long eSet, T sum, T set) {
+    __device__ __forceinline__ void blockLin(long eSum, long eSet, T sum, T set) {
         if (lane == 0) {
-            const T ws = wOf(sum, eSum, T(0)), wt = wOf(set, eSet, T(0));
+            const T ws = wOf(sum, zd[eSum], T(0)), wt = wOf(set, zd[eSet], T(0));
             cd[eSum] = (ws - projBelow(ws, wt)) * P.gamma;
             cd[eSet] = (wt - wt) * P.gamma;
         }
@@ -615,42 +633,40 @@ struct ProxL {
 // max |y / gamma - ell| over the dual part (src/cache.cuh:722-734 and :917-931).
 template <typename T, int R>
 struct ReduceL {
-    const Inst<T> &P;
-    const T *xd, *yd;  // dual parts of the partner and input vectors
-    int lane;
+    IP<T> P;
+    GP<T> xd, yd;  // dual parts of the partner and input vectors
+    unsigned lane;
     T dot, mx;
-    __device__ __forceinline__ void acc(long k, T ell) {
-        const T y = yd[k];
-        dot += xd[k] * (ell * (-P.gamma) + y);
+    __device__ __forceinline__ void acc(T x, T y, T ell) {
+        dot += x * (ell * (-P.gamma) + y);
         mx = fmax(mx, fabs(y * P.gammaRecip - ell));
     }
-    __device__ void blockI(int n, T yk, T IIval) {
-        if (lane < P.yD) acc(P.oI + (long) n * P.yD + lane, yk);
-        if (lane == 0) acc(P.oII + n, IIval);
+    __device__ __forceinline__ void blockI(int n, T yk, T IIval) {
+        const long base = P.oI + (long) n * P.yD, k = P.oII + n;
+        if (lane < (unsigned) P.yD) acc((xd + base)[lane], (yd + base)[lane], yk);
+        if (lane == 0) acc(xd[k], yd[k], IIval);
     }
-    __device__ void blockElem(long base, const T (&a)[R], int rows, const T *, const T *) {
+    __device__ __forceinline__ void blockElem(long base, const T (&a)[R], int rows, CP<T>, CP<T>) {
+        GP<T> xb = xd + base, yb = yd + base;
+        eachRow<R>(rows, lane, [&](int rc, unsigned r) { acc(xb[r], yb[r], a[rc]); });
+    }
+    __device__ __forceinline__ void blockSoc(long base, const T (&xs)[R], int nxr, const T (&us)[R], int nur, T hv, CP<T>) {
+        GP<T> xx = xd + base, yx = yd + base, xu = xx + nxr, yu = yx + nxr, xh = xu + nur, yh = yu + nur;
 #pragma unroll
         for (int rc = 0; rc < R; rc++) {
-            const int r = lane + 64 * rc;
-            if (r < rows) acc(base + r, a[rc]);
-        }
-    }
-    __device__ void blockSoc(long base, const T (&xs)[R], int nxr, const T (&us)[R], int nur, T hv, const T *) {
-#pragma unroll
-        for (int rc = 0; rc < R; rc++) {
-            const int r = lane + 64 * rc;
-            if (r < nxr) acc(base + r, xs[rc]);
-            if (r < nur) acc(base + nxr + r, us[rc]);
+            const unsigned r = lane + 64 * rc;
+            if (64 * rc < nxr && r < (unsigned) nxr) acc(xx[r], yx[r], xs[rc]);
+            if (64 * rc < nur && r < (unsigned) nur) acc(xu[r], yu[r], us[rc]);
         }
         if (lane == 0) {
-            acc(base + nxr + nur, hv);
-            acc(base + nxr + nur + 1, hv);
+            acc(xh[0], yh[0], hv);
+            acc(xh[1], yh[1], hv);
         }
     }
-    __device__ void blockLin(long eSum, long eSet, T sum, T set) {
+    __device__ __forceinline__ void blockLin(long eSum, long eSet, T sum, T set) {
         if (lane == 0) {
-            acc(eSum, sum);
-            acc(eSet, set);
+            acc(xd[eSum], yd[eSum], sum);
+            acc(xd[eSet], yd[eSet], set);
         }
     }
 };
@@ -659,32 +675,28 @@ struct ReduceL {
 // modifyPrimal + proxRootS (src/cache.cuh:748-753, 639-642): cand_p = z_p - gamma L*(z_d); s_0 -= gamma.
 // Leaf tasks also seed the dynamics sweep with q_leaf = -xbar_leaf (src/dynamics.cuh:79-81).
 template <typename T, int R, int V>
-__device__ __noinline__ void phaseAdjAxpy(const Inst<T> &P, const Tc &c, const T *z, T *cand) {
-    const T *zd = z + P.sPrim;
+__device__ __noinline__ void phaseAdjAxpy(const Inst<T> *Pp, int grid, T *zIn, T *candIn) {
+    IP<T> P = *cst(uniformPtr(Pp));
+    const Tc c = threadCtx(grid);
+    GP<T> z = glb(zIn), cand = glb(candIn), qd = (GP<T>) P.qd;
+    GP<T> zd = z + P.sPrim;
     const T g = -P.gamma;
     const int nx = P.nx, nu = P.nu;
+    const unsigned lane = c.lane;
     for (int n = c.wave; n < P.N; n += c.nw) {
         AdjOut<T, R> o;
-        adjNode<T, R, V>(P, zd, n, c.lane, o);
-#pragma unroll
-        for (int rc = 0; rc < R; rc++) {
-            const int r = c.lane + 64 * rc;
-            if (r < nx) {
-                const long k = P.oX + (long) n * nx + r;
-                const T v = o.x[rc] * g + z[k];
-                cand[k] = v;
-                if (n >= P.nl) P.qd[(long) n * nx + r] = -v;
-            }
-            if (n < P.nl && r < nu) {
-                const long k = P.oU + (long) n * nu + r;
-                cand[k] = o.u[rc] * g + z[k];
-            }
+        adjNode<T, R, V>(P, zd, n, lane, o);
+        const long xn = P.oX + (long) n * nx, un = P.oU + (long) n * nu, yn = P.oY + (long) n * P.yD;
+        eachRow<R>(nx, lane, [&](int rc, unsigned r) {
+            const T v = o.x[rc] * g + (z + xn)[r];
+            (cand + xn)[r] = v;
+            if (n >= P.nl) (qd + (long) n * nx)[r] = -v;
+        });
+        if (n < P.nl) {
+            eachRow<R>(nu, lane, [&](int rc, unsigned r) { (cand + un)[r] = o.u[rc] * g + (z + un)[r]; });
+            if (lane < (unsigned) P.yD) (cand + yn)[lane] = o.y * g + (z + yn)[lane];
         }
-        if (n < P.nl && c.lane < P.yD) {
-            const long k = P.oY + (long) n * P.yD + c.lane;
-            cand[k] = o.y * g + z[k];
-        }
-        if (c.lane == 0) {
+        if (lane == 0) {
             T sv = o.s * g + z[P.oS + n];
             if (n == 0) sv -= P.gamma;
             cand[P.oS + n] = sv;
@@ -696,148 +708,143 @@ __device__ __noinline__ void phaseAdjAxpy(const Inst<T> &P, const Tc &c, const T
 // Backward sweep step for node i (src/dynamics.cuh:85-139).  With affine dynamics the children's
 // q enter as q_j + P_j e_j (src/dynamics.cuh:93-97).
 template <typename T, int R, int V>
-__device__ __forceinline__ void dynBackwardNode(const Inst<T> &P, T *cand, int i, int stage, int lane) {
+__device__ __forceinline__ void dynBackwardNode(IP<T> P, GP<T> cand, int i, int stage, unsigned lane) {
     const int nx = P.nx, nu = P.nu;
-    const T *ubar = cand + P.oU + (long) i * nu;
-    const T *xbar = cand + P.oX + (long) i * nx;
+    GP<T> ubar = cand + (P.oU + (long) i * nu);
+    GP<T> xbar = cand + (P.oX + (long) i * nx);
+    GP<T> qd = (GP<T>) P.qd;
     T v[V], w[R], acc[R];
     zero(acc);
-    const int c0 = P.chFrom[i], nc = P.numCh[i];
+    const int c0 = cst(P.chFrom)[i], nc = cst(P.numCh)[i];
+    const bool mine = lane < (unsigned) nu;
     auto loadQ = [&](int j) {
-        const T *qj = P.qd + (long) j * nx;
+        GP<T> qj = qd + (long) j * nx;
         if (P.affine) {
-            const T *pe = P.Pe.at(j);
-            loadV(v, nx, lane, [&](int k) { return qj[k] + pe[k]; });
+            CP<T> pe = tab(P.Pe, j);
+            loadV(v, nx, lane, [&](unsigned k) -> T { return qj[k] + pe[k]; });
         } else {
             loadPtr(v, qj, nx, lane);
         }
     };
+    const T ub = mine ? ubar[lane] : T(0);
+#pragma unroll 1
     for (int ci = 0; ci < nc; ci++) {
         const int j = c0 + ci;
         loadQ(j);
         zero(w);
-        mvAcc(w, P.BTr.at(j), nu, nu, nx, v, lane);
+        mvAcc(w, tab(P.BTr, j), nu, nu, nx, v, lane);
 #pragma unroll
         for (int rc = 0; rc < R; rc++) acc[rc] = (ci == 0) ? w[rc] : acc[rc] + w[rc];
     }
     // d = R~^-1 (u - sum B'q) with R~ = L L': one matvec with the precomputed inverse, or the
     // two triangular solves of potrs
-    T d = (lane < nu) ? (-acc[0] + ubar[lane]) : T(0);
+    T d = mine ? (-acc[0] + ub) : T(0);
     if (P.dynInverse) {
         T dvin[V], dout[R];
         zero(dvin);
         dvin[0] = d;
         zero(dout);
-        mvAcc(dout, P.RtInv.at(i), nu, nu, nu, dvin, lane);
-        d = (lane < nu) ? dout[0] : T(0);
+        mvAcc(dout, tab(P.RtInv, i), nu, nu, nu, dvin, lane);
+        d = mine ? dout[0] : T(0);
     } else {
-        const T *L = P.cholL.at(i);
+        CP<T> L = tab(P.cholL, i);
         for (int k = 0; k < nu; k++) {
             const T dk = bcastLane(d, k) / L[k + (size_t) k * nu];
-            if (lane == k) d = dk;
-            else if (lane > k && lane < nu) d -= L[lane + (size_t) k * nu] * dk;
+            if ((int) lane == k) d = dk;
+            else if ((int) lane > k && mine) d -= L[lane + (size_t) k * nu] * dk;
         }
-        const T *U = P.cholU.at(i);
+        CP<T> U = tab(P.cholU, i);
         for (int k = nu - 1; k >= 0; k--) {
             const T dk = bcastLane(d, k) / U[k + (size_t) k * nu];
-            if (lane == k) d = dk;
-            else if (lane < k) d -= U[lane + (size_t) k * nu] * dk;
+            if ((int) lane == k) d = dk;
+            else if ((int) lane < k) d -= U[lane + (size_t) k * nu] * dk;
         }
     }
-    if (lane < nu) P.dd[(long) i * nu + lane] = d;
+    if (mine) ((GP<T>) P.dd + (long) i * nu)[lane] = d;
     if (stage == 0) return;
     // q_i = sum_j (APB_j d_i + ABKTr_j q_j) + K_i'(d_i - u_i) - x_i
     T dv[V];
     zero(dv);
-    dv[0] = (lane < nu) ? d : T(0);
+    dv[0] = d;
     zero(acc);
+#pragma unroll 1
     for (int ci = 0; ci < nc; ci++) {
         const int j = c0 + ci;
         zero(w);
-        mvAcc(w, P.APB.at(j), nx, nx, nu, dv, lane);
-        loadQ(j);
-        mvAcc(w, P.ABKTr.at(j), nx, nx, nx, v, lane);
+        mvAcc(w, tab(P.APB, j), nx, nx, nu, dv, lane);
+        if (nc > 1) loadQ(j);  // a single child's q is still in v
+        mvAcc(w, tab(P.ABKTr, j), nx, nx, nx, v, lane);
 #pragma unroll
         for (int rc = 0; rc < R; rc++) acc[rc] = (ci == 0) ? w[rc] : acc[rc] + w[rc];
     }
-    dv[0] = (lane < nu) ? d - ubar[lane] : T(0);
+    dv[0] = mine ? d - ub : T(0);
     zero(w);
-    mvAcc(w, P.KTr.at(i), nx, nx, nu, dv, lane);
-#pragma unroll
-    for (int rc = 0; rc < R; rc++) {
-        const int r = lane + 64 * rc;
-        if (r < nx) P.qd[(long) i * nx + r] = (acc[rc] + w[rc]) - xbar[r];
-    }
+    mvAcc(w, tab(P.KTr, i), nx, nx, nu, dv, lane);
+    eachRow<R>(nx, lane, [&](int rc, unsigned r) { (qd + (long) i * nx)[r] = (acc[rc] + w[rc]) - xbar[r]; });
 }
 
 // Kernel projection for nonleaf node i (src/cache.cuh:650-676); padded child slots enter as 0.
 template <typename T, int R, int V>
-__device__ __forceinline__ void kernelNode(const Inst<T> &P, T *cand, int i, int lane) {
-    const int yD = P.yD, E = P.E, nc = P.numCh[i], c0 = P.chFrom[i];
-    T v = T(0);
-    if (lane < yD) v = cand[P.oY + (long) i * yD + lane];
-    else if (lane < yD + E) {
-        if (lane - yD < nc) v = cand[P.oT + c0 + (lane - yD)];
-    } else if (lane < yD + 2 * E) {
-        if (lane - yD - E < nc) v = cand[P.oS + c0 + (lane - yD - E)];
-    }
+__device__ __forceinline__ void kernelNode(IP<T> P, GP<T> cand, int i, unsigned lane) {
+    const int yD = P.yD, E = P.E, nc = cst(P.numCh)[i], c0 = cst(P.chFrom)[i];
+    // this lane's entry of [y; t of the children; s of the children], or none
+    const int k = (int) lane;
+    const bool isY = k < yD, isT = !isY && k < yD + E && k - yD < nc;
+    const bool isS = k >= yD + E && k < yD + 2 * E && k - yD - E < nc;
+    const bool any = isY || isT || isS;
+    const long at = isY ? P.oY + (long) i * yD + k : isT ? P.oT + c0 + (k - yD) : P.oS + c0 + (k - yD - E);
     T vin[V], w[R];
     zero(vin);
-    vin[0] = v;
+    if (any) vin[0] = cand[at];
     zero(w);
-    mvAcc(w, P.NN.at(i), P.nD, P.nD, P.nD, vin, lane);
-    if (lane < yD) cand[P.oY + (long) i * yD + lane] = w[0];
-    else if (lane < yD + E) {
-        if (lane - yD < nc) cand[P.oT + c0 + (lane - yD)] = w[0];
-    } else if (lane < yD + 2 * E) {
-        if (lane - yD - E < nc) cand[P.oS + c0 + (lane - yD - E)] = w[0];
-    }
+    mvAcc(w, tab(P.NN, i), P.nD, P.nD, P.nD, vin, lane);
+    if (any) cand[at] = w[0];
 }
 
 // Forward rollout for node i (src/dynamics.cuh:144-173); affine dynamics add e_j to each child.
 template <typename T, int R, int V>
-__device__ __forceinline__ void dynForwardNode(const Inst<T> &P, T *cand, int i, int lane) {
+__device__ __forceinline__ void dynForwardNode(IP<T> P, GP<T> cand, int i, unsigned lane) {
     const int nx = P.nx, nu = P.nu;
     T xv[V], uv[V], w[R];
+    GP<T> xi = cand + (P.oX + (long) i * nx);
     if (i == 0) {
-        loadPtr(xv, P.x0s, nx, lane);
-#pragma unroll
-        for (int c = 0; c < V; c++) {
-            const int k = lane + 64 * c;
-            if (k < nx) cand[P.oX + k] = xv[c];
-        }
+        loadPtr(xv, cst(P.x0s), nx, lane);
+        eachRow<V>(nx, lane, [&](int c, unsigned k) { xi[k] = xv[c]; });
     } else {
-        loadPtr(xv, cand + P.oX + (long) i * nx, nx, lane);
+        loadPtr(xv, xi, nx, lane);
     }
+    const bool mine = lane < (unsigned) nu;
+    const T di = mine ? ((GP<T>) P.dd + (long) i * nu)[lane] : T(0);
     zero(w);
-    mvAcc(w, P.K.at(i), nu, nu, nx, xv, lane);
-    const T u = (lane < nu) ? w[0] + P.dd[(long) i * nu + lane] : T(0);
-    if (lane < nu) cand[P.oU + (long) i * nu + lane] = u;
+    mvAcc(w, tab(P.K, i), nu, nu, nx, xv, lane);
+    const T u = mine ? w[0] + di : T(0);
+    if (mine) (cand + (P.oU + (long) i * nu))[lane] = u;
     zero(uv);
     uv[0] = u;
-    const int c0 = P.chFrom[i], nc = P.numCh[i];
+    const int c0 = cst(P.chFrom)[i], nc = cst(P.numCh)[i];
+#pragma unroll 1
     for (int ci = 0; ci < nc; ci++) {
         const int j = c0 + ci;
-        const T *AB = P.AB.at(j);
+        CP<T> AB = tab(P.AB, j);
         zero(w);
         mvAcc(w, AB, nx, nx, nx, xv, lane);
         mvAcc(w, AB + (size_t) nx * nx, nx, nx, nu, uv, lane);
-        const T *ej = P.e.at(j);
-#pragma unroll
-        for (int rc = 0; rc < R; rc++) {
-            const int r = lane + 64 * rc;
-            if (r < nx) cand[P.oX + (long) j * nx + r] = P.affine ? w[rc] + ej[r] : w[rc];
-        }
+        CP<T> ej = tab(P.e, j);
+        GP<T> xj = cand + (P.oX + (long) j * nx);
+        eachRow<R>(nx, lane, [&](int rc, unsigned r) { xj[r] = P.affine ? w[rc] + ej[r] : w[rc]; });
     }
 }
 
 // Dynamics projection + kernel projection on cand (in place).  The kernel projection touches
 // (y, t, s) only, so it shares the first backward stage's barrier interval.
 template <typename T, int R, int V>
-__device__ __noinline__ void phaseProjections(const Inst<T> &P, const Tc &c, T *cand, bool doDyn, bool doKernel) {
+__device__ __noinline__ void phaseProjections(const Inst<T> *Pp, int grid, T *candIn, bool doDyn, bool doKernel) {
+    IP<T> P = *cst(uniformPtr(Pp));
+    const Tc c = threadCtx(grid);
+    GP<T> cand = glb(candIn);
     if (doDyn) {
         for (int stage = P.S - 2; stage >= 0; stage--) {
-            const int f = P.stageFrom[stage], nStage = P.stageTo[stage] - f + 1;
+            const int f = cst(P.stageFrom)[stage], nStage = cst(P.stageTo)[stage] - f + 1;
             const int extra = (doKernel && stage == P.S - 2) ? P.nl : 0;
             for (int task = c.wave; task < nStage + extra; task += c.nw) {
                 if (task < nStage) dynBackwardNode<T, R, V>(P, cand, f + task, stage, c.lane);
@@ -846,7 +853,7 @@ __device__ __noinline__ void phaseProjections(const Inst<T> &P, const Tc &c, T *
             sync(c);
         }
         for (int stage = 0; stage <= P.S - 2; stage++) {
-            const int f = P.stageFrom[stage], nStage = P.stageTo[stage] - f + 1;
+            const int f = cst(P.stageFrom)[stage], nStage = cst(P.stageTo)[stage] - f + 1;
             for (int task = c.wave; task < nStage; task += c.nw) dynForwardNode<T, R, V>(P, cand, f + task, c.lane);
             sync(c);
         }
@@ -858,66 +865,84 @@ __device__ __noinline__ void phaseProjections(const Inst<T> &P, const Tc &c, T *
 
 // modifyDual + proximalDual (src/cache.cuh:770-789) on 2 x-bar - z_p.
 template <typename T, int R, int V>
-__device__ __noinline__ void phaseDualProx(const Inst<T> &P, const Tc &c, const T *z, T *cand) {
+__device__ __noinline__ void phaseDualProx(const Inst<T> *Pp, int grid, T *zIn, T *candIn) {
+    IP<T> P = *cst(uniformPtr(Pp));
+    const Tc c = threadCtx(grid);
+    GP<T> z = glb(zIn), cand = glb(candIn);
     ProxL<T, R> h{P, z + P.sPrim, cand + P.sPrim, c.lane};
-    auto pv = [&](long k) { return cand[k] * T(2) - z[k]; };
+    auto pv = [&](long base, unsigned k) -> T { return (cand + base)[k] * T(2) - (z + base)[k]; };
     for (int n = c.wave; n < P.N; n += c.nw) opNode<T, R, V>(P, n, c.lane, pv, h);
     sync(c);
 }
 
 // The CP operator T (src/cache.cuh:796-801): cand = T(z).
 template <typename T, int R, int V>
-__device__ __forceinline__ void applyT(const Inst<T> &P, const Tc &c, const T *z, T *cand, PhaseClock *clk = nullptr) {
-    phaseAdjAxpy<T, R, V>(P, c, z, cand);
+__device__ __forceinline__ void applyT(const Inst<T> *P, const Tc &c, T *z, T *cand, PhaseClock *clk = nullptr) {
+    phaseAdjAxpy<T, R, V>(P, c.grid, z, cand);
     sync(c);
     if (clk) clk->mark(PH_ADJ);
-    phaseProjections<T, R, V>(P, c, cand, true, true);
+    phaseProjections<T, R, V>(P, c.grid, cand, true, true);
     if (clk) clk->mark(PH_PROJ);
-    phaseDualProx<T, R, V>(P, c, z, cand);
+    phaseDualProx<T, R, V>(P, c.grid, z, cand);
     if (clk) clk->mark(PH_DUAL);
 }
 
-// sum x.(y - gamma ell(y)) and max |y/gamma - ell(y)| with ell(y) = [L* y_d; L y_p].
-// SPLIT: also the maxima over the primal and the dual part apart, in split[0] and split[1]
-// (err1 and err2 of the debug trace).
-template <typename T, int R, int V, bool SPLIT = false>
-__device__ __noinline__ void reduceEll(const Inst<T> &P, const Tc &c, const T *x, const T *y, T *lds, T &dotOut, T &maxOut,
-                                       T *split = nullptr) {
+// sum x.(y - gamma ell(y)) and max |y/gamma - ell(y)| with ell(y) = [L* y_d; L y_p]; mx[0] and mx[1]
+// are the maxima over the primal and the dual part (err1 and err2 of the debug trace).
+template <typename T>
+struct EllSums {
+    T dot, mxPrim, mxDual;
+};
+
+template <typename T, int R, int V>
+__device__ __noinline__ EllSums<T> reduceEllNodes(const Inst<T> *Pp, int grid, T *xIn, T *yIn) {
+    IP<T> P = *cst(uniformPtr(Pp));
+    const Tc c = threadCtx(grid);
+    GP<T> x = glb(xIn), y = glb(yIn);
     const int nx = P.nx, nu = P.nu;
+    const unsigned lane = c.lane;
     T dot = T(0), mx = T(0);
-    auto acc = [&](long k, T ell) {
-        const T yk = y[k];
-        dot += x[k] * (ell * (-P.gamma) + yk);
+    auto acc = [&](T xk, T yk, T ell) {
+        dot += xk * (ell * (-P.gamma) + yk);
         mx = fmax(mx, fabs(yk * P.gammaRecip - ell));
     };
-    const T *yd = y + P.sPrim;
-    ReduceL<T, R> h{P, x + P.sPrim, yd, c.lane, T(0), T(0)};
-    auto pv = [&](long k) { return y[k]; };
+    GP<T> yd = y + P.sPrim;
+    ReduceL<T, R> h{P, x + P.sPrim, yd, lane, T(0), T(0)};
+    auto pv = [&](long base, unsigned k) -> T { return (y + base)[k]; };
     for (int n = c.wave; n < P.N; n += c.nw) {
         AdjOut<T, R> o;
-        adjNode<T, R, V>(P, yd, n, c.lane, o);
+        adjNode<T, R, V>(P, yd, n, lane, o);
+        const long xn = P.oX + (long) n * nx, un = P.oU + (long) n * nu, yn = P.oY + (long) n * P.yD;
 #pragma unroll
         for (int rc = 0; rc < R; rc++) {
-            const int r = c.lane + 64 * rc;
-            if (r < nx) acc(P.oX + (long) n * nx + r, o.x[rc]);
-            if (n < P.nl && r < nu) acc(P.oU + (long) n * nu + r, o.u[rc]);
+            const unsigned r = lane + 64 * rc;
+            if (64 * rc < nx && r < (unsigned) nx) acc((x + xn)[r], (y + xn)[r], o.x[rc]);
+            if (n < P.nl && 64 * rc < nu && r < (unsigned) nu) acc((x + un)[r], (y + un)[r], o.u[rc]);
         }
-        if (n < P.nl && c.lane < P.yD) acc(P.oY + (long) n * P.yD + c.lane, o.y);
-        if (c.lane == 0) {
-            acc(P.oS + n, o.s);
-            acc(P.oT + n, o.t);
+        if (n < P.nl && lane < (unsigned) P.yD) acc((x + yn)[lane], (y + yn)[lane], o.y);
+        if (lane == 0) {
+            acc(x[P.oS + n], y[P.oS + n], o.s);
+            acc(x[P.oT + n], y[P.oT + n], o.t);
         }
-        opNode<T, R, V>(P, n, c.lane, pv, h);
+        opNode<T, R, V>(P, n, lane, pv, h);
     }
-    T v[1] = {dot + h.dot};
+    return EllSums<T>{dot + h.dot, mx, h.mx};
+}
+
+// SPLIT: also the maxima over the primal and the dual part apart, in split[0] and split[1].
+template <typename T, int R, int V, bool SPLIT = false>
+__device__ __forceinline__ void reduceEll(const Inst<T> *P, const Tc &c, T *x, T *y, SPK_LDS T *lds, T &dotOut,
+                                          T &maxOut, T *split = nullptr) {
+    const EllSums<T> s = reduceEllNodes<T, R, V>(P, c.grid, x, y);
+    T v[1] = {s.dot};
     blockSum(v, lds, c);
     dotOut = v[0];
     if constexpr (SPLIT) {
-        split[0] = blockMax(mx, lds, c);
-        split[1] = blockMax(h.mx, lds, c);
+        split[0] = blockMax(s.mxPrim, lds, c);
+        split[1] = blockMax(s.mxDual, lds, c);
         maxOut = fmax(split[0], split[1]);
     } else {
-        maxOut = blockMax(fmax(mx, h.mx), lds, c);
+        maxOut = blockMax(fmax(s.mxPrim, s.mxDual), lds, c);
     }
 }
 
@@ -952,16 +977,20 @@ struct V4 {
 // src/cache.cuh:861-904 with the least squares argmin ||Y g - r|| solved by Householder QR
 // (geqrf + ormqr + trsm).  Y and S are rings of andBuff columns; logical column 0 is the newest.
 template <typename T>
-__device__ __noinline__ void andersonHouseholder(const Inst<T> &P, const Tc &c, int head, const T *r, T *lds,
+__device__ __noinline__ void andersonHouseholder(const Inst<T> *Pp, int grid, int head, T *rIn, SPK_LDS T *lds,
                                                 double (&gs)[8]) {
+    IP<T> P = *cst(uniformPtr(Pp));
+    const Tc c = threadCtx(grid, P.gpart);
+    GP<T> r = glb(rIn);
+    head = __builtin_amdgcn_readfirstlane(head);
     const long n = P.sIter;
     const int m = P.andBuff;
     auto slot = [&](int lc) { return (head - lc + m) % m; };
-    T *W = P.W;
+    GP<T> W = (GP<T>) P.W;
     // copy [Y (logical order) | r] and the first column's tail norm
-    const T *Yl[8];
+    GP<T> Yl[8];
 #pragma unroll
-    for (int lc = 0; lc < 8; lc++) Yl[lc] = P.hY + (long) slot(lc < m ? lc : 0) * n;
+    for (int lc = 0; lc < 8; lc++) Yl[lc] = (GP<T>) P.hY + (long) slot(lc < m ? lc : 0) * n;
     T sig[1] = {T(0)};
     stream<4>(
         n, c, [&](long k) { return k; },
@@ -989,7 +1018,7 @@ __device__ __noinline__ void andersonHouseholder(const Inst<T> &P, const Tc &c, 
 #pragma unroll
         for (int q = 0; q < 8; q++)
             if (q == kk) Rd[q] = beta;
-        const T *Wk = W + (long) kk * n;
+        GP<T> Wk = W + (long) kk * n;
         const long len = n - kk;
         if (tau != T(0)) {
             T wj[8];
@@ -1017,8 +1046,9 @@ __device__ __noinline__ void andersonHouseholder(const Inst<T> &P, const Tc &c, 
 #pragma unroll
                     for (int jj = 0; jj < 8; jj++) {
                         if (kk + 1 + jj <= m) {
-                            T &e = W[(long) (kk + 1 + jj) * n + k];
+                            T e = W[(long) (kk + 1 + jj) * n + k];
                             e -= wt[jj] * vk;
+                            W[(long) (kk + 1 + jj) * n + k] = e;
                             if (jj == 0 && k >= kk + 2) sg[0] += e * e;
                         }
                     }
@@ -1060,11 +1090,15 @@ __device__ __noinline__ void andersonHouseholder(const Inst<T> &P, const Tc &c, 
 // With the Gram least squares it also accumulates, in FP64, <Y_h, Y_s> for every slot s and
 // <Y_s, r> for every slot, and updates the slot-indexed Gram matrix G held in LDS.
 template <typename T>
-__device__ __noinline__ void andersonColumn(const Inst<T> &P, const Tc &c, int head, const T *Rv, const T *RP,
-                                            const T *Z, const T *ZP, bool gram, double *G, double *gb, double *ldsd) {
+__device__ __noinline__ void andersonColumn(const Inst<T> *Pp, int grid, int head, T *RIn, T *RPIn, T *ZIn, T *ZPIn,
+                                            bool gram, SPK_LDS double *G, SPK_LDS double *gb, SPK_LDS double *ldsd) {
+    IP<T> P = *cst(uniformPtr(Pp));
+    const Tc c = threadCtx(grid, P.gpart);
+    GP<T> Rv = glb(RIn), RP = glb(RPIn), Z = glb(ZIn), ZP = glb(ZPIn);
+    head = __builtin_amdgcn_readfirstlane(head);
     const long n = P.sIter;
     const int m = P.andBuff;
-    T *Yh = P.hY + (long) head * n, *Sh = P.hS + (long) head * n;
+    GP<T> Yh = (GP<T>) P.hY + (long) head * n, Sh = (GP<T>) P.hS + (long) head * n;
     if (!gram) {
         stream<8>(
             n, c, [&](long k) { return V4<T>{Rv[k], RP[k], Z[k], ZP[k]}; },
@@ -1079,9 +1113,9 @@ __device__ __noinline__ void andersonColumn(const Inst<T> &P, const Tc &c, int h
     double acc[16];
 #pragma unroll
     for (int q = 0; q < 16; q++) acc[q] = 0.;
-    const T *Ys[8];
+    GP<T> Ys[8];
 #pragma unroll
-    for (int s2 = 0; s2 < 8; s2++) Ys[s2] = P.hY + (long) (s2 < m ? s2 : 0) * n;
+    for (int s2 = 0; s2 < 8; s2++) Ys[s2] = (GP<T>) P.hY + (long) (s2 < m ? s2 : 0) * n;
     stream<4>(
         n, c, [&](long k) { return V4<T>{Rv[k], RP[k], Z[k], ZP[k]}; },
         [&](long k, const V4<T> &v) {
@@ -1111,7 +1145,7 @@ __device__ __noinline__ void andersonColumn(const Inst<T> &P, const Tc &c, int h
 
 // Least squares argmin ||Y g - r|| from the Gram matrix: Cholesky of G + eps * max(diag) I in
 // FP64 (uniform in every thread).  Returns false when the factorisation breaks down.
-__device__ __forceinline__ bool gramSolve(const double *G, const double *gb, int m, double (&g)[8]) {
+__device__ __forceinline__ bool gramSolve(const SPK_LDS double *G, const SPK_LDS double *gb, int m, double (&g)[8]) {
     double Lm[8][8];
     double dmax = 0.;
     for (int i = 0; i < m; i++) dmax = fmax(dmax, G[i * 8 + i]);
@@ -1164,16 +1198,19 @@ __device__ __forceinline__ bool gramSolve(const double *G, const double *gb, int
 // d = -S g - r (src/cache.cuh:897-898); with toCand the K0 update cand = z_prev + d is written
 // directly (src/cache.cuh:1055-1057) and d itself is not stored.
 template <typename T>
-__device__ __noinline__ void andersonApply(const Inst<T> &P, const Tc &c, const double (&gs)[8], bool useLS,
-                                           const T *Rv, const T *ZP, T *out, bool toCand) {
+__device__ __noinline__ void andersonApply(const Inst<T> *Pp, int grid, const double (&gs)[8], bool useLS, T *RIn,
+                                           T *ZPIn, T *outIn, bool toCand) {
+    IP<T> P = *cst(uniformPtr(Pp));
+    const Tc c = threadCtx(grid);
+    GP<T> Rv = glb(RIn), ZP = glb(ZPIn), out = glb(outIn);
     const long n = P.sIter;
     const int m = P.andBuff;
     T gg[8];
-    const T *Ss[8];
+    GP<T> Ss[8];
 #pragma unroll
     for (int s2 = 0; s2 < 8; s2++) {
         gg[s2] = (useLS && s2 < m) ? (T) gs[s2] : T(0);
-        Ss[s2] = P.hS + (long) (s2 < m ? s2 : 0) * n;
+        Ss[s2] = (GP<T>) P.hS + (long) (s2 < m ? s2 : 0) * n;
     }
     if (!useLS) {
         stream<8>(
@@ -1201,7 +1238,8 @@ __device__ __noinline__ void andersonApply(const Inst<T> &P, const Tc &c, const 
 // Index of the first non-finite entry of v[0, n), or -1.  The index travels through the block's
 // T-valued max reduction as n - k, exact while n < 2^24 in FP32 (2^53 in FP64).
 template <typename T>
-__device__ __noinline__ long firstNonfinite(const T *v, long n, T *lds, const Tc &c) {
+__device__ __noinline__ long firstNonfinite(const T *v, long n, SPK_LDS T *lds, int grid, void *gpart) {
+    const Tc c = threadCtx(grid, gpart);
     T bad = T(0);
     for (long k = c.tid; k < n; k += c.nt)
         if (!isfinite(v[k])) bad = fmax(bad, T(n - k));
@@ -1218,8 +1256,10 @@ __device__ __noinline__ long firstNonfinite(const T *v, long n, T *lds, const Tc
 //   callsL      calls to L and L* counted so far: two per application of T (src/cache.cuh:704-716,
 //               :750, :773); the host adds the count of earlier solves
 template <typename T>
-__device__ __noinline__ void debugRecord(const Inst<T> &P, const Tc &c, T *lds, long it, long callsL,
+__device__ __noinline__ void debugRecord(const Inst<T> *Pp, int grid, SPK_LDS T *lds, long it, long callsL,
                                          const T (&split)[2], const T *RR, const T *C, long &nDbg) {
+    IP<T> P = *cst(uniformPtr(Pp));
+    const Tc c = threadCtx(grid, P.gpart);
     T acc[2] = {T(0), T(0)};
     for (long k = c.tid; k < P.sIter; k += c.nt) acc[0] += RR[k] * RR[k];
     T *E = P.dbgE;
@@ -1247,12 +1287,14 @@ __device__ __noinline__ void debugRecord(const Inst<T> &P, const Tc &c, T *lds, 
 // The six iterate buffers rotate by pointer instead of being copied: acceptCandidate,
 // backup/restore and saveToPrev are pointer moves.
 template <typename T, int R, int V>
-__device__ void solveInstance(const Inst<T> &P, Out &out, T *lds, double *ldsd, double tickRate, int grid) {
+__device__ void solveInstance(const Inst<T> *Pp, Out &out, SPK_LDS T *lds, SPK_LDS double *ldsd, int grid) {
+    IP<T> P = *cst(uniformPtr(Pp));
     const Tc c = threadCtx(grid, P.gpart);
     const long n = P.sIter;
     const int m = P.andBuff;
     const bool gram = P.lsMethod == 1;
-    __shared__ double G[64], gb[8];
+    __shared__ double gramMat[64], gramRhs[8];
+    SPK_LDS double *G = (SPK_LDS double *) gramMat, *gb = (SPK_LDS double *) gramRhs;
     T *Z = P.z, *C = P.cand, *ZP = P.zPrev, *RR = P.res, *RP = P.resPrev, *BK = P.backup;
     T *D = P.dir, *DS = P.dirS;
     int head = m - 1;
@@ -1279,6 +1321,7 @@ __device__ void solveInstance(const Inst<T> &P, Out &out, T *lds, double *ldsd, 
         }
     }
     if (c.ltid < 64) G[c.ltid] = 0.;
+    if (c.ltid == 0) *gridSeq() = 0;
     sync(c);
     // a given tolerance (> 0) skips the reference's first-check calibration, so warm starts and
     // polish solves are accepted against the threshold of the cold solve they continue
@@ -1302,11 +1345,11 @@ __device__ void solveInstance(const Inst<T> &P, Out &out, T *lds, double *ldsd, 
             C = tmp;
         }
         clk.mark(PH_OTHER);
-        applyT<T, R, V>(P, c, Z, C, &clk);
+        applyT<T, R, V>(Pp, c, Z, C, &clk);
         nT++;
         // computeError (src/cache.cuh:910-961): r = z - cand
         if (P.dbg) {  // isFinite(candidate) (src/cache.cuh:912): stop at the first non-finite entry
-            const long bad = firstNonfinite<T>(C, n, lds, c);
+            const long bad = firstNonfinite<T>(C, n, lds, grid, P.gpart);
             if (bad >= 0) {
                 status = ST_NONFINITE;
                 iters = it;
@@ -1324,10 +1367,10 @@ __device__ void solveInstance(const Inst<T> &P, Out &out, T *lds, double *ldsd, 
             T mx;
             if (P.dbg) {
                 T split[2];
-                reduceEll<T, R, V, true>(P, c, RR, RR, lds, dotRR, mx, split);
-                debugRecord<T>(P, c, lds, it, 2 * nT, split, RR, C, nDbg);
+                reduceEll<T, R, V, true>(Pp, c, RR, RR, lds, dotRR, mx, split);
+                debugRecord<T>(Pp, grid, lds, it, 2 * nT, split, RR, C, nDbg);
             } else {
-                reduceEll<T, R, V>(P, c, RR, RR, lds, dotRR, mx);
+                reduceEll<T, R, V>(Pp, c, RR, RR, lds, dotRR, mx);
             }
             nEll++;
             haveDot = true;
@@ -1366,7 +1409,7 @@ __device__ void solveInstance(const Inst<T> &P, Out &out, T *lds, double *ldsd, 
         // normM(r) (src/cache.cuh:740-742)
         if (!haveDot) {
             T mx;
-            reduceEll<T, R, V>(P, c, RR, RR, lds, dotRR, mx);
+            reduceEll<T, R, V>(Pp, c, RR, RR, lds, dotRR, mx);
             nEll++;
             clk.mark(PH_ELL);
         }
@@ -1374,7 +1417,7 @@ __device__ void solveInstance(const Inst<T> &P, Out &out, T *lds, double *ldsd, 
         wLast = w;
         // delta iterate/residual, new Anderson column, then saveToPrev as pointer moves
         head = (head + 1) % m;
-        andersonColumn<T>(P, c, head, RR, RP, Z, ZP, gram, G, gb, ldsd);
+        andersonColumn<T>(Pp, grid, head, RR, RP, Z, ZP, gram, G, gb, ldsd);
         clk.mark(PH_ACOL);
         {
             T *tmp = ZP;
@@ -1393,13 +1436,13 @@ __device__ void solveInstance(const Inst<T> &P, Out &out, T *lds, double *ldsd, 
             if (gram) {
                 useLS = gramSolve(G, gb, m, gs);
             } else {
-                andersonHouseholder<T>(P, c, head, RP, lds, gs);
+                andersonHouseholder<T>(Pp, grid, head, RP, lds, gs);
                 useLS = true;
             }
         }
         clk.mark(PH_ALS);
         const bool blind = w <= c0 * zeta;
-        andersonApply<T>(P, c, gs, useLS, RP, ZP, blind ? C : D, blind);
+        andersonApply<T>(Pp, grid, gs, useLS, RP, ZP, blind ? C : D, blind);
         clk.mark(PH_AAPPLY);
         if (blind) {  // K0 blind update (src/cache.cuh:1055-1061)
             zeta = w;
@@ -1417,14 +1460,14 @@ __device__ void solveInstance(const Inst<T> &P, Out &out, T *lds, double *ldsd, 
                 });
             sync(c);
             clk.mark(PH_LINE);
-            applyT<T, R, V>(P, c, Z, C, &clk);
+            applyT<T, R, V>(Pp, c, Z, C, &clk);
             nT++;
             stream<8>(
                 n, c, [&](long k) { return V2<T>{Z[k], C[k]}; }, [&](long k, const V2<T> &v) { RR[k] = v.a - v.b; });
             sync(c);
             clk.mark(PH_RES);
             T dot, mx;
-            reduceEll<T, R, V>(P, c, RR, RR, lds, dot, mx);
+            reduceEll<T, R, V>(Pp, c, RR, RR, lds, dot, mx);
             nEll++;
             clk.mark(PH_ELL);
             const T wTilde = sqrt(dot);
@@ -1437,7 +1480,7 @@ __device__ void solveInstance(const Inst<T> &P, Out &out, T *lds, double *ldsd, 
                 break;
             }
             T dotRD;
-            reduceEll<T, R, V>(P, c, RR, DS, lds, dotRD, mx);
+            reduceEll<T, R, V>(Pp, c, RR, DS, lds, dotRD, mx);
             nEll++;
             clk.mark(PH_ELL);
             const T rho = wTilde * wTilde - dotRD;
@@ -1501,76 +1544,16 @@ __device__ void solveInstance(const Inst<T> &P, Out &out, T *lds, double *ldsd, 
     }
 }
 
-// Copies the instance descriptor into LDS and, when they fit in the dynamic LDS budget,
-// its per-node index arrays and tree arrays, repointing the copy at the LDS arrays.
-template <typename T>
-__device__ const Inst<T> &stageInstance(const Inst<T> &G, Inst<T> &L, int *pool, int poolInts) {
-    const Tc c = threadCtx();
-    if (c.tid == 0) L = G;
-    __syncthreads();
-    if (poolInts <= 0) return L;
-    int used = 0;
-    auto take = [&](const int *&p, int count) {
-        if (!p || count <= 0 || used + count > poolInts) return;
-        int *dst = pool + used;
-        for (int i = c.tid; i < count; i += c.nt) dst[i] = p[i];
-        used += count;
-        __syncthreads();
-        if (c.tid == 0) p = dst;
-        __syncthreads();
-    };
-    const int N = G.N, nl = G.nl, nlf = G.nlf;
-    take(L.anc, N);
-    take(L.chFrom, nl);
-    take(L.numCh, nl);
-    take(L.stageFrom, G.S);
-    take(L.stageTo, G.S);
-    take(L.BTr.idx, N);
-    take(L.AB.idx, N);
-    take(L.ABKTr.idx, N);
-    take(L.APB.idx, N);
-    take(L.sQ.idx, N);
-    take(L.sR.idx, N);
-    take(L.trans.idx, N);
-    take(L.q.idx, N);
-    take(L.r.idx, N);
-    take(L.K.idx, nl);
-    take(L.KTr.idx, nl);
-    take(L.RtInv.idx, nl);
-    take(L.cholL.idx, nl);
-    take(L.cholU.idx, nl);
-    take(L.NN.idx, nl);
-    take(L.b.idx, nl);
-    take(L.nLB.idx, nl);
-    take(L.nUB.idx, nl);
-    take(L.nG.idx, nl);
-    take(L.nGT.idx, nl);
-    take(L.lsQ.idx, nlf);
-    take(L.lq.idx, nlf);
-    take(L.ltrans.idx, nlf);
-    take(L.lLB.idx, nlf);
-    take(L.lUB.idx, nlf);
-    take(L.lG.idx, nlf);
-    take(L.lGT.idx, nlf);
-    take(L.e.idx, N);
-    take(L.Pe.idx, N);
-    return L;
-}
-
 // grid = 0: workgroup k solves instance k.  grid = 1 (cooperative launch, count = 1): every
 // workgroup works on instance 0.
 template <typename T, int R, int V>
 __global__ void __launch_bounds__(SPK_MAX_THREADS) k_solve(const Inst<T> *__restrict__ insts, Out *outs, int count,
-                                                double tickRate, int poolInts, int grid) {
+                                                int grid) {
     __shared__ T lds[8 * 32];
     __shared__ double ldsd[16 * 32];
-    __shared__ __align__(16) char localBuf[sizeof(Inst<T>)];
-    Inst<T> &local = *reinterpret_cast<Inst<T> *>(localBuf);
-    extern __shared__ int pool[];
     const int k = grid ? 0 : (int) blockIdx.x;
     if (k >= count) return;
-    const Inst<T> &P = stageInstance(insts[k], local, pool, poolInts);
-    solveInstance<T, R, V>(P, outs[P.slot], lds, ldsd, tickRate, grid);
+    solveInstance<T, R, V>(insts + k, outs[insts[k].slot], (SPK_LDS T *) lds, (SPK_LDS double *) ldsd, grid);
 }
 
 // ---------------------------------------------------------------- single-operator kernels
@@ -1579,31 +1562,30 @@ enum DebugOp { OP_L = 0, OP_LADJ = 1, OP_DYN = 2, OP_KERNEL = 3, OP_T = 4, OP_EL
 
 template <typename T, int R, int V>
 __global__ void __launch_bounds__(SPK_MAX_THREADS) k_debug(const Inst<T> *__restrict__ insts, Out *outs, int count, int op,
-                                                int poolInts, int grid) {
-    __shared__ T lds[8 * 32];
-    __shared__ __align__(16) char localBuf[sizeof(Inst<T>)];
-    Inst<T> &local = *reinterpret_cast<Inst<T> *>(localBuf);
-    extern __shared__ int pool[];
+                                                int grid) {
+    __shared__ T ldsBuf[8 * 32];
+    SPK_LDS T *lds = (SPK_LDS T *) ldsBuf;
     const int kInst = grid ? 0 : (int) blockIdx.x;
     if (kInst >= count) return;
-    const Inst<T> &P = stageInstance(insts[kInst], local, pool, poolInts);
+    const Inst<T> *Pp = insts + kInst;
+    IP<T> P = *cst(Pp);
     const Tc c = threadCtx(grid, P.gpart);
-    T *z = P.z, *cand = P.cand;
+    if (c.ltid == 0) *gridSeq() = 0;
+    __syncthreads();
+    GP<T> z = (GP<T>) P.z, cand = (GP<T>) P.cand;
     if (op == OP_L) {
         StoreL<T, R> h{P, cand + P.sPrim, c.lane};
-        auto pv = [&](long k) { return z[k]; };
+        auto pv = [&](long base, unsigned k) -> T { return (z + base)[k]; };
         for (int n = c.wave; n < P.N; n += c.nw) opNode<T, R, V>(P, n, c.lane, pv, h);
     } else if (op == OP_LADJ) {
-        const T *zd = z + P.sPrim;
         for (int n = c.wave; n < P.N; n += c.nw) {
             AdjOut<T, R> o;
-            adjNode<T, R, V>(P, zd, n, c.lane, o);
-            for (int rc = 0; rc < R; rc++) {
-                const int r = c.lane + 64 * rc;
-                if (r < P.nx) cand[P.oX + (long) n * P.nx + r] = o.x[rc];
-                if (n < P.nl && r < P.nu) cand[P.oU + (long) n * P.nu + r] = o.u[rc];
+            adjNode<T, R, V>(P, z + P.sPrim, n, c.lane, o);
+            eachRow<R>(P.nx, c.lane, [&](int rc, unsigned r) { cand[P.oX + (long) n * P.nx + r] = o.x[rc]; });
+            if (n < P.nl) {
+                eachRow<R>(P.nu, c.lane, [&](int rc, unsigned r) { cand[P.oU + (long) n * P.nu + r] = o.u[rc]; });
+                if (c.lane < (unsigned) P.yD) cand[P.oY + (long) n * P.yD + c.lane] = o.y;
             }
-            if (n < P.nl && c.lane < P.yD) cand[P.oY + (long) n * P.yD + c.lane] = o.y;
             if (c.lane == 0) {
                 cand[P.oS + n] = o.s;
                 cand[P.oT + n] = o.t;
@@ -1615,16 +1597,17 @@ __global__ void __launch_bounds__(SPK_MAX_THREADS) k_debug(const Inst<T> *__rest
         if (op == OP_DYN)
             for (int n = c.wave; n < P.N; n += c.nw)
                 if (n >= P.nl)
-                    for (int r = c.lane; r < P.nx; r += 64) P.qd[(long) n * P.nx + r] = -cand[P.oX + (long) n * P.nx + r];
+                    for (int r = c.lane; r < P.nx; r += 64)
+                        ((GP<T>) P.qd)[(long) n * P.nx + r] = -cand[P.oX + (long) n * P.nx + r];
         sync(c);
-        phaseProjections<T, R, V>(P, c, cand, op == OP_DYN, op == OP_KERNEL);
+        phaseProjections<T, R, V>(Pp, grid, P.cand, op == OP_DYN, op == OP_KERNEL);
     } else if (op == OP_T) {
-        applyT<T, R, V>(P, c, z, cand);
+        applyT<T, R, V>(Pp, c, P.z, P.cand);
     } else if (op == OP_DUAL) {  // Cache::getDual (src/cache.cuh:371-376): dual prox of the given primal
-        phaseDualProx<T, R, V>(P, c, z, cand);
+        phaseDualProx<T, R, V>(Pp, grid, P.z, P.cand);
     } else if (op == OP_ELL) {
         T dot, mx;
-        reduceEll<T, R, V>(P, c, z, cand, lds, dot, mx);
+        reduceEll<T, R, V>(Pp, c, P.z, P.cand, lds, dot, mx);
         if (c.tid == 0) {
             outs[P.slot].w = (double) dot;
             outs[P.slot].err = (double) mx;
@@ -1632,33 +1615,11 @@ __global__ void __launch_bounds__(SPK_MAX_THREADS) k_debug(const Inst<T> *__rest
     }
 }
 
-// Elementwise conversions used by the FP32-bulk / FP64-polish path.
-__global__ void k_f32_to_f64(const float *in, double *out, long n) {
-    for (long k = blockIdx.x * (long) blockDim.x + threadIdx.x; k < n; k += (long) gridDim.x * blockDim.x) out[k] = in[k];
-}
-
-__global__ void k_f64_to_f32(const double *in, float *out, long n) {
-    for (long k = blockIdx.x * (long) blockDim.x + threadIdx.x; k < n; k += (long) gridDim.x * blockDim.x) out[k] = (float) in[k];
-}
-
-template <typename T>
-__global__ void k_fill(T *p, T v, long n) {
-    for (long k = blockIdx.x * (long) blockDim.x + threadIdx.x; k < n; k += (long) gridDim.x * blockDim.x) p[k] = v;
-}
-
-// explicit instantiations: register chunk classes (R, V) = (1,1) for dims <= 64,
-// and (4,4) for dims <= 256
-#define SPK_INST(T, R, V)                                                                  \
-    template __global__ void k_solve<T, R, V>(const Inst<T> *, Out *, int, double, int, int); \
-    template __global__ void k_debug<T, R, V>(const Inst<T> *, Out *, int, int, int, int);
-SPK_INST(double, 1, 1)
-#ifndef SPK_FAST_BUILD
-SPK_INST(double, 4, 4)
-SPK_INST(float, 1, 1)
-SPK_INST(float, 4, 4)
-#endif
-#undef SPK_INST
-template __global__ void k_fill<double>(double *, double, long);
-template __global__ void k_fill<float>(float *, float, long);
+// Explicit instantiations: register chunk classes (R, V) = (1,1) for dims <= 64, and (4,4) for
+// dims <= 256.  The library compiles this file once per type and class (SPK_KERNEL_T, SPK_KERNEL_CLASS).
+template __global__ void k_solve<SPK_KERNEL_T, SPK_KERNEL_CLASS, SPK_KERNEL_CLASS>(const Inst<SPK_KERNEL_T> *, Out *, int,
+                                                                                 int);
+template __global__ void k_debug<SPK_KERNEL_T, SPK_KERNEL_CLASS, SPK_KERNEL_CLASS>(const Inst<SPK_KERNEL_T> *, Out *, int,
+                                                                                 int, int);
 
 }  // namespace spk

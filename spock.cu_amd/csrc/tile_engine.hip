@@ -103,7 +103,6 @@ struct TV {
 };
 
 // A wave's LDS staging slices.
-#define SPK_LDS __attribute__((address_space(3)))
 template <typename T>
 using SP = SPK_LDS T *;
 
