@@ -1055,7 +1055,7 @@ int spk_batch_create(spk_ctx *ctx, int count, spk_problem *const *problems, int 
         }
         b->coreElems = off;
         b->core.alloc(off * b->elSize());
-        check(hipMemset(b->core.p, 0, off * b->elSize()), "zero state");
+        check(hipMemsetAsync(b->core.p, 0, off * b->elSize(), ctx->stream), "zero state");
         b->x0Off.resize(count);
         off = 0;
         for (int k = 0; k < count; k++) {
@@ -1064,7 +1064,7 @@ int spk_batch_create(spk_ctx *ctx, int count, spk_problem *const *problems, int 
         }
         b->x0Elems = off;
         b->x0buf.alloc(off * b->elSize());
-        check(hipMemset(b->x0buf.p, 0, off * b->elSize()), "zero x0");
+        check(hipMemsetAsync(b->x0buf.p, 0, off * b->elSize(), ctx->stream), "zero x0");
         check(hipEventCreate(&b->ev0), "event");
         check(hipEventCreate(&b->ev1), "event");
         ensureAnderson(b.get(), 3);
@@ -1095,12 +1095,15 @@ int spk_batch_create_shared(spk_ctx *ctx, spk_problem *problem, int count, int d
         if (dtype == SPK_F64) ensureUploaded<double>(problem);
         else ensureUploaded<float>(problem);
         const size_t total = laneLayout(b.get());
+        // cleared on the batch's own stream, here and in resets: that stream does not wait for the null
+        // stream, so a relayout or a solve could otherwise read a region before it was cleared
         b->lbuf.alloc(total * b->elSize());
         b->lsave.alloc(sizeof(spk::LaneSave) * b->Bpad);
         b->lgsave.alloc(sizeof(spk::LaneGroupSave) * (b->Bpad / 16));  // one per workgroup of either engine
-        check(hipMemset(b->lbuf.p, 0, total * b->elSize()), "zero state");
+        check(hipMemsetAsync(b->lbuf.p, 0, total * b->elSize(), ctx->stream), "zero state");
         check(hipEventCreate(&b->ev0), "event");
         check(hipEventCreate(&b->ev1), "event");
+        check(hipStreamSynchronize(ctx->stream), "sync");
         *out = b.release();
         return 0;
     } catch (const std::exception &e) {
@@ -1161,7 +1164,7 @@ int spk_batch_set_debug(spk_batch *b, long max_records) {
             return 0;
         }
         b->dbgRec.alloc((size_t) b->count * max_records * spk::DBG_WORDS * sizeof(double));
-        check(hipMemset(b->dbgRec.p, 0, b->dbgRec.bytes), "zero debug records");
+        check(hipMemsetAsync(b->dbgRec.p, 0, b->dbgRec.bytes, b->ctx->stream), "zero debug records");
         b->dbgEOff.resize(b->count);
         size_t off = 0;
         for (int k = 0; k < b->count; k++) {
@@ -1169,7 +1172,8 @@ int spk_batch_set_debug(spk_batch *b, long max_records) {
             off += alignUp((size_t) b->probs[k]->hp.sPrim, 64);
         }
         b->dbgE.alloc(off * b->elSize());
-        check(hipMemset(b->dbgE.p, 0, b->dbgE.bytes), "zero debug vectors");
+        check(hipMemsetAsync(b->dbgE.p, 0, b->dbgE.bytes, b->ctx->stream), "zero debug vectors");
+        check(hipStreamSynchronize(b->ctx->stream), "sync");
         return 0;
     } catch (const std::exception &e) {
         return fail(b->ctx, e);
@@ -1203,12 +1207,14 @@ int spk_batch_reset(spk_batch *b) {
     try {
         check(hipStreamSynchronize(b->ctx->stream), "sync");
         if (b->lanes) {  // everything before the initial states
-            check(hipMemset(b->lbuf.p, 0, b->lRegion[LR_X0] * b->elSize()), "reset");
+            check(hipMemsetAsync(b->lbuf.p, 0, b->lRegion[LR_X0] * b->elSize(), b->ctx->stream), "reset");
+            check(hipStreamSynchronize(b->ctx->stream), "sync");
             return 0;
         }
-        check(hipMemset(b->core.p, 0, b->coreElems * b->elSize()), "reset");
-        if (b->anders.p) check(hipMemset(b->anders.p, 0, b->andElems * b->elSize()), "reset");
-        if (b->dbgE.p) check(hipMemset(b->dbgE.p, 0, b->dbgE.bytes), "reset");  // err0's vector (src/cache.cuh:469)
+        check(hipMemsetAsync(b->core.p, 0, b->coreElems * b->elSize(), b->ctx->stream), "reset");
+        if (b->anders.p) check(hipMemsetAsync(b->anders.p, 0, b->andElems * b->elSize(), b->ctx->stream), "reset");
+        if (b->dbgE.p) check(hipMemsetAsync(b->dbgE.p, 0, b->dbgE.bytes, b->ctx->stream), "reset");  // err0's vector (src/cache.cuh:469)
+        check(hipStreamSynchronize(b->ctx->stream), "sync");
         // the initial states are inputs of the next solve (spk_batch_set_x0) and stay; the
         // reference zeroes its copy because runSpock(x0) uploads x0 again (src/cache.cuh:448,1011)
         return 0;
@@ -2008,7 +2014,7 @@ int spk_batch_debug_op(spk_batch *b, int op, const double *in, double *out, doub
             spk_options o;
             spk_default_options(&o);
             b->dOut.alloc(sizeof(spk::Out) * b->count);
-            check(hipMemset(b->dOut.p, 0, sizeof(spk::Out) * b->count), "zero out");
+            check(hipMemsetAsync(b->dOut.p, 0, sizeof(spk::Out) * b->count, b->ctx->stream), "zero out");
             const dim3 grid((unsigned) (b->Bpad / b->laneW)), block(laneBlock(b, o));
             auto *outs = static_cast<spk::Out *>(b->dOut.p);
             const bool tile = b->laneW == 16;
@@ -2060,7 +2066,7 @@ int spk_batch_debug_op(spk_batch *b, int op, const double *in, double *out, doub
         spk_default_options(&o);
         ensureAnderson(b, o.anderson_buffer);
         b->dOut.alloc(sizeof(spk::Out) * b->count);
-        check(hipMemset(b->dOut.p, 0, sizeof(spk::Out) * b->count), "zero out");
+        check(hipMemsetAsync(b->dOut.p, 0, sizeof(spk::Out) * b->count, b->ctx->stream), "zero out");
         if (b->dtype == SPK_F64) {
             buildInsts<double>(b, o, 0);
             launchKernel<double>(b, 256, true, op);

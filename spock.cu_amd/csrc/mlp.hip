@@ -663,9 +663,9 @@ int spk_mlp_create(spk_ctx *ctx, int in, int hidden, int layers, int out, unsign
         m->m.alloc(off * 4);
         m->v.alloc(off * 4);
         check(hipMemcpy(m->w.p, p.data(), off * 4, hipMemcpyHostToDevice), "params");
-        check(hipMemset(m->g.p, 0, off * 4), "zero");
-        check(hipMemset(m->m.p, 0, off * 4), "zero");
-        check(hipMemset(m->v.p, 0, off * 4), "zero");
+        check(hipMemsetAsync(m->g.p, 0, off * 4, ctx->stream), "zero");
+        check(hipMemsetAsync(m->m.p, 0, off * 4, ctx->stream), "zero");
+        check(hipMemsetAsync(m->v.p, 0, off * 4, ctx->stream), "zero");
         refreshBf16(m.get());
         m->hInMean.assign(in, 0.f);
         m->hInStd.assign(in, 1.f);
