@@ -265,15 +265,22 @@ __device__ void lockstepSolve(const LaneInst<T> *Pp, Out *outs, double *lds, lon
         T sRR;
         const bool spock = P.method == METHOD_SPOCK;
         if (spock) head = (head + 1) % m;
-        if (!spock) {  // r = z - T(z) and ||r||^2
+        const bool checkIt = (it - it0) % P.checkPeriod == 0;
+        if (!spock) {
+            // r = z - T(z): of the plain method only the error checks read it, and the iteration cap, which
+            // outputs the residual of the iteration before it
+            if (!anyLane(active && (checkIt || it - it0 + 1 >= hardCap))) {
+                T *t = Z;
+                Z = C;
+                C = t;
+                clk.mark(PH_RES);
+                continue;
+            }
             const VW rr = V(RR), z = V(Z), cc = V(C);
-            T acc = T(0);
-            E::template pass<16>(n, c, [&](long e) { return V2<T>{z[e], cc[e]}; }, [&](long e, const V2<T> &v) {
-                const T d = v.a - v.b;
-                rr[e] = d;
-                acc += d * d;
-            });
-            sRR = (T) E::sum((double) acc, lds, c);
+            E::template pass<16>(n, c, [&](long e) { return V2<T>{z[e], cc[e]}; },
+                                 [&](long e, const V2<T> &v) { rr[e] = v.a - v.b; });
+            __syncthreads();
+            sRR = T(0);
         } else {
             // r = z - T(z), ||r||^2 and, in the same pass, the new Anderson column
             // (src/cache.cuh:861-896) with its Gram entries: Y_head = r - r_prev,
@@ -336,17 +343,16 @@ __device__ void lockstepSolve(const LaneInst<T> *Pp, Out *outs, double *lds, lon
         }
         clk.mark(PH_RES);
         // <r, M r> = ||r||^2 - 2 gamma r_p . L* r_d; the full [L*; L] only at the error checks
-        const bool checkIt = (it - it0) % P.checkPeriod == 0;
-        T mx = T(0), crossRR;
+        T mx = T(0), crossRR = T(0);
         if (anyLane(active && checkIt)) {
             const DotMax<T> dm = E::reduceEll(Pp, RR, RR, lds);
             mx = dm.mx;
             crossRR = dm.cross;
-        } else {
+        } else if (spock) {
             crossRR = E::adjDots(Pp, RR, RR, lds, false).c1;
         }
         const T dotRR = sRR - T(2) * P.gamma * crossRR;
-        if (active) nEll++;
+        if (active && (spock || checkIt)) nEll++;
         clk.mark(PH_ELL);
         bool done = false;
         if (active && checkIt) {  // computeError (src/cache.cuh:910-961)
