@@ -833,7 +833,7 @@ size_t uniformCoreStride(const spk_batch *b) {
 template <typename S, typename D>
 void launchInterleave(const spk_batch *src, spk_batch *dst, size_t n) {
     const size_t stride = uniformCoreStride(src);
-    hipLaunchKernelGGL((spk::k_interleave<S, D>), dim3(1024), dim3(256), 0, dst->ctx->stream,
+    hipLaunchKernelGGL((spk::k_interleave<S, D>), dim3(4096), dim3(256), 0, dst->ctx->stream,
                        static_cast<const S *>(src->core.p), (long) stride, lanePtr<D>(dst, LR_ZIO), (long) n,
                        dst->count, (long) dst->laneW);
 }
@@ -841,7 +841,7 @@ void launchInterleave(const spk_batch *src, spk_batch *dst, size_t n) {
 template <typename S, typename D>
 void launchDeinterleave(const spk_batch *src, spk_batch *dst, size_t n) {
     const size_t stride = uniformCoreStride(dst);
-    hipLaunchKernelGGL((spk::k_deinterleave<S, D>), dim3(1024), dim3(256), 0, dst->ctx->stream,
+    hipLaunchKernelGGL((spk::k_deinterleave<S, D>), dim3(4096), dim3(256), 0, dst->ctx->stream,
                        lanePtr<S>(src, LR_ZIO), (long) src->laneW, static_cast<D *>(dst->core.p), (long) stride, (long) n,
                        dst->count);
 }
@@ -1381,11 +1381,11 @@ int spk_batch_set_iterates_device(spk_batch *b, const float *src, long ld) {
         hipStream_t st = b->ctx->stream;
         if (b->lanes) {
             if (b->dtype == SPK_F64) {
-                hipLaunchKernelGGL((spk::k_interleave<float, double>), dim3(1024), dim3(256), 0, st, src, ld,
+                hipLaunchKernelGGL((spk::k_interleave<float, double>), dim3(4096), dim3(256), 0, st, src, ld,
                                    lanePtr<double>(b, LR_ZIO), (long) n, b->count, (long) b->laneW);
                 fillDevice<double>(b, lanePtr<double>(b, LR_RIO), n * b->Bpad);
             } else {
-                hipLaunchKernelGGL((spk::k_interleave<float, float>), dim3(1024), dim3(256), 0, st, src, ld,
+                hipLaunchKernelGGL((spk::k_interleave<float, float>), dim3(4096), dim3(256), 0, st, src, ld,
                                    lanePtr<float>(b, LR_ZIO), (long) n, b->count, (long) b->laneW);
                 fillDevice<float>(b, lanePtr<float>(b, LR_RIO), n * b->Bpad);
             }
@@ -1421,10 +1421,10 @@ int spk_batch_get_iterates_device(spk_batch *b, float *dst, long ld) {
         check(hipStreamSynchronize(st), "sync");
         if (b->lanes) {
             if (b->dtype == SPK_F64)
-                hipLaunchKernelGGL((spk::k_deinterleave<double, float>), dim3(1024), dim3(256), 0, st,
+                hipLaunchKernelGGL((spk::k_deinterleave<double, float>), dim3(4096), dim3(256), 0, st,
                                    lanePtr<double>(b, LR_ZIO), (long) b->laneW, dst, ld, (long) n, b->count);
             else
-                hipLaunchKernelGGL((spk::k_deinterleave<float, float>), dim3(1024), dim3(256), 0, st,
+                hipLaunchKernelGGL((spk::k_deinterleave<float, float>), dim3(4096), dim3(256), 0, st,
                                    lanePtr<float>(b, LR_ZIO), (long) b->laneW, dst, ld, (long) n, b->count);
         } else {
             for (int k = 0; k < b->count; k++) {

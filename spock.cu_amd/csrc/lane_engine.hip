@@ -892,22 +892,83 @@ template __global__ void SPK_LANE_KERNEL(k_lane_debug)<double>(const LaneInst<do
 #if SPK_MV_XB == 0
 // [instance][element] rows (leading dimension ld) to the block-interleaved layout of a region of
 // n rows and back, with dtype conversion.
-template <typename S, typename D>
-__global__ void k_interleave(const S *__restrict__ in, long ld, D *__restrict__ out, long n, int count, long w) {
-    const long total = n * (long) count;
-    for (long t = blockIdx.x * (long) blockDim.x + threadIdx.x; t < total; t += (long) gridDim.x * blockDim.x) {
-        const long b = t % count, e = t / count;
-        out[laneIndex(n, e, b, w)] = (D) in[b * ld + e];
+// Transposition between instance rows and interleaved blocks, bound by HBM.  A workgroup moves tiles
+// of one block of w (16 or 64) instances by 4096 / w elements through LDS, so both sides are read and
+// written in runs of 64 words (before: one side in single words 4 n bytes apart, 1.41 and 1.83 ms for the
+// 4,096 FP32 iterates of the 229-node problem, 0.37 ms at the copy rate; now 0.35 and 0.40 ms).  A thread's
+// 16 words are requested together (clamped, not conditional).  The LDS row stride puts the w instances
+// of an element, and the next elements a wave reaches, in different banks.
+constexpr int XT_WORDS = 16 * (256 + 4);  // at least 64 * (64 + 1)
+
+struct XTile {
+    long b0, e0;
+    int nb, ne, lw, lE, stride;  // lw, lE: log2 of the block width and of the tile's elements
+};
+
+template <typename F>
+__device__ __forceinline__ void forTiles(long n, int count, long w, F f) {
+    XTile x;
+    x.lw = w == 16 ? 4 : 6;
+    x.lE = 12 - x.lw;
+    x.stride = w == 16 ? 256 + 4 : 64 + 1;
+    const long tilesE = (n + (1 << x.lE) - 1) >> x.lE, tiles = tilesE * ((count + w - 1) >> x.lw);
+    for (long t = blockIdx.x; t < tiles; t += gridDim.x) {
+        x.b0 = t / tilesE * w;
+        x.e0 = t % tilesE << x.lE;
+        x.nb = (int) min(w, count - x.b0);
+        x.ne = (int) min(1L << x.lE, n - x.e0);
+        f(x);
+        __syncthreads();
     }
 }
 
 template <typename S, typename D>
-__global__ void k_deinterleave(const S *__restrict__ in, long w, D *__restrict__ out, long ld, long n, int count) {
-    const long total = n * (long) count;
-    for (long t = blockIdx.x * (long) blockDim.x + threadIdx.x; t < total; t += (long) gridDim.x * blockDim.x) {
-        const long e = t % n, b = t / n;
-        out[b * ld + e] = (D) in[laneIndex(n, e, b, w)];
-    }
+__global__ void __launch_bounds__(256) k_interleave(const S *__restrict__ in, long ld, D *__restrict__ out, long n,
+                                                    int count, long w) {
+    __shared__ D tile[XT_WORDS];
+    forTiles(n, count, w, [&](const XTile &x) {
+        S v[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int t = threadIdx.x + 256 * i, b = min(t >> x.lE, x.nb - 1), e = min(t & ((1 << x.lE) - 1), x.ne - 1);
+            v[i] = in[(x.b0 + b) * ld + x.e0 + e];
+        }
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int t = threadIdx.x + 256 * i;
+            tile[(t >> x.lE) * x.stride + (t & ((1 << x.lE) - 1))] = (D) v[i];
+        }
+        __syncthreads();
+        D *dst = out + laneIndex(n, x.e0, x.b0, w);
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int t = threadIdx.x + 256 * i, b = t & ((1 << x.lw) - 1), e = t >> x.lw;
+            if (b < x.nb && e < x.ne) dst[t] = tile[b * x.stride + e];
+        }
+    });
+}
+
+template <typename S, typename D>
+__global__ void __launch_bounds__(256) k_deinterleave(const S *__restrict__ in, long w, D *__restrict__ out, long ld, long n,
+                                                      int count) {
+    __shared__ D tile[XT_WORDS];
+    forTiles(n, count, w, [&](const XTile &x) {
+        const S *src = in + laneIndex(n, x.e0, x.b0, w);
+        S v[16];
+#pragma unroll
+        for (int i = 0; i < 16; i++) v[i] = src[min((int) threadIdx.x + 256 * i, (x.ne << x.lw) - 1)];
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int t = threadIdx.x + 256 * i;
+            tile[(t & ((1 << x.lw) - 1)) * x.stride + (t >> x.lw)] = (D) v[i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int t = threadIdx.x + 256 * i, b = t >> x.lE, e = t & ((1 << x.lE) - 1);
+            if (b < x.nb && e < x.ne) out[(x.b0 + b) * ld + x.e0 + e] = tile[b * x.stride + e];
+        }
+    });
 }
 
 // A region of n rows from blocks of win instances to blocks of wout instances (all padded slots).
