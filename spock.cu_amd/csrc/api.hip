@@ -196,8 +196,9 @@ void uploadTable(spk_problem *p, const std::string &name, const Table &t) {
     s.rows = t.rows;
     s.cols = t.cols;
     std::vector<T> d(t.data.begin(), t.data.end());
-    // 64 zero elements of padding: the lane engine reads fixed row blocks past a table's end
-    d.resize(d.size() + 64, T(0));
+    // zero padding: the engines read fixed row blocks (up to 64 elements) and, in the fused engine, up to 7
+    // columns past a table's end
+    d.resize(d.size() + 64 + (size_t) 8 * t.rows, T(0));
     s.data = std::make_unique<DevBuf>();
     s.data->alloc(d.size() * sizeof(T));
     check(hipMemcpy(s.data->p, d.data(), d.size() * sizeof(T), hipMemcpyHostToDevice), "upload table");

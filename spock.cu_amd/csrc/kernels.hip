@@ -6,8 +6,7 @@
 // same branch decisions).
 //
 // Work decomposition inside the workgroup: a "node task" is handled by one 64-lane
-// wavefront with lanes over the rows of the node's blocks (node data are column major,
-// so every matrix column is one coalesced load); stage-sequential sweeps are separated
+// wavefront with lanes over the rows of the node's blocks; stage-sequential sweeps are separated
 // by workgroup barriers; iterate-wide passes are block-strided; reductions use
 // cross-lane shuffles and an LDS combine in a fixed order (bitwise repeatable).
 //
@@ -18,6 +17,8 @@
 #include <hip/hip_cooperative_groups.h>
 #include <hip/hip_runtime.h>
 #include <math.h>
+
+#include <utility>
 
 #ifndef SPK_MAX_THREADS
 #define SPK_MAX_THREADS 512
@@ -68,6 +69,7 @@ __device__ __forceinline__ GP<T> glb(T *p) {
 // instance (the workgroup, or the whole grid in grid mode); ltid/lw/lnw are workgroup-local.
 struct Tc {
     unsigned lane;
+    unsigned row;  // the row of a node's blocks (of each 64) this lane holds
     int wave, nw, tid, nt;
     int ltid, lw, lnw;
     int grid;
@@ -84,6 +86,7 @@ __device__ __forceinline__ Tc threadCtx(int grid = 0, void *gpart = nullptr) {
     c.tid = c.grid ? (int) (blockIdx.x * blockDim.x + threadIdx.x) : c.ltid;
     c.nt = c.grid ? (int) (gridDim.x * blockDim.x) : (int) blockDim.x;
     c.lane = threadIdx.x & 63;
+    c.row = 4 * (c.lane & 15) + (c.lane >> 4);  // rowOf
     c.wave = c.grid ? (int) blockIdx.x * c.lnw + c.lw : c.lw;
     c.nw = c.nt >> 6;
     return c;
@@ -150,74 +153,156 @@ __device__ __forceinline__ void zero(T (&a)[K]) {
     for (int i = 0; i < K; i++) a[i] = T(0);
 }
 
-// v[c] holds element lane + 64 c of a vector of length len (0 beyond)
+// v[c] holds element row + 64 c of a vector of length len (0 beyond)
 template <typename T, int V, typename F>
-__device__ __forceinline__ void loadV(T (&v)[V], int len, unsigned lane, F f) {
+__device__ __forceinline__ void loadV(T (&v)[V], int len, unsigned row, F f) {
 #pragma unroll
     for (int c = 0; c < V; c++) {
-        const unsigned k = lane + 64 * c;
+        const unsigned k = row + 64 * c;
         v[c] = T(0);
         if (64 * c < len && k < (unsigned) len) v[c] = f(k);
     }
 }
 
 template <typename T, int V, typename P>
-__device__ __forceinline__ void loadPtr(T (&v)[V], P p, int len, unsigned lane) {
-    loadV(v, len, lane, [&](unsigned k) -> T { return p[k]; });
+__device__ __forceinline__ void loadPtr(T (&v)[V], P p, int len, unsigned row) {
+    loadV(v, len, row, [&](unsigned k) -> T { return p[k]; });
 }
 
-// acc[rc] (row lane + 64 rc) += sum_{c < n} M[row + c * ld] * v(c) in column order, n <= U columns,
-// RR row chunks.  All columns are requested before any is consumed, so this costs one memory round
-// trip.  Loads are unconditional: rows past the end repeat the last row (outputs nobody reads),
-// columns past the end repeat the last column against v = 0, and whole blocks of 8 columns past the
-// end are skipped by scalar branches.
-template <typename T, int RR, int U, int R>
-__device__ __forceinline__ void mvBlock(T (&acc)[R], CP<T> M, const unsigned (&row)[RR], int ld, int n, T v, int v0) {
-    T m[U][RR];
-#pragma unroll
-    for (int b = 0; b < U; b += 8) {
-        if (b < n) {
-            CP<T> col = M + (size_t) b * ld;
-#pragma unroll
-            for (int u = b; u < b + 8; u++) {
-#pragma unroll
-                for (int rc = 0; rc < RR; rc++) m[u][rc] = col[row[rc]];
-                col += u + 1 < n ? ld : 0;
-            }
-        }
-    }
-#pragma unroll
-    for (int b = 0; b < U; b += 8) {
-        if (b < n) {
-#pragma unroll
-            for (int u = b; u < b + 8; u++) {
-                const T xc = bcastLane(v, v0 + u);
-#pragma unroll
-                for (int rc = 0; rc < RR; rc++) acc[rc] += m[u][rc] * xc;
-            }
-        }
-    }
+// ------------------------------------------------------------------ products of a node
+// Rows of a node's blocks sit in lanes by rowOf(): lane 16 g + q holds row 4 q + g of each 64.  A
+// product y += M v (M column major, up to 64 columns) then runs as four column groups of 16 lanes:
+// lane 16 g + q loads rows 4 q .. 4 q + 3 of columns g, g + 4, ... (16 bytes a load in FP32, two such
+// loads in FP64), the vector entry it needs, v[4 s + g], is in lane s of its own 16 (a row broadcast),
+// and the four groups' sums meet in two swaps between lane rows that leave row 4 q + g in lane
+// 16 g + q again.  This is bound by instruction issue and latency, so what counts is that a step of
+// four columns is one or two loads, a broadcast and four multiply-adds (one column at a time with
+// lanes over rows: 15 instructions a column; T of the 229-node FP64 instance in one workgroup
+// 1.22 ms, now 0.75).  All loads of a chunk are issued before the first is used and none is
+// conditional: rows past the end repeat the last four, and up to 7 columns past the end are read
+// against v = 0 (the tables are padded for it) before the remaining blocks of 8 columns are skipped.
+__device__ __forceinline__ unsigned rowOf(unsigned lane) { return 4 * (lane & 15) + (lane >> 4); }
+__device__ __forceinline__ int laneOf(int row) { return 16 * (row & 3) + (row >> 2); }  // row < 64
+
+template <int S>
+__device__ __forceinline__ float rowBcast(float v) {  // lane S of each 16
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + S, 0xf, 0xf, true));
+}
+template <int S>
+__device__ __forceinline__ double rowBcast(double v) {
+    return __longlong_as_double(__builtin_amdgcn_update_dpp(0LL, __double_as_longlong(v), 0x150 + S, 0xf, 0xf, true));
 }
 
-// One 64-column chunk (cols <= 64) of RR row chunks.  Never inlined: a product is a few KB of
-// straight-line code, and with a copy at each of its call sites the phases of a solve missed the
-// instruction cache all the time (229-node FP64 instance, 32 workgroups: 1.6 ms of tree sweeps per
-// application of T inlined, 0.28 ms called).
+// Four consecutive rows of a column, at element alignment.
+template <typename T>
+struct Quad;
+template <>
+struct Quad<float> {
+    typedef float V __attribute__((ext_vector_type(4), aligned(4)));
+    V a;
+    __device__ __forceinline__ void load(CP<float> p) { a = *(const SPK_CONST V *) p; }
+    __device__ __forceinline__ float get(int i) const { return a[i]; }
+};
+template <>
+struct Quad<double> {
+    typedef double V __attribute__((ext_vector_type(2), aligned(8)));
+    V a, b;
+    __device__ __forceinline__ void load(CP<double> p) {
+        a = *(const SPK_CONST V *) p;
+        b = *(const SPK_CONST V *) (p + 2);
+    }
+    __device__ __forceinline__ double get(int i) const { return i < 2 ? a[i] : b[i - 2]; }
+};
+
+// a + b where both hold values of both 32-lane halves (16-lane rows): lanes of the lower half (even
+// rows) get the sum of a over the pair, the others the sum of b.
+__device__ __forceinline__ float halfSum32(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float halfSum16(float a, float b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ double halfSum32(double a, double b) {
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+__device__ __forceinline__ double halfSum16(double a, double b) {
+    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+
 template <typename T, int RR>
 struct RowVals {
     T a[RR];
 };
 
+// p[rc][i] += the columns 4 (S0 + s) + g, s < NS, of four rows, of a chunk with `cols` columns.
+template <typename T, int RR, int S0, int NS>
+__device__ __forceinline__ void mvSteps(T (&p)[RR][4], CP<T> M, const unsigned (&off)[RR], int ld, int cols, T v) {
+    Quad<T> m[NS][RR];
+#pragma unroll
+    for (int s = 0; s < NS; s += 2) {
+        if (4 * (S0 + s) < cols) {
+#pragma unroll
+            for (int u = s; u < s + 2; u++) {
+                CP<T> col = M + (size_t) (4 * (S0 + u)) * ld;
+#pragma unroll
+                for (int rc = 0; rc < RR; rc++) m[u][rc].load(col + off[rc]);
+            }
+        }
+    }
+    [&]<int... B>(std::integer_sequence<int, B...>) {
+        ([&] {
+            if (4 * (S0 + 2 * B) < cols) {
+                const T x0 = rowBcast<S0 + 2 * B>(v), x1 = rowBcast<S0 + 2 * B + 1>(v);
+#pragma unroll
+                for (int rc = 0; rc < RR; rc++) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) p[rc][i] += m[2 * B][rc].get(i) * x0;
+#pragma unroll
+                    for (int i = 0; i < 4; i++) p[rc][i] += m[2 * B + 1][rc].get(i) * x1;
+                }
+            }
+        }(), ...);
+    }(std::make_integer_sequence<int, NS / 2>{});
+}
+
+// acc + M v over one chunk of up to 64 columns, RR chunks of 64 rows.  Never inlined: with a copy of
+// this code at each of its call sites the phases of a solve missed the instruction cache all the time
+// (229-node FP64 instance, 32 workgroups, one column at a time: 1.6 ms of tree sweeps per application
+// of T inlined, 0.28 ms called).
 template <typename T, int RR>
 __device__ __noinline__ RowVals<T, RR> mvChunk(RowVals<T, RR> acc, const T *Mp, int rows, int ldIn, int colsIn, T v) {
-    constexpr int U = RR == 1 ? 64 : 64 / RR;  // up to 128 registers of matrix entries in FP64
     CP<T> M = cst(uniformPtr(Mp));
     const int ld = __builtin_amdgcn_readfirstlane(ldIn), cols = __builtin_amdgcn_readfirstlane(colsIn);
-    unsigned row[RR];
+    const unsigned lane = threadIdx.x & 63, q = lane & 15, g = lane >> 4;
+    unsigned off[RR];
+    T p[RR][4];
 #pragma unroll
-    for (int rc = 0; rc < RR; rc++) row[rc] = min((threadIdx.x & 63) + 64 * rc, (unsigned) rows - 1);
-#pragma unroll 1
-    for (int c0 = 0; c0 < cols; c0 += U) mvBlock<T, RR, U>(acc.a, M + (size_t) c0 * ld, row, ld, cols - c0, v, c0);
+    for (int rc = 0; rc < RR; rc++) {
+        off[rc] = min(64 * rc + 4 * q, ((unsigned) rows - 1) & ~3u) + g * ld;
+#pragma unroll
+        for (int i = 0; i < 4; i++) p[rc][i] = T(0);
+    }
+    // up to 128 registers of matrix entries in flight in FP64
+    if constexpr (RR == 1) {
+        mvSteps<T, RR, 0, 16>(p, M, off, ld, cols, v);
+    } else if constexpr (RR == 2) {
+        mvSteps<T, RR, 0, 8>(p, M, off, ld, cols, v);
+        if (32 < cols) mvSteps<T, RR, 8, 8>(p, M, off, ld, cols, v);
+    } else {
+        mvSteps<T, RR, 0, 4>(p, M, off, ld, cols, v);
+        if (16 < cols) mvSteps<T, RR, 4, 4>(p, M, off, ld, cols, v);
+        if (32 < cols) mvSteps<T, RR, 8, 4>(p, M, off, ld, cols, v);
+        if (48 < cols) mvSteps<T, RR, 12, 4>(p, M, off, ld, cols, v);
+    }
+#pragma unroll
+    for (int rc = 0; rc < RR; rc++)
+        acc.a[rc] += halfSum16(halfSum32(p[rc][0], p[rc][2]), halfSum32(p[rc][1], p[rc][3]));
     return acc;
 }
 
@@ -234,10 +319,10 @@ __device__ __forceinline__ void mvRows(T (&acc)[R], CP<T> M, int rows, int ld, i
     for (int rc = 0; rc < RR; rc++) acc[rc] = a.a[rc];
 }
 
-// acc[rc] (row lane + 64 rc) += sum_{c < cols} M[row + c * ld] * v(c), M column major, v 0 beyond
-// its length.
+// acc[rc] (row rowOf(lane) + 64 rc) += sum_{c < cols} M[row + c * ld] * v(c), M column major, v 0
+// beyond its length.
 template <typename T, int R, int V>
-__device__ __forceinline__ void mvAcc(T (&acc)[R], CP<T> M, int rows, int ld, int cols, const T (&v)[V], unsigned) {
+__device__ __forceinline__ void mvAcc(T (&acc)[R], CP<T> M, int rows, int ld, int cols, const T (&v)[V]) {
     if constexpr (R == 1) {
         mvRows<T, 1>(acc, M, rows, ld, cols, v);
     } else {
@@ -292,12 +377,12 @@ __device__ __forceinline__ T projBox(T v, T lb, T ub) {
     return v * T(1 - lower) * T(1 - upper) + lbi + ubi;
 }
 
-// f(rc, r) for every row r = lane + 64 rc < rows of this lane.
+// f(rc, r) for every row r = row + 64 rc < rows of this row.
 template <int R, typename F>
-__device__ __forceinline__ void eachRow(int rows, unsigned lane, F f) {
+__device__ __forceinline__ void eachRow(int rows, unsigned row, F f) {
 #pragma unroll
     for (int rc = 0; rc < R; rc++) {
-        const unsigned r = lane + 64 * rc;
+        const unsigned r = row + 64 * rc;
         if (64 * rc < rows && r < (unsigned) rows) f(rc, r);
     }
 }
@@ -309,12 +394,12 @@ template <typename T, int R>
 struct AdjOut {
     T x[R];  // rows nx
     T u[R];  // rows nu (nonleaf only)
-    T y;        // lane < yD (nonleaf only)
+    T y;        // row < yD (nonleaf only)
     T s, t;     // uniform scalars
 };
 
 template <typename T, int R, int V>
-__device__ __forceinline__ void adjNode(IP<T> P, GP<T> dual, int n, unsigned lane, AdjOut<T, R> &o) {
+__device__ __forceinline__ void adjNode(IP<T> P, GP<T> dual, int n, unsigned row, AdjOut<T, R> &o) {
     const int nx = P.nx, nu = P.nu, nxu = nx + nu, d4 = nxu + 2;
     zero(o.x);
     zero(o.u);
@@ -325,17 +410,17 @@ __device__ __forceinline__ void adjNode(IP<T> P, GP<T> dual, int n, unsigned lan
     if (n < P.nl) {
         const T II = dual[P.oII + n];
         o.s = II;
-        if (lane < (unsigned) P.yD) o.y = (dual + (P.oI + (long) n * P.yD))[lane] - tab(P.b, n)[lane] * II;
+        if (row < (unsigned) P.yD) o.y = (dual + (P.oI + (long) n * P.yD))[row] - tab(P.b, n)[row] * II;
         GP<T> d3 = dual + (P.oIII + (long) n * P.con3);
         if (P.ncon == CON_RECT_DEV) {
-            eachRow<R>(nx, lane, [&](int rc, unsigned r) { o.x[rc] = d3[r]; });
+            eachRow<R>(nx, row, [&](int rc, unsigned r) { o.x[rc] = d3[r]; });
             GP<T> d3u = d3 + nx;
-            eachRow<R>(nu, lane, [&](int rc, unsigned r) { o.u[rc] = d3u[r]; });
+            eachRow<R>(nu, row, [&](int rc, unsigned r) { o.u[rc] = d3u[r]; });
         } else if (P.ncon == CON_POLY_DEV) {
-            loadPtr(v, d3, P.con3, lane);
+            loadPtr(v, d3, P.con3, row);
             CP<T> GT = tab(P.nGT, n);
-            mvAcc(o.x, GT, nx, nxu, P.con3, v, lane);
-            mvAcc(o.u, GT + nx, nu, nxu, P.con3, v, lane);
+            mvAcc(o.x, GT, nx, nxu, P.con3, v);
+            mvAcc(o.u, GT + nx, nu, nxu, P.con3, v);
         }
         const int c0 = cst(P.chFrom)[n], nc = cst(P.numCh)[n];
 #pragma unroll 1
@@ -344,27 +429,27 @@ __device__ __forceinline__ void adjNode(IP<T> P, GP<T> dual, int n, unsigned lan
             if (P.ncost == COST_LIN_DEV) {  // x_i += q_j sum_j, u_i += r_j sum_j (src/costs.cuh:274-285)
                 const T sj = dual[P.oIV + j];
                 CP<T> qj = tab(P.q, j), rj = tab(P.r, j);
-                eachRow<R>(nx, lane, [&](int rc, unsigned r) { o.x[rc] += qj[r] * sj; });
-                eachRow<R>(nu, lane, [&](int rc, unsigned r) { o.u[rc] += rj[r] * sj; });
+                eachRow<R>(nx, row, [&](int rc, unsigned r) { o.x[rc] += qj[r] * sj; });
+                eachRow<R>(nu, row, [&](int rc, unsigned r) { o.u[rc] += rj[r] * sj; });
                 continue;
             }
             GP<T> iv = dual + (P.oIV + (long) j * d4);
             const T a = iv[nxu], bb = iv[nxu + 1];
-            loadPtr(v, iv, nx, lane);
+            loadPtr(v, iv, nx, row);
             zero(w);
-            mvAcc(w, tab(P.sQ, j), nx, nx, nx, v, lane);
+            mvAcc(w, tab(P.sQ, j), nx, nx, nx, v);
             if (P.ncost == COST_QUADLIN_DEV) {
                 CP<T> qj = tab(P.q, j);
-                eachRow<R>(nx, lane, [&](int rc, unsigned r) { w[rc] = w[rc] - T(0.5) * qj[r] * a - T(0.5) * qj[r] * bb; });
+                eachRow<R>(nx, row, [&](int rc, unsigned r) { w[rc] = w[rc] - T(0.5) * qj[r] * a - T(0.5) * qj[r] * bb; });
             }
 #pragma unroll
             for (int rc = 0; rc < R; rc++) o.x[rc] += w[rc];
-            loadPtr(v, iv + nx, nu, lane);
+            loadPtr(v, iv + nx, nu, row);
             zero(w);
-            mvAcc(w, tab(P.sR, j), nu, nu, nu, v, lane);
+            mvAcc(w, tab(P.sR, j), nu, nu, nu, v);
             if (P.ncost == COST_QUADLIN_DEV) {
                 CP<T> rj = tab(P.r, j);
-                eachRow<R>(nu, lane, [&](int rc, unsigned r) { w[rc] = w[rc] - T(0.5) * rj[r] * a - T(0.5) * rj[r] * bb; });
+                eachRow<R>(nu, row, [&](int rc, unsigned r) { w[rc] = w[rc] - T(0.5) * rj[r] * a - T(0.5) * rj[r] * bb; });
             }
 #pragma unroll
             for (int rc = 0; rc < R; rc++) o.u[rc] += w[rc];
@@ -373,27 +458,27 @@ __device__ __forceinline__ void adjNode(IP<T> P, GP<T> dual, int n, unsigned lan
         const int l = n - P.nl;
         GP<T> d5 = dual + (P.oV + (long) l * P.con5);
         if (P.lcon == CON_RECT_DEV) {
-            eachRow<R>(nx, lane, [&](int rc, unsigned r) { o.x[rc] = d5[r]; });
+            eachRow<R>(nx, row, [&](int rc, unsigned r) { o.x[rc] = d5[r]; });
         } else if (P.lcon == CON_POLY_DEV) {
-            loadPtr(v, d5, P.con5, lane);
-            mvAcc(o.x, tab(P.lGT, l), nx, nx, P.con5, v, lane);
+            loadPtr(v, d5, P.con5, row);
+            mvAcc(o.x, tab(P.lGT, l), nx, nx, P.con5, v);
         }
         if (P.lcost == COST_LIN_DEV) {  // x_l += q sum_l, s_l = set_l (src/costs.cuh:289-292)
             const T sl = dual[P.oVI + l];
             CP<T> lq = tab(P.lq, l);
-            eachRow<R>(nx, lane, [&](int rc, unsigned r) { o.x[rc] += lq[r] * sl; });
+            eachRow<R>(nx, row, [&](int rc, unsigned r) { o.x[rc] += lq[r] * sl; });
             o.s = dual[P.oVI + P.nlf + l];
         } else {
             GP<T> vi = dual + (P.oVI + (long) l * (nx + 2));
             const T a = vi[nx], bb = vi[nx + 1];
-            loadPtr(v, vi, nx, lane);
+            loadPtr(v, vi, nx, row);
             zero(w);
-            mvAcc(w, tab(P.lsQ, l), nx, nx, nx, v, lane);
+            mvAcc(w, tab(P.lsQ, l), nx, nx, nx, v);
 #pragma unroll
             for (int rc = 0; rc < R; rc++) o.x[rc] += w[rc];
             if (P.lcost == COST_QUADLIN_DEV) {
                 CP<T> lq = tab(P.lq, l);
-                eachRow<R>(nx, lane,
+                eachRow<R>(nx, row,
                            [&](int rc, unsigned r) { o.x[rc] = o.x[rc] - T(0.5) * lq[r] * a - T(0.5) * lq[r] * bb; });
             }
             o.s = (a + bb) * T(0.5);
@@ -412,18 +497,18 @@ __device__ __forceinline__ void adjNode(IP<T> P, GP<T> dual, int n, unsigned lan
 // src/constraints.cuh:158-169 (rectangle), :251-263 (polyhedron).
 // pv(base, k): element base + k of the primal vector, base wave-uniform.
 // The handler H receives each dual block of node n as register values:
-//   blockI(n, yk (lane < yD), IIval)
+//   blockI(n, yk (row < yD), IIval)
 //   blockElem(dualIndexBase, vals, rows, lb table entry, ub table entry)  [III and V]
 //   blockSoc(dualIndexBase, xs (rows nx), us (rows nu, may be 0 rows), h, transEntry)  [IV and VI]
 template <typename T, int R, int V, typename PV, typename H>
-__device__ __forceinline__ void opNode(IP<T> P, int n, unsigned lane, PV pv, H &h) {
+__device__ __forceinline__ void opNode(IP<T> P, int n, unsigned row, PV pv, H &h) {
     const int nx = P.nx, nu = P.nu, nxu = nx + nu;
     T v[V], v2[V], acc[R], acc2[R];
     if (n < P.nl) {
         const long xn = P.oX + (long) n * nx, un = P.oU + (long) n * nu;
         // I and II
-        const T yk = (lane < (unsigned) P.yD) ? pv(P.oY + (long) n * P.yD, lane) : T(0);
-        const T bk = (lane < (unsigned) P.yD) ? tab(P.b, n)[lane] : T(0);
+        const T yk = (row < (unsigned) P.yD) ? pv(P.oY + (long) n * P.yD, row) : T(0);
+        const T bk = (row < (unsigned) P.yD) ? tab(P.b, n)[row] : T(0);
         const T by = waveSum(bk * yk);
         const T IIval = pv(P.oS + n, 0) - by;
         h.blockI(n, yk, IIval);
@@ -431,18 +516,18 @@ __device__ __forceinline__ void opNode(IP<T> P, int n, unsigned lane, PV pv, H &
         if (P.ncon == CON_RECT_DEV) {
             zero(acc);
             zero(acc2);
-            eachRow<R>(nx, lane, [&](int rc, unsigned r) { acc[rc] = pv(xn, r); });
-            eachRow<R>(nu, lane, [&](int rc, unsigned r) { acc2[rc] = pv(un, r); });
+            eachRow<R>(nx, row, [&](int rc, unsigned r) { acc[rc] = pv(xn, r); });
+            eachRow<R>(nu, row, [&](int rc, unsigned r) { acc2[rc] = pv(un, r); });
             const long base = P.oIII + (long) n * P.con3;
             h.blockElem(base, acc, nx, tab(P.nLB, n), tab(P.nUB, n));
             h.blockElem(base + nx, acc2, nu, tab(P.nLB, n) + nx, tab(P.nUB, n) + nx);
         } else if (P.ncon == CON_POLY_DEV) {
-            loadV(v, nx, lane, [&](unsigned k) { return pv(xn, k); });
-            loadV(v2, nu, lane, [&](unsigned k) { return pv(un, k); });
+            loadV(v, nx, row, [&](unsigned k) { return pv(xn, k); });
+            loadV(v2, nu, row, [&](unsigned k) { return pv(un, k); });
             zero(acc);
             CP<T> G = tab(P.nG, n);
-            mvAcc(acc, G, P.con3, P.con3, nx, v, lane);
-            mvAcc(acc, G + (size_t) P.con3 * nx, P.con3, P.con3, nu, v2, lane);
+            mvAcc(acc, G, P.con3, P.con3, nx, v);
+            mvAcc(acc, G + (size_t) P.con3 * nx, P.con3, P.con3, nu, v2);
             h.blockElem(P.oIII + (long) n * P.con3, acc, P.con3, tab(P.nLB, n), tab(P.nUB, n));
         }
     }
@@ -453,8 +538,8 @@ __device__ __forceinline__ void opNode(IP<T> P, int n, unsigned lane, PV pv, H &
             const int a = cst(P.anc)[n];
             CP<T> qn = tab(P.q, n), rn = tab(P.r, n);
             T pq = T(0), pr = T(0);
-            eachRow<V>(nx, lane, [&](int, unsigned k) { pq += qn[k] * pv(P.oX + (long) a * nx, k); });
-            eachRow<V>(nu, lane, [&](int, unsigned k) { pr += rn[k] * pv(P.oU + (long) a * nu, k); });
+            eachRow<V>(nx, row, [&](int, unsigned k) { pq += qn[k] * pv(P.oX + (long) a * nx, k); });
+            eachRow<V>(nu, row, [&](int, unsigned k) { pr += rn[k] * pv(P.oU + (long) a * nu, k); });
             sum = waveSum(pq) + waveSum(pr);
         }
         h.blockLin(P.oIV + n, P.oIV + P.N + n, sum, pv(P.oT + n, 0));
@@ -464,16 +549,16 @@ __device__ __forceinline__ void opNode(IP<T> P, int n, unsigned lane, PV pv, H &
         T hv = T(0);
         if (n >= 1) {
             const int a = cst(P.anc)[n];
-            loadV(v, nx, lane, [&](unsigned k) { return pv(P.oX + (long) a * nx, k); });
-            loadV(v2, nu, lane, [&](unsigned k) { return pv(P.oU + (long) a * nu, k); });
-            mvAcc(acc, tab(P.sQ, n), nx, nx, nx, v, lane);
-            mvAcc(acc2, tab(P.sR, n), nu, nu, nu, v2, lane);
+            loadV(v, nx, row, [&](unsigned k) { return pv(P.oX + (long) a * nx, k); });
+            loadV(v2, nu, row, [&](unsigned k) { return pv(P.oU + (long) a * nu, k); });
+            mvAcc(acc, tab(P.sQ, n), nx, nx, nx, v);
+            mvAcc(acc2, tab(P.sR, n), nu, nu, nu, v2);
             hv = pv(P.oT + n, 0) * T(0.5);
             if (P.ncost == COST_QUADLIN_DEV) {
                 CP<T> qn = tab(P.q, n), rn = tab(P.r, n);
                 T pq = T(0), pr = T(0);
-                eachRow<V>(nx, lane, [&](int c, unsigned k) { pq += qn[k] * v[c]; });
-                eachRow<V>(nu, lane, [&](int c, unsigned k) { pr += rn[k] * v2[c]; });
+                eachRow<V>(nx, row, [&](int c, unsigned k) { pq += qn[k] * v[c]; });
+                eachRow<V>(nu, row, [&](int c, unsigned k) { pr += rn[k] * v2[c]; });
                 hv = hv + T(-0.5) * waveSum(pq);
                 hv = hv + T(-0.5) * waveSum(pr);
             }
@@ -484,31 +569,31 @@ __device__ __forceinline__ void opNode(IP<T> P, int n, unsigned lane, PV pv, H &
     if (n >= P.nl) {
         const int l = n - P.nl;
         const long xn = P.oX + (long) n * nx;
-        loadV(v, nx, lane, [&](unsigned k) { return pv(xn, k); });
+        loadV(v, nx, row, [&](unsigned k) { return pv(xn, k); });
         if (P.lcon == CON_RECT_DEV) {
             zero(acc);
-            eachRow<R>(nx, lane, [&](int rc, unsigned) { acc[rc] = v[rc]; });
+            eachRow<R>(nx, row, [&](int rc, unsigned) { acc[rc] = v[rc]; });
             h.blockElem(P.oV + (long) l * P.con5, acc, nx, tab(P.lLB, l), tab(P.lUB, l));
         } else if (P.lcon == CON_POLY_DEV) {
             zero(acc);
-            mvAcc(acc, tab(P.lG, l), P.con5, P.con5, nx, v, lane);
+            mvAcc(acc, tab(P.lG, l), P.con5, P.con5, nx, v);
             h.blockElem(P.oV + (long) l * P.con5, acc, P.con5, tab(P.lLB, l), tab(P.lUB, l));
         }
         if (P.lcost == COST_LIN_DEV) {  // (q' x_l, s_l) (src/costs.cuh:269-272)
             CP<T> lq = tab(P.lq, l);
             T pq = T(0);
-            eachRow<V>(nx, lane, [&](int c, unsigned k) { pq += lq[k] * v[c]; });
+            eachRow<V>(nx, row, [&](int c, unsigned k) { pq += lq[k] * v[c]; });
             h.blockLin(P.oVI + l, P.oVI + P.nlf + l, waveSum(pq), pv(P.oS + n, 0));
             return;
         }
         zero(acc);
         zero(acc2);
-        mvAcc(acc, tab(P.lsQ, l), nx, nx, nx, v, lane);
+        mvAcc(acc, tab(P.lsQ, l), nx, nx, nx, v);
         T hs = pv(P.oS + n, 0) * T(0.5);
         if (P.lcost == COST_QUADLIN_DEV) {
             CP<T> lq = tab(P.lq, l);
             T pq = T(0);
-            eachRow<V>(nx, lane, [&](int c, unsigned k) { pq += lq[k] * v[c]; });
+            eachRow<V>(nx, row, [&](int c, unsigned k) { pq += lq[k] * v[c]; });
             hs = hs + T(-0.5) * waveSum(pq);
         }
         h.blockSoc(P.oVI + (long) l * (nx + 2), acc, nx, acc2, 0, hs, tab(P.ltrans, l));
@@ -521,26 +606,26 @@ template <typename T, int R>
 struct StoreL {
     IP<T> P;
     GP<T> out;
-    unsigned lane;
+    unsigned row;
     __device__ __forceinline__ void blockI(int n, T yk, T IIval) {
-        if (lane < (unsigned) P.yD) (out + (P.oI + (long) n * P.yD))[lane] = yk;
-        if (lane == 0) out[P.oII + n] = IIval;
+        if (row < (unsigned) P.yD) (out + (P.oI + (long) n * P.yD))[row] = yk;
+        if (row == 0) out[P.oII + n] = IIval;
     }
     __device__ __forceinline__ void blockElem(long base, const T (&a)[R], int rows, CP<T>, CP<T>) {
         GP<T> ob = out + base;
-        eachRow<R>(rows, lane, [&](int rc, unsigned r) { ob[r] = a[rc]; });
+        eachRow<R>(rows, row, [&](int rc, unsigned r) { ob[r] = a[rc]; });
     }
     __device__ __forceinline__ void blockSoc(long base, const T (&xs)[R], int nxr, const T (&us)[R], int nur, T hv, CP<T>) {
         GP<T> ob = out + base;
-        eachRow<R>(nxr, lane, [&](int rc, unsigned r) { ob[r] = xs[rc]; });
-        eachRow<R>(nur, lane, [&](int rc, unsigned r) { (ob + nxr)[r] = us[rc]; });
-        if (lane == 0) {
+        eachRow<R>(nxr, row, [&](int rc, unsigned r) { ob[r] = xs[rc]; });
+        eachRow<R>(nur, row, [&](int rc, unsigned r) { (ob + nxr)[r] = us[rc]; });
+        if (row == 0) {
             ob[nxr + nur] = hv;
             ob[nxr + nur + 1] = hv;
         }
     }
     __device__ __forceinline__ void blockLin(long eSum, long eSet, T sum, T set) {
-        if (lane == 0) {
+        if (row == 0) {
             out[eSum] = sum;
             out[eSet] = set;
         }
@@ -554,17 +639,17 @@ template <typename T, int R>
 struct ProxL {
     IP<T> P;
     GP<T> zd, cd;
-    unsigned lane;
+    unsigned row;
     __device__ __forceinline__ T wOf(T Lv, T z, T trans) const { return (Lv * P.gamma + z) * P.gammaRecip + trans; }
     __device__ __forceinline__ void blockI(int n, T yk, T IIval) {
-        if (lane < (unsigned) P.yD) {
+        if (row < (unsigned) P.yD) {
             const long base = P.oI + (long) n * P.yD;
-            const T w = wOf(yk, (zd + base)[lane], T(0));
-            const int idx = ((int) lane < 2 * cst(P.numCh)[n]) && (w < T(0));
+            const T w = wOf(yk, (zd + base)[row], T(0));
+            const int idx = ((int) row < 2 * cst(P.numCh)[n]) && (w < T(0));
             const T p = T(1 - idx) * w;
-            (cd + base)[lane] = (w - p) * P.gamma;
+            (cd + base)[row] = (w - p) * P.gamma;
         }
-        if (lane == 0) {
+        if (row == 0) {
             const long k = P.oII + n;
             const T w = wOf(IIval, zd[k], T(0));
             const T p = fmax(T(0), w);
@@ -573,7 +658,7 @@ struct ProxL {
     }
     __device__ __forceinline__ void blockElem(long base, const T (&a)[R], int rows, CP<T> lb, CP<T> ub) {
         GP<T> zb = zd + base, cb = cd + base;
-        eachRow<R>(rows, lane, [&](int rc, unsigned r) {
+        eachRow<R>(rows, row, [&](int rc, unsigned r) {
             const T w = wOf(a[rc], zb[r], T(0));
             const T p = projBox(w, lb[r], ub[r]);
             cb[r] = (w - p) * P.gamma;
@@ -587,7 +672,7 @@ struct ProxL {
         CP<T> tu = tr + nxr, th = tu + nur;
 #pragma unroll
         for (int rc = 0; rc < R; rc++) {
-            const unsigned r = lane + 64 * rc;
+            const unsigned r = row + 64 * rc;
             wx[rc] = T(0);
             wu[rc] = T(0);
             if (64 * rc < nxr && r < (unsigned) nxr) {
@@ -608,9 +693,9 @@ struct ProxL {
         const int i3 = !i1 && !i2;
         const T sc = (nrm + tl) / (T(2) * nrm + T(1 - i3));
         const T mult = T(1 - i2) * (T(i3) * sc + T(1 - i3));
-        eachRow<R>(nxr, lane, [&](int rc, unsigned r) { cx[r] = (wx[rc] - wx[rc] * mult) * P.gamma; });
-        eachRow<R>(nur, lane, [&](int rc, unsigned r) { cu[r] = (wu[rc] - wu[rc] * mult) * P.gamma; });
-        if (lane == 0) {
+        eachRow<R>(nxr, row, [&](int rc, unsigned r) { cx[r] = (wx[rc] - wx[rc] * mult) * P.gamma; });
+        eachRow<R>(nur, row, [&](int rc, unsigned r) { cu[r] = (wu[rc] - wu[rc] * mult) * P.gamma; });
+        if (row == 0) {
             const T p1 = w1 * mult;
             const int i1b = (1 - i2) * (1 - i3);
             const T p2 = T(i1b) * (w2 * T(1 - i2)) + T((1 - i1b) * (1 - i2)) * (T(i3) * (sc * nrm - T(1)) + T(1));
@@ -621,7 +706,7 @@ struct ProxL {
     // linear cost: the cost entry clamped to at most the epigraph entry, which is kept
     // (src/costs.cuh:296-301 with k_projectRectangle, lower bound -inf)
     __device__ __forceinline__ void blockLin(long eSum, long eSet, T sum, T set) {
-        if (lane == 0) {
+        if (row == 0) {
             const T ws = wOf(sum, zd[eSum], T(0)), wt = wOf(set, zd[eSet], T(0));
             cd[eSum] = (ws - projBelow(ws, wt)) * P.gamma;
             cd[eSet] = (wt - wt) * P.gamma;
@@ -635,7 +720,7 @@ template <typename T, int R>
 struct ReduceL {
     IP<T> P;
     GP<T> xd, yd;  // dual parts of the partner and input vectors
-    unsigned lane;
+    unsigned row;
     T dot, mx;
     __device__ __forceinline__ void acc(T x, T y, T ell) {
         dot += x * (ell * (-P.gamma) + y);
@@ -643,28 +728,28 @@ struct ReduceL {
     }
     __device__ __forceinline__ void blockI(int n, T yk, T IIval) {
         const long base = P.oI + (long) n * P.yD, k = P.oII + n;
-        if (lane < (unsigned) P.yD) acc((xd + base)[lane], (yd + base)[lane], yk);
-        if (lane == 0) acc(xd[k], yd[k], IIval);
+        if (row < (unsigned) P.yD) acc((xd + base)[row], (yd + base)[row], yk);
+        if (row == 0) acc(xd[k], yd[k], IIval);
     }
     __device__ __forceinline__ void blockElem(long base, const T (&a)[R], int rows, CP<T>, CP<T>) {
         GP<T> xb = xd + base, yb = yd + base;
-        eachRow<R>(rows, lane, [&](int rc, unsigned r) { acc(xb[r], yb[r], a[rc]); });
+        eachRow<R>(rows, row, [&](int rc, unsigned r) { acc(xb[r], yb[r], a[rc]); });
     }
     __device__ __forceinline__ void blockSoc(long base, const T (&xs)[R], int nxr, const T (&us)[R], int nur, T hv, CP<T>) {
         GP<T> xx = xd + base, yx = yd + base, xu = xx + nxr, yu = yx + nxr, xh = xu + nur, yh = yu + nur;
 #pragma unroll
         for (int rc = 0; rc < R; rc++) {
-            const unsigned r = lane + 64 * rc;
+            const unsigned r = row + 64 * rc;
             if (64 * rc < nxr && r < (unsigned) nxr) acc(xx[r], yx[r], xs[rc]);
             if (64 * rc < nur && r < (unsigned) nur) acc(xu[r], yu[r], us[rc]);
         }
-        if (lane == 0) {
+        if (row == 0) {
             acc(xh[0], yh[0], hv);
             acc(xh[1], yh[1], hv);
         }
     }
     __device__ __forceinline__ void blockLin(long eSum, long eSet, T sum, T set) {
-        if (lane == 0) {
+        if (row == 0) {
             acc(xd[eSum], yd[eSum], sum);
             acc(xd[eSet], yd[eSet], set);
         }
@@ -682,21 +767,21 @@ __device__ __noinline__ void phaseAdjAxpy(const Inst<T> *Pp, int grid, T *zIn, T
     GP<T> zd = z + P.sPrim;
     const T g = -P.gamma;
     const int nx = P.nx, nu = P.nu;
-    const unsigned lane = c.lane;
+    const unsigned row = c.row;
     for (int n = c.wave; n < P.N; n += c.nw) {
         AdjOut<T, R> o;
-        adjNode<T, R, V>(P, zd, n, lane, o);
+        adjNode<T, R, V>(P, zd, n, row, o);
         const long xn = P.oX + (long) n * nx, un = P.oU + (long) n * nu, yn = P.oY + (long) n * P.yD;
-        eachRow<R>(nx, lane, [&](int rc, unsigned r) {
+        eachRow<R>(nx, row, [&](int rc, unsigned r) {
             const T v = o.x[rc] * g + (z + xn)[r];
             (cand + xn)[r] = v;
             if (n >= P.nl) (qd + (long) n * nx)[r] = -v;
         });
         if (n < P.nl) {
-            eachRow<R>(nu, lane, [&](int rc, unsigned r) { (cand + un)[r] = o.u[rc] * g + (z + un)[r]; });
-            if (lane < (unsigned) P.yD) (cand + yn)[lane] = o.y * g + (z + yn)[lane];
+            eachRow<R>(nu, row, [&](int rc, unsigned r) { (cand + un)[r] = o.u[rc] * g + (z + un)[r]; });
+            if (row < (unsigned) P.yD) (cand + yn)[row] = o.y * g + (z + yn)[row];
         }
-        if (lane == 0) {
+        if (row == 0) {
             T sv = o.s * g + z[P.oS + n];
             if (n == 0) sv -= P.gamma;
             cand[P.oS + n] = sv;
@@ -708,7 +793,7 @@ __device__ __noinline__ void phaseAdjAxpy(const Inst<T> *Pp, int grid, T *zIn, T
 // Backward sweep step for node i (src/dynamics.cuh:85-139).  With affine dynamics the children's
 // q enter as q_j + P_j e_j (src/dynamics.cuh:93-97).
 template <typename T, int R, int V>
-__device__ __forceinline__ void dynBackwardNode(IP<T> P, GP<T> cand, int i, int stage, unsigned lane) {
+__device__ __forceinline__ void dynBackwardNode(IP<T> P, GP<T> cand, int i, int stage, unsigned row) {
     const int nx = P.nx, nu = P.nu;
     GP<T> ubar = cand + (P.oU + (long) i * nu);
     GP<T> xbar = cand + (P.oX + (long) i * nx);
@@ -716,23 +801,23 @@ __device__ __forceinline__ void dynBackwardNode(IP<T> P, GP<T> cand, int i, int 
     T v[V], w[R], acc[R];
     zero(acc);
     const int c0 = cst(P.chFrom)[i], nc = cst(P.numCh)[i];
-    const bool mine = lane < (unsigned) nu;
+    const bool mine = row < (unsigned) nu;
     auto loadQ = [&](int j) {
         GP<T> qj = qd + (long) j * nx;
         if (P.affine) {
             CP<T> pe = tab(P.Pe, j);
-            loadV(v, nx, lane, [&](unsigned k) -> T { return qj[k] + pe[k]; });
+            loadV(v, nx, row, [&](unsigned k) -> T { return qj[k] + pe[k]; });
         } else {
-            loadPtr(v, qj, nx, lane);
+            loadPtr(v, qj, nx, row);
         }
     };
-    const T ub = mine ? ubar[lane] : T(0);
+    const T ub = mine ? ubar[row] : T(0);
 #pragma unroll 1
     for (int ci = 0; ci < nc; ci++) {
         const int j = c0 + ci;
         loadQ(j);
         zero(w);
-        mvAcc(w, tab(P.BTr, j), nu, nu, nx, v, lane);
+        mvAcc(w, tab(P.BTr, j), nu, nu, nx, v);
 #pragma unroll
         for (int rc = 0; rc < R; rc++) acc[rc] = (ci == 0) ? w[rc] : acc[rc] + w[rc];
     }
@@ -744,23 +829,23 @@ __device__ __forceinline__ void dynBackwardNode(IP<T> P, GP<T> cand, int i, int 
         zero(dvin);
         dvin[0] = d;
         zero(dout);
-        mvAcc(dout, tab(P.RtInv, i), nu, nu, nu, dvin, lane);
+        mvAcc(dout, tab(P.RtInv, i), nu, nu, nu, dvin);
         d = mine ? dout[0] : T(0);
     } else {
         CP<T> L = tab(P.cholL, i);
         for (int k = 0; k < nu; k++) {
-            const T dk = bcastLane(d, k) / L[k + (size_t) k * nu];
-            if ((int) lane == k) d = dk;
-            else if ((int) lane > k && mine) d -= L[lane + (size_t) k * nu] * dk;
+            const T dk = bcastLane(d, laneOf(k)) / L[k + (size_t) k * nu];
+            if ((int) row == k) d = dk;
+            else if ((int) row > k && mine) d -= L[row + (size_t) k * nu] * dk;
         }
         CP<T> U = tab(P.cholU, i);
         for (int k = nu - 1; k >= 0; k--) {
-            const T dk = bcastLane(d, k) / U[k + (size_t) k * nu];
-            if ((int) lane == k) d = dk;
-            else if ((int) lane < k) d -= U[lane + (size_t) k * nu] * dk;
+            const T dk = bcastLane(d, laneOf(k)) / U[k + (size_t) k * nu];
+            if ((int) row == k) d = dk;
+            else if ((int) row < k) d -= U[row + (size_t) k * nu] * dk;
         }
     }
-    if (mine) ((GP<T>) P.dd + (long) i * nu)[lane] = d;
+    if (mine) ((GP<T>) P.dd + (long) i * nu)[row] = d;
     if (stage == 0) return;
     // q_i = sum_j (APB_j d_i + ABKTr_j q_j) + K_i'(d_i - u_i) - x_i
     T dv[V];
@@ -771,24 +856,24 @@ __device__ __forceinline__ void dynBackwardNode(IP<T> P, GP<T> cand, int i, int 
     for (int ci = 0; ci < nc; ci++) {
         const int j = c0 + ci;
         zero(w);
-        mvAcc(w, tab(P.APB, j), nx, nx, nu, dv, lane);
+        mvAcc(w, tab(P.APB, j), nx, nx, nu, dv);
         if (nc > 1) loadQ(j);  // a single child's q is still in v
-        mvAcc(w, tab(P.ABKTr, j), nx, nx, nx, v, lane);
+        mvAcc(w, tab(P.ABKTr, j), nx, nx, nx, v);
 #pragma unroll
         for (int rc = 0; rc < R; rc++) acc[rc] = (ci == 0) ? w[rc] : acc[rc] + w[rc];
     }
     dv[0] = mine ? d - ub : T(0);
     zero(w);
-    mvAcc(w, tab(P.KTr, i), nx, nx, nu, dv, lane);
-    eachRow<R>(nx, lane, [&](int rc, unsigned r) { (qd + (long) i * nx)[r] = (acc[rc] + w[rc]) - xbar[r]; });
+    mvAcc(w, tab(P.KTr, i), nx, nx, nu, dv);
+    eachRow<R>(nx, row, [&](int rc, unsigned r) { (qd + (long) i * nx)[r] = (acc[rc] + w[rc]) - xbar[r]; });
 }
 
 // Kernel projection for nonleaf node i (src/cache.cuh:650-676); padded child slots enter as 0.
 template <typename T, int R, int V>
-__device__ __forceinline__ void kernelNode(IP<T> P, GP<T> cand, int i, unsigned lane) {
+__device__ __forceinline__ void kernelNode(IP<T> P, GP<T> cand, int i, unsigned row) {
     const int yD = P.yD, E = P.E, nc = cst(P.numCh)[i], c0 = cst(P.chFrom)[i];
-    // this lane's entry of [y; t of the children; s of the children], or none
-    const int k = (int) lane;
+    // this row's entry of [y; t of the children; s of the children], or none
+    const int k = (int) row;
     const bool isY = k < yD, isT = !isY && k < yD + E && k - yD < nc;
     const bool isS = k >= yD + E && k < yD + 2 * E && k - yD - E < nc;
     const bool any = isY || isT || isS;
@@ -797,28 +882,28 @@ __device__ __forceinline__ void kernelNode(IP<T> P, GP<T> cand, int i, unsigned 
     zero(vin);
     if (any) vin[0] = cand[at];
     zero(w);
-    mvAcc(w, tab(P.NN, i), P.nD, P.nD, P.nD, vin, lane);
+    mvAcc(w, tab(P.NN, i), P.nD, P.nD, P.nD, vin);
     if (any) cand[at] = w[0];
 }
 
 // Forward rollout for node i (src/dynamics.cuh:144-173); affine dynamics add e_j to each child.
 template <typename T, int R, int V>
-__device__ __forceinline__ void dynForwardNode(IP<T> P, GP<T> cand, int i, unsigned lane) {
+__device__ __forceinline__ void dynForwardNode(IP<T> P, GP<T> cand, int i, unsigned row) {
     const int nx = P.nx, nu = P.nu;
     T xv[V], uv[V], w[R];
     GP<T> xi = cand + (P.oX + (long) i * nx);
     if (i == 0) {
-        loadPtr(xv, cst(P.x0s), nx, lane);
-        eachRow<V>(nx, lane, [&](int c, unsigned k) { xi[k] = xv[c]; });
+        loadPtr(xv, cst(P.x0s), nx, row);
+        eachRow<V>(nx, row, [&](int c, unsigned k) { xi[k] = xv[c]; });
     } else {
-        loadPtr(xv, xi, nx, lane);
+        loadPtr(xv, xi, nx, row);
     }
-    const bool mine = lane < (unsigned) nu;
-    const T di = mine ? ((GP<T>) P.dd + (long) i * nu)[lane] : T(0);
+    const bool mine = row < (unsigned) nu;
+    const T di = mine ? ((GP<T>) P.dd + (long) i * nu)[row] : T(0);
     zero(w);
-    mvAcc(w, tab(P.K, i), nu, nu, nx, xv, lane);
+    mvAcc(w, tab(P.K, i), nu, nu, nx, xv);
     const T u = mine ? w[0] + di : T(0);
-    if (mine) (cand + (P.oU + (long) i * nu))[lane] = u;
+    if (mine) (cand + (P.oU + (long) i * nu))[row] = u;
     zero(uv);
     uv[0] = u;
     const int c0 = cst(P.chFrom)[i], nc = cst(P.numCh)[i];
@@ -827,11 +912,11 @@ __device__ __forceinline__ void dynForwardNode(IP<T> P, GP<T> cand, int i, unsig
         const int j = c0 + ci;
         CP<T> AB = tab(P.AB, j);
         zero(w);
-        mvAcc(w, AB, nx, nx, nx, xv, lane);
-        mvAcc(w, AB + (size_t) nx * nx, nx, nx, nu, uv, lane);
+        mvAcc(w, AB, nx, nx, nx, xv);
+        mvAcc(w, AB + (size_t) nx * nx, nx, nx, nu, uv);
         CP<T> ej = tab(P.e, j);
         GP<T> xj = cand + (P.oX + (long) j * nx);
-        eachRow<R>(nx, lane, [&](int rc, unsigned r) { xj[r] = P.affine ? w[rc] + ej[r] : w[rc]; });
+        eachRow<R>(nx, row, [&](int rc, unsigned r) { xj[r] = P.affine ? w[rc] + ej[r] : w[rc]; });
     }
 }
 
@@ -847,18 +932,18 @@ __device__ __noinline__ void phaseProjections(const Inst<T> *Pp, int grid, T *ca
             const int f = cst(P.stageFrom)[stage], nStage = cst(P.stageTo)[stage] - f + 1;
             const int extra = (doKernel && stage == P.S - 2) ? P.nl : 0;
             for (int task = c.wave; task < nStage + extra; task += c.nw) {
-                if (task < nStage) dynBackwardNode<T, R, V>(P, cand, f + task, stage, c.lane);
-                else kernelNode<T, R, V>(P, cand, task - nStage, c.lane);
+                if (task < nStage) dynBackwardNode<T, R, V>(P, cand, f + task, stage, c.row);
+                else kernelNode<T, R, V>(P, cand, task - nStage, c.row);
             }
             sync(c);
         }
         for (int stage = 0; stage <= P.S - 2; stage++) {
             const int f = cst(P.stageFrom)[stage], nStage = cst(P.stageTo)[stage] - f + 1;
-            for (int task = c.wave; task < nStage; task += c.nw) dynForwardNode<T, R, V>(P, cand, f + task, c.lane);
+            for (int task = c.wave; task < nStage; task += c.nw) dynForwardNode<T, R, V>(P, cand, f + task, c.row);
             sync(c);
         }
     } else if (doKernel) {
-        for (int task = c.wave; task < P.nl; task += c.nw) kernelNode<T, R, V>(P, cand, task, c.lane);
+        for (int task = c.wave; task < P.nl; task += c.nw) kernelNode<T, R, V>(P, cand, task, c.row);
         sync(c);
     }
 }
@@ -869,9 +954,9 @@ __device__ __noinline__ void phaseDualProx(const Inst<T> *Pp, int grid, T *zIn, 
     IP<T> P = *cst(uniformPtr(Pp));
     const Tc c = threadCtx(grid);
     GP<T> z = glb(zIn), cand = glb(candIn);
-    ProxL<T, R> h{P, z + P.sPrim, cand + P.sPrim, c.lane};
+    ProxL<T, R> h{P, z + P.sPrim, cand + P.sPrim, c.row};
     auto pv = [&](long base, unsigned k) -> T { return (cand + base)[k] * T(2) - (z + base)[k]; };
-    for (int n = c.wave; n < P.N; n += c.nw) opNode<T, R, V>(P, n, c.lane, pv, h);
+    for (int n = c.wave; n < P.N; n += c.nw) opNode<T, R, V>(P, n, c.row, pv, h);
     sync(c);
 }
 
@@ -900,31 +985,31 @@ __device__ __noinline__ EllSums<T> reduceEllNodes(const Inst<T> *Pp, int grid, T
     const Tc c = threadCtx(grid);
     GP<T> x = glb(xIn), y = glb(yIn);
     const int nx = P.nx, nu = P.nu;
-    const unsigned lane = c.lane;
+    const unsigned row = c.row;
     T dot = T(0), mx = T(0);
     auto acc = [&](T xk, T yk, T ell) {
         dot += xk * (ell * (-P.gamma) + yk);
         mx = fmax(mx, fabs(yk * P.gammaRecip - ell));
     };
     GP<T> yd = y + P.sPrim;
-    ReduceL<T, R> h{P, x + P.sPrim, yd, lane, T(0), T(0)};
+    ReduceL<T, R> h{P, x + P.sPrim, yd, row, T(0), T(0)};
     auto pv = [&](long base, unsigned k) -> T { return (y + base)[k]; };
     for (int n = c.wave; n < P.N; n += c.nw) {
         AdjOut<T, R> o;
-        adjNode<T, R, V>(P, yd, n, lane, o);
+        adjNode<T, R, V>(P, yd, n, row, o);
         const long xn = P.oX + (long) n * nx, un = P.oU + (long) n * nu, yn = P.oY + (long) n * P.yD;
 #pragma unroll
         for (int rc = 0; rc < R; rc++) {
-            const unsigned r = lane + 64 * rc;
+            const unsigned r = row + 64 * rc;
             if (64 * rc < nx && r < (unsigned) nx) acc((x + xn)[r], (y + xn)[r], o.x[rc]);
             if (n < P.nl && 64 * rc < nu && r < (unsigned) nu) acc((x + un)[r], (y + un)[r], o.u[rc]);
         }
-        if (n < P.nl && lane < (unsigned) P.yD) acc((x + yn)[lane], (y + yn)[lane], o.y);
-        if (lane == 0) {
+        if (n < P.nl && row < (unsigned) P.yD) acc((x + yn)[row], (y + yn)[row], o.y);
+        if (row == 0) {
             acc(x[P.oS + n], y[P.oS + n], o.s);
             acc(x[P.oT + n], y[P.oT + n], o.t);
         }
-        opNode<T, R, V>(P, n, lane, pv, h);
+        opNode<T, R, V>(P, n, row, pv, h);
     }
     return EllSums<T>{dot + h.dot, mx, h.mx};
 }
@@ -1574,19 +1659,19 @@ __global__ void __launch_bounds__(SPK_MAX_THREADS) k_debug(const Inst<T> *__rest
     __syncthreads();
     GP<T> z = (GP<T>) P.z, cand = (GP<T>) P.cand;
     if (op == OP_L) {
-        StoreL<T, R> h{P, cand + P.sPrim, c.lane};
+        StoreL<T, R> h{P, cand + P.sPrim, c.row};
         auto pv = [&](long base, unsigned k) -> T { return (z + base)[k]; };
-        for (int n = c.wave; n < P.N; n += c.nw) opNode<T, R, V>(P, n, c.lane, pv, h);
+        for (int n = c.wave; n < P.N; n += c.nw) opNode<T, R, V>(P, n, c.row, pv, h);
     } else if (op == OP_LADJ) {
         for (int n = c.wave; n < P.N; n += c.nw) {
             AdjOut<T, R> o;
-            adjNode<T, R, V>(P, z + P.sPrim, n, c.lane, o);
-            eachRow<R>(P.nx, c.lane, [&](int rc, unsigned r) { cand[P.oX + (long) n * P.nx + r] = o.x[rc]; });
+            adjNode<T, R, V>(P, z + P.sPrim, n, c.row, o);
+            eachRow<R>(P.nx, c.row, [&](int rc, unsigned r) { cand[P.oX + (long) n * P.nx + r] = o.x[rc]; });
             if (n < P.nl) {
-                eachRow<R>(P.nu, c.lane, [&](int rc, unsigned r) { cand[P.oU + (long) n * P.nu + r] = o.u[rc]; });
-                if (c.lane < (unsigned) P.yD) cand[P.oY + (long) n * P.yD + c.lane] = o.y;
+                eachRow<R>(P.nu, c.row, [&](int rc, unsigned r) { cand[P.oU + (long) n * P.nu + r] = o.u[rc]; });
+                if (c.row < (unsigned) P.yD) cand[P.oY + (long) n * P.yD + c.row] = o.y;
             }
-            if (c.lane == 0) {
+            if (c.row == 0) {
                 cand[P.oS + n] = o.s;
                 cand[P.oT + n] = o.t;
             }
