@@ -243,7 +243,9 @@ size_t alignUp(size_t v, size_t a) { return (v + a - 1) / a * a; }
 size_t coreCount(const HostProblem &h) {
     return alignUp(8 * (size_t) h.sIter + (size_t) h.nx * h.N + (size_t) h.nu * h.nl, 64);
 }
-size_t andCount(const HostProblem &h, int m) { return alignUp((size_t) (3 * m + 1) * h.sIter, 64); }
+size_t andCount(const HostProblem &h, int m) { return alignUp((size_t) 2 * m * h.sIter, 64); }
+// the same in the fixed scratch of allocation-free solves, whose documented size per instance it is
+size_t scratchAndCount(const HostProblem &h, int m) { return alignUp((size_t) (3 * m + 1) * h.sIter, 64); }
 
 // Problem sizes, offsets, tree arrays and device tables shared by both instance descriptors.
 template <typename T, typename I>
@@ -311,7 +313,7 @@ void fillInsts(spk_batch *b, const spk_options &o, int warm, T *anders, const st
         I.x0s = static_cast<const T *>(b->x0buf.p) + b->x0Off[k];
         T *a = and_ + andOff[k];
         const int m = o.anderson_buffer;
-        I.hS = a; I.hY = a + (size_t) m * n; I.W = a + (size_t) 2 * m * n;
+        I.hS = a; I.hY = a + (size_t) m * n;
         double tolScale = 1.;
         if (h.precond) tolScale = *std::min_element(h.scaling.begin(), h.scaling.end());
         I.tolAbs = (T) (o.tol_abs * tolScale);
@@ -572,7 +574,7 @@ size_t scratchLayout(const spk_batch *b, int m, std::vector<size_t> &andOff, siz
     size_t el = 0;
     for (int k = 0; k < b->count; k++) {
         andOff[k] = el;
-        el += andCount(b->probs[k]->hp, m);
+        el += scratchAndCount(b->probs[k]->hp, m);
     }
     andAt = alignUp(sizeof(spk::Inst<T>) * b->count, 256);
     gpartAt = alignUp(andAt + el * sizeof(T), 256);

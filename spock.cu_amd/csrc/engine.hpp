@@ -57,7 +57,6 @@ struct Inst {
     // state (iterate-sized unless noted)
     T *z, *zPrev, *cand, *backup, *res, *resPrev, *dir, *dirS;
     T *hS, *hY;    // Anderson histories (iterate and residual differences), andBuff columns each
-    T *W;          // Householder scratch, andBuff + 1 columns
     T *qd, *dd;    // dynamics sweep intermediates: nx*N and nu*nl
     const T *x0s;  // scaled initial state (nx)
     // options
