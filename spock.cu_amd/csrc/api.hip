@@ -100,7 +100,7 @@ using spk::fail;
 template <typename T>
 struct DevTableSet {  // device copies of one table: data as T, index as int
     std::unique_ptr<DevBuf> data, idx;
-    int rows = 0, cols = 0;
+    int rows = 0, cols = 0, stride = 0;
 };
 
 }  // namespace
@@ -115,7 +115,7 @@ struct spk_problem : spk::Counted {
     DevBuf anc, chFrom, numCh, stageFrom, stageTo;
     std::map<std::string, DevTableSet<double>> t64;
     std::map<std::string, DevTableSet<float>> t32;
-    bool up64 = false, up32 = false;
+    bool up64 = false, up32 = false, packed64 = false, packed32 = false;
 };
 
 struct spk_batch {
@@ -222,6 +222,68 @@ void ensureUploaded(spk_problem *p) {
     SPK_TABLES(UP)
 #undef UP
     done = true;
+}
+
+// The factors of the tile engine's products in its operand order (spk::PTab), made once per problem
+// and type, by the first shared batch.
+#define SPK_PACKED(X) \
+    X(BTr, BTr, 0, h.nu) X(AB, AB, 0, h.nx) X(K, K, 0, h.nu) X(KTr, KTr, 0, h.nx) X(ABKTr, ABKTr, 0, h.nx) \
+    X(APB, APB, 0, h.nx) X(RtInv, RtInv, 0, h.nu) X(NN, NN, 0, h.nD) X(sQ, sQ, 0, h.nx) X(sR, sR, 0, h.nu) \
+    X(lsQ, lsQ, 0, h.nx) X(G, nG, 0, h.con3) X(GTx, nGT, 0, h.nx) X(GTu, nGT, h.nx, h.nu) X(lG, lG, 0, h.con5) \
+    X(lGT, lGT, 0, h.nx)
+
+template <typename T>
+void uploadPacked(spk_problem *p, const std::string &name, const Table &t, int row0, int rows) {
+    DevTableSet<T> s;
+    s.rows = rows;
+    s.cols = t.cols;
+    const int kg = (t.cols + 15) / 16;
+    const size_t sz = (size_t) t.rows * t.cols, count = sz && rows ? t.data.size() / sz : 0;
+    size_t stride = 0;
+    for (int r0 = 0; r0 < rows; r0 += 64) stride += (size_t) kg * (rows - r0 > 32 ? 4 : 2) * 256;
+    std::vector<T> d(std::max<size_t>(1, count * stride), T(0));
+    for (size_t m = 0; m < count; m++) {
+        T *out = d.data() + m * stride;
+        const double *M = t.data.data() + m * sz + row0;
+        for (int r0 = 0; r0 < rows; r0 += 64) {
+            const int tiles = rows - r0 > 32 ? 4 : 2;
+            for (int c = 0; c < t.cols; c++)
+                for (int r = r0; r < std::min(rows, r0 + 64); r++) {
+                    const int tile = (r - r0) / 16, lane = (r & 15) + 16 * (c & 3);
+                    out[(((size_t) (c / 16) * tiles + tile) * 64 + lane) * 4 + (c & 15) / 4] = (T) M[(size_t) c * t.rows + r];
+                }
+            out += (size_t) kg * tiles * 256;
+        }
+    }
+    s.stride = (int) stride;
+    s.data = std::make_unique<DevBuf>();
+    s.data->alloc(d.size() * sizeof(T));
+    check(hipMemcpy(s.data->p, d.data(), d.size() * sizeof(T), hipMemcpyHostToDevice), "upload packed table");
+    tablesOf<T>(p)["packed " + name] = std::move(s);
+}
+
+template <typename T>
+void ensurePacked(spk_problem *p) {
+    bool &done = std::is_same<T, double>::value ? p->packed64 : p->packed32;
+    if (done) return;
+    const HostProblem &h = p->hp;
+#define PK(name, src, row0, rows) uploadPacked<T>(p, #name, h.src, row0, rows);
+    SPK_PACKED(PK)
+#undef PK
+    done = true;
+}
+
+template <typename T>
+spk::PTab<T> ptab(spk_problem *p, const std::string &name, const std::string &src) {
+    auto &m = tablesOf<T>(p);
+    auto &e = m.at("packed " + name);
+    spk::PTab<T> t;
+    t.data = static_cast<const T *>(e.data->p);
+    t.idx = static_cast<const int *>(m.at(src).idx->p);
+    t.rows = e.rows;
+    t.cols = e.cols;
+    t.stride = e.stride;
+    return t;
 }
 
 template <typename T>
@@ -648,6 +710,9 @@ void buildLaneInst(spk_batch *b, const spk_options &o, int warm, int resume = 0)
     spk_problem *p = b->probs[0];
     const HostProblem &h = p->hp;
     fillProblem<T>(L, p);
+#define PK(name, src, row0, rows) L.p##name = ptab<T>(p, #name, #src);
+    SPK_PACKED(PK)
+#undef PK
     L.B = b->Bpad;
     L.count = b->count;
     for (int r = 0; r < 9; r++) L.work[r] = lanePtr<T>(b, r);
@@ -1095,8 +1160,13 @@ int spk_batch_create_shared(spk_ctx *ctx, spk_problem *problem, int count, int d
         b->probs.assign(count, problem);
         b->holdProblems();
         check(hipSetDevice(ctx->device), "hipSetDevice");
-        if (dtype == SPK_F64) ensureUploaded<double>(problem);
-        else ensureUploaded<float>(problem);
+        if (dtype == SPK_F64) {
+            ensureUploaded<double>(problem);
+            ensurePacked<double>(problem);
+        } else {
+            ensureUploaded<float>(problem);
+            ensurePacked<float>(problem);
+        }
         const size_t total = laneLayout(b.get());
         // cleared on the batch's own stream, here and in resets: that stream does not wait for the null
         // stream, so a relayout or a solve could otherwise read a region before it was cleared

@@ -43,6 +43,17 @@ __device__ __forceinline__ CP<T> tab(const SPK_CONST DTab<T> &t, int n) {
     return cst(t.data) + (size_t) cst(t.idx)[n] * t.rows * t.cols;
 }
 
+// The same table packed for the tile engine's products: per distinct matrix and block of 64 rows,
+// [16-column group][16-row tile][lane][4], lane l holding M[16 t + l % 16][16 k + 4 s + l / 16] at
+// position s, zero past the matrix, with 2 row tiles in a block of up to 32 rows and 4 in a larger one.
+// `stride` entries per matrix.
+template <typename T>
+struct PTab {
+    const T *data = nullptr;
+    const int *idx = nullptr;
+    int rows = 0, cols = 0, stride = 0;
+};
+
 // One solve instance: problem sizes, device tables, state buffers and options.
 template <typename T>
 struct Inst {
@@ -121,6 +132,8 @@ struct LaneInst {
     DTab<T> nG, nLB, nUB, lG, lLB, lUB, nGT, lGT;
     DTab<T> e, Pe;  // affine dynamics (zero tables when linear)
     int affine;
+    // tile engine: packed factors (GTx, GTu: the state and the input rows of nGT)
+    PTab<T> pBTr, pAB, pK, pKTr, pABKTr, pAPB, pRtInv, pNN, psQ, psR, plsQ, pG, pGTx, pGTu, plG, plGT;
     long B;     // padded instance count (multiple of 64); a region of r rows holds r * B words
     int count;  // instances in use
     T *work[9];   // rotating roles z, cand, zPrev, res, resPrev, backup + cand2, dir, dirS

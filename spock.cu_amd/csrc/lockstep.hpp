@@ -18,6 +18,8 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include <type_traits>
+
 namespace spk {
 
 template <typename T>
@@ -126,6 +128,182 @@ __device__ __forceinline__ bool gramSolve(const double (&G)[MAXM][MAXM], const d
     return true;
 }
 
+// ---------------------------------------------------------------- iterate-wide passes
+// Never inlined: inside the solve its own state (Gram matrix, counters, tolerances: over 100 registers)
+// left the passes' loads in flight to be spilled to memory (1,000 FP64 instances of the 229-node problem, 63
+// of 256 CUs: residual and direction passes 2.5 + 2.0 ms an iteration, now 1.4 + 0.9; the 4,096 FP32
+// instances, bound by HBM, 1.36 + 1.16 ms, now 1.35 + 0.82).
+template <typename T>
+struct ColumnSums {
+    T rr;                  // |r|^2
+    double yy[MAXM], yr[MAXM];  // <Y_head, Y_s> and <Y_s, r>
+};
+
+// r = z - T(z), ||r||^2 and, in the same pass, the new Anderson column (src/cache.cuh:861-896) with its
+// Gram entries: Y_head = r - r_prev, S_head = (z - z_prev) - Y_head, of M columns.  Sums per lane.
+template <typename T, typename E, int M>
+__device__ __noinline__ ColumnSums<T> columnPass(const LaneInst<T> *Pp, T *zIn, T *cIn, T *rpIn, T *zpIn, T *rIn, int headIn) {
+    LP<T> P = *cst(uniformPtr(Pp));
+    const auto c = E::ctx();
+    const long n = P.sIter, B = P.B;
+    const int head = __builtin_amdgcn_readfirstlane(headIn);
+    auto V = [&](T *p) { return E::template view<T>(uniformPtr(p), n, c); };
+    const auto Yh = V(P.hY + (long) head * n * B), Sh = V(P.hS + (long) head * n * B);
+    const auto rr = V(rIn), cc = V(cIn), rp = V(rpIn), z = V(zIn), zp = V(zpIn);
+    constexpr int O = M > 1 ? M - 1 : 1;  // the other columns: slots head + 1 .. head + M - 1
+    typename E::template View<T> Yo[O];
+#pragma unroll
+    for (int i = 0; i < O; i++) Yo[i] = V(P.hY + (long) ((head + 1 + i) % M) * n * B);
+    T sr = T(0);
+    double hh = 0., hr = 0., oh[O], orr[O];
+#pragma unroll
+    for (int i = 0; i < O; i++) oh[i] = orr[i] = 0.;
+    E::template pass<4>(
+        n, c,
+        [&](long e) {
+            V4H<T, O> v;
+            v.a = z[e];
+            v.b = cc[e];
+            v.c = rp[e];
+            v.d = zp[e];
+#pragma unroll
+            for (int i = 0; i < M - 1; i++) v.h[i] = Yo[i][e];
+            return v;
+        },
+        [&](long e, const V4H<T, O> &v) {
+            const T r = v.a - v.b;
+            rr[e] = r;
+            sr += r * r;
+            const T dr = r - v.c;
+            Yh[e] = dr;
+            Sh[e] = (v.a - v.d) - dr;
+            const double drd = (double) dr, rd = (double) r;
+            hh += drd * drd;
+            hr += drd * rd;
+#pragma unroll
+            for (int i = 0; i < M - 1; i++) {
+                oh[i] += drd * (double) v.h[i];
+                orr[i] += (double) v.h[i] * rd;
+            }
+        });
+    ColumnSums<T> a;
+    a.rr = sr;
+#pragma unroll
+    for (int q = 0; q < MAXM; q++) {
+        a.yy[q] = q == head ? hh : 0.;
+        a.yr[q] = q == head ? hr : 0.;
+#pragma unroll
+        for (int i = 0; i < M - 1; i++) {
+            a.yy[q] = q == (head + 1 + i) % M ? oh[i] : a.yy[q];
+            a.yr[q] = q == (head + 1 + i) % M ? orr[i] : a.yr[q];
+        }
+    }
+    return a;
+}
+
+// d = -S g - r; K0 lanes write cand = z_prev + d (src/cache.cuh:897-898, 1055-1057).
+template <typename T>
+struct Coeffs {
+    T g[MAXM];
+};
+
+template <typename T, typename E, int M>
+__device__ __noinline__ void directionPass(const LaneInst<T> *Pp, T *rpIn, T *zpIn, T *dIn, T *cIn, Coeffs<T> k, bool blind) {
+    LP<T> P = *cst(uniformPtr(Pp));
+    const auto c = E::ctx();
+    const long n = P.sIter, B = P.B;
+    auto V = [&](T *p) { return E::template view<T>(uniformPtr(p), n, c); };
+    typename E::template View<T> Ss[M];
+#pragma unroll
+    for (int i = 0; i < M; i++) Ss[i] = V(P.hS + (long) i * n * B);
+    const auto rp = V(rpIn), zp = V(zpIn), dd = V(dIn), cc = V(cIn);
+    E::template pass<4>(
+        n, c,
+        [&](long e) {
+            VH<T, M> v;
+            v.a = rp[e];
+            v.b = zp[e];
+#pragma unroll
+            for (int i = 0; i < M; i++) v.h[i] = Ss[i][e];
+            return v;
+        },
+        [&](long e, const VH<T, M> &v) {
+            T sg = T(0);
+#pragma unroll
+            for (int i = 0; i < M; i++) sg += v.h[i] * k.g[i];
+            const T d = -sg - v.a;
+            if (blind) cc[e] = v.b + d;
+            else dd[e] = d;
+        });
+}
+
+// f<M>() for the Anderson memory m (1 .. MAXM).
+template <typename F>
+__device__ __forceinline__ void withMemory(int m, F f) {
+    if (m == 3) f(std::integral_constant<int, 3>{});
+    else if (m == 1) f(std::integral_constant<int, 1>{});
+    else if (m == 2) f(std::integral_constant<int, 2>{});
+    else f(std::integral_constant<int, 4>{});
+}
+
+// out = a - f b for the lanes with `take` (f = 0: a copy).
+template <typename T, typename E>
+__device__ __noinline__ void takePass(long n, T *outIn, T *aIn, T *bIn, T f, bool take) {
+    const auto c = E::ctx();
+    n = __builtin_amdgcn_readfirstlane((int) n);  // an iterate's size is an int (spk_problem_sizes)
+    auto V = [&](T *p) { return E::template view<T>(uniformPtr(p), n, c); };
+    const auto out = V(outIn), a = V(aIn);
+    if (bIn == nullptr) {
+        E::template pass<8>(n, c, [&](long e) -> T { return a[e]; }, [&](long e, T v) {
+            if (take) out[e] = v;
+        });
+        return;
+    }
+    const auto b = V(bIn);
+    E::template pass<8>(n, c, [&](long e) { return V2<T>{a[e], b[e]}; }, [&](long e, const V2<T> &v) {
+        if (take) out[e] = v.a - v.b * f;
+    });
+}
+
+// The line search's trial point: ds = tau d, z = z_prev + ds (src/cache.cuh:1063-1065).
+template <typename T, typename E>
+__device__ __noinline__ void trialPass(long n, T *dIn, T *zpIn, T *dsIn, T *zIn, T tau, bool ls) {
+    const auto c = E::ctx();
+    n = __builtin_amdgcn_readfirstlane((int) n);
+    auto V = [&](T *p) { return E::template view<T>(uniformPtr(p), n, c); };
+    const auto d = V(dIn), zp = V(zpIn), ds = V(dsIn), z = V(zIn);
+    E::template pass<8>(n, c, [&](long e) { return V2<T>{d[e], zp[e]}; }, [&](long e, const V2<T> &v) {
+        if (ls) {
+            const T s = v.a * tau;
+            ds[e] = s;
+            z[e] = v.b + s;
+        }
+    });
+}
+
+// r = z - T(z), |r|^2 and <r, ds> (ds == nullptr: r only).  Sums per lane.
+template <typename T, typename E>
+__device__ __noinline__ V2<T> residualPass(long n, T *zIn, T *cIn, T *dsIn, T *rIn) {
+    const auto c = E::ctx();
+    n = __builtin_amdgcn_readfirstlane((int) n);
+    auto V = [&](T *p) { return E::template view<T>(uniformPtr(p), n, c); };
+    const auto rr = V(rIn), z = V(zIn), cc = V(cIn);
+    V2<T> a{T(0), T(0)};
+    if (dsIn == nullptr) {
+        E::template pass<8>(n, c, [&](long e) { return V2<T>{z[e], cc[e]}; },
+                            [&](long e, const V2<T> &v) { rr[e] = v.a - v.b; });
+        return a;
+    }
+    const auto ds = V(dsIn);
+    E::template pass<8>(n, c, [&](long e) { return V4<T>{z[e], cc[e], ds[e], T(0)}; }, [&](long e, const V4<T> &v) {
+        const T d = v.a - v.b;
+        rr[e] = d;
+        a.a += d * d;
+        a.b += d * v.c;
+    });
+    return a;
+}
+
 }  // namespace ls
 
 // ---------------------------------------------------------------- the lockstep solve
@@ -227,15 +405,8 @@ __device__ void lockstepSolve(const LaneInst<T> *Pp, Out *outs, double *lds, lon
     for (it = itStart;; it++) {
         const bool capNow = active && it - it0 >= hardCap;
         if (anyLane(capNow)) {  // the current iterate is the output
-            const VW zio = V(P.zio), rio = V(P.rio), z = V(Z), rr = V(RR);
-            E::template pass<16>(
-                n, c, [&](long e) { return V2<T>{z[e], rr[e]}; },
-                [&](long e, const V2<T> &v) {
-                    if (capNow) {
-                        zio[e] = v.a;
-                        rio[e] = v.b;
-                    }
-                });
+            takePass<T, E>(n, P.zio, Z, nullptr, T(0), capNow);
+            takePass<T, E>(n, P.rio, RR, nullptr, T(0), capNow);
             __syncthreads();
         }
         if (capNow) {
@@ -276,68 +447,31 @@ __device__ void lockstepSolve(const LaneInst<T> *Pp, Out *outs, double *lds, lon
                 clk.mark(PH_RES);
                 continue;
             }
-            const VW rr = V(RR), z = V(Z), cc = V(C);
-            E::template pass<16>(n, c, [&](long e) { return V2<T>{z[e], cc[e]}; },
-                                 [&](long e, const V2<T> &v) { rr[e] = v.a - v.b; });
+            residualPass<T, E>(n, Z, C, nullptr, RR);
             __syncthreads();
             sRR = T(0);
         } else {
-            // r = z - T(z), ||r||^2 and, in the same pass, the new Anderson column
-            // (src/cache.cuh:861-896) with its Gram entries: Y_head = r - r_prev,
-            // S_head = (z - z_prev) - Y_head
-            double acc[2 * MAXM];
+            ColumnSums<T> a;
+            withMemory(m, [&](auto M) { a = columnPass<T, E, M()>(Pp, Z, C, RP, ZP, RR, head); });
+            sRR = (T) E::sum((double) a.rr, lds, c);
 #pragma unroll
-            for (int q = 0; q < 2 * MAXM; q++) acc[q] = 0.;
-            T accR = T(0);
-            const VW Yh = V(P.hY + (long) head * n * B), Sh = V(P.hS + (long) head * n * B);
-            const VW rr = V(RR), cc = V(C), rp = V(RP), z = V(Z), zp = V(ZP);
-            VW Ys[MAXM];
-#pragma unroll
-            for (int s2 = 0; s2 < MAXM; s2++) Ys[s2] = V(P.hY + (long) (s2 < m ? s2 : 0) * n * B);
-            E::template pass<4>(
-                n, c,
-                [&](long e) {
-                    V4H<T, MAXM> v;
-                    v.a = z[e];
-                    v.b = cc[e];
-                    v.c = rp[e];
-                    v.d = zp[e];
-#pragma unroll
-                    for (int s2 = 0; s2 < MAXM; s2++) v.h[s2] = (s2 < m && s2 != head) ? Ys[s2][e] : T(0);
-                    return v;
-                },
-                [&](long e, const V4H<T, MAXM> &v) {
-                    const T r = v.a - v.b;
-                    rr[e] = r;
-                    accR += r * r;
-                    const T dr = r - v.c;
-                    Yh[e] = dr;
-                    Sh[e] = (v.a - v.d) - dr;
-                    const double drd = (double) dr, rd = (double) r;
-#pragma unroll
-                    for (int s2 = 0; s2 < MAXM; s2++) {
-                        if (s2 < m) {
-                            const double ys = (s2 == head) ? drd : (double) v.h[s2];
-                            acc[s2] += drd * ys;
-                            acc[MAXM + s2] += ys * rd;
-                        }
-                    }
-                });
-            sRR = (T) E::sum((double) accR, lds, c);
-#pragma unroll
-            for (int q = 0; q < 2 * MAXM; q++)
-                if ((q & (MAXM - 1)) < m) acc[q] = E::sum(acc[q], lds, c);
+            for (int q = 0; q < MAXM; q++) {
+                if (q < m) {
+                    a.yy[q] = E::sum(a.yy[q], lds, c);
+                    a.yr[q] = E::sum(a.yr[q], lds, c);
+                }
+            }
 #pragma unroll
             for (int s2 = 0; s2 < MAXM; s2++) {
                 if (s2 < m) {
 #pragma unroll
                     for (int hh = 0; hh < MAXM; hh++) {
                         if (hh == head) {
-                            G[hh][s2] = acc[s2];
-                            G[s2][hh] = acc[s2];
+                            G[hh][s2] = a.yy[s2];
+                            G[s2][hh] = a.yy[s2];
                         }
                     }
-                    gb[s2] = acc[MAXM + s2];
+                    gb[s2] = a.yr[s2];
                 }
             }
         }
@@ -375,15 +509,8 @@ __device__ void lockstepSolve(const LaneInst<T> *Pp, Out *outs, double *lds, lon
             }
         }
         if (anyLane(done)) {  // accepted candidate and its residual are the solve's output
-            const VW zio = V(P.zio), rio = V(P.rio), cc = V(C), rr = V(RR);
-            E::template pass<16>(
-                n, c, [&](long e) { return V2<T>{cc[e], rr[e]}; },
-                [&](long e, const V2<T> &v) {
-                    if (done) {
-                        zio[e] = v.a;
-                        rio[e] = v.b;
-                    }
-                });
+            takePass<T, E>(n, P.zio, C, nullptr, T(0), done);
+            takePass<T, E>(n, P.rio, RR, nullptr, T(0), done);
             __syncthreads();
         }
         if (done) active = false;
@@ -415,35 +542,10 @@ __device__ void lockstepSolve(const LaneInst<T> *Pp, Out *outs, double *lds, lon
         const bool useLS = (it - it0 >= m) && gramSolve(G, gb, m, gs);
         clk.mark(PH_ALS);
         const bool blind = active && (w <= c0 * zeta);
-        {  // d = -S g - r; K0 lanes write cand = z_prev + d (src/cache.cuh:897-898, 1055-1057)
-            T gg[MAXM];
-            VW Ss[MAXM];
+        Coeffs<T> gg;
 #pragma unroll
-            for (int s2 = 0; s2 < MAXM; s2++) {
-                gg[s2] = (useLS && s2 < m) ? (T) gs[s2] : T(0);
-                Ss[s2] = V(P.hS + (long) (s2 < m ? s2 : 0) * n * B);
-            }
-            const VW rp = V(RP), zp = V(ZP), dd = V(D), cc = V(C);
-            E::template pass<4>(
-                n, c,
-                [&](long e) {
-                    VH<T, MAXM> v;
-                    v.a = rp[e];
-                    v.b = zp[e];
-#pragma unroll
-                    for (int s2 = 0; s2 < MAXM; s2++) v.h[s2] = (s2 < m) ? Ss[s2][e] : T(0);
-                    return v;
-                },
-                [&](long e, const VH<T, MAXM> &v) {
-                    T sg = T(0);
-#pragma unroll
-                    for (int s2 = 0; s2 < MAXM; s2++)
-                        if (s2 < m) sg += v.h[s2] * gg[s2];
-                    const T d = -sg - v.a;
-                    if (blind) cc[e] = v.b + d;
-                    else dd[e] = d;
-                });
-        }
+        for (int s2 = 0; s2 < MAXM; s2++) gg.g[s2] = (useLS && s2 < m) ? (T) gs[s2] : T(0);
+        withMemory(m, [&](auto M) { directionPass<T, E, M()>(Pp, RP, ZP, D, C, gg, blind); });
         __syncthreads();
         clk.mark(PH_AAPPLY);
         if (blind) {
@@ -454,37 +556,16 @@ __device__ void lockstepSolve(const LaneInst<T> *Pp, Out *outs, double *lds, lon
         T tau = T(1);
         for (int in = 0; in < P.maxInner; in++) {  // line search (src/cache.cuh:1063-1099)
             if (!anyLane(ls)) break;
-            {
-                const VW d = V(D), zp = V(ZP), ds = V(DS), z = V(Z);
-                E::template pass<16>(
-                    n, c, [&](long e) { return V2<T>{d[e], zp[e]}; },
-                    [&](long e, const V2<T> &v) {
-                        if (ls) {
-                            const T s = v.a * tau;
-                            ds[e] = s;
-                            z[e] = v.b + s;
-                        }
-                    });
-            }
+            trialPass<T, E>(n, D, ZP, DS, Z, tau, ls);
             __syncthreads();
             clk.mark(PH_LINE);
             E::applyT(Pp, Z, C2, phaseAcc);
             clk.skip();
             if (ls) nT++;
-            T sRRt, sRD;
-            {  // r~ = z - T(z), ||r~||^2 and r~ . ds
-                const VW rr = V(RR), z = V(Z), cc = V(C2), ds = V(DS);
-                T a1 = T(0), a2 = T(0);
-                E::template pass<16>(n, c, [&](long e) { return V4<T>{z[e], cc[e], ds[e], T(0)}; },
-                        [&](long e, const V4<T> &v) {
-                            const T d = v.a - v.b;
-                            rr[e] = d;
-                            a1 += d * d;
-                            a2 += d * v.c;
-                        });
-                sRRt = (T) E::sum((double) a1, lds, c);
-                sRD = (T) E::sum((double) a2, lds, c);
-            }
+            // r~ = z - T(z), ||r~||^2 and r~ . ds
+            const V2<T> sums = residualPass<T, E>(n, Z, C2, DS, RR);
+            const T sRRt = (T) E::sum((double) sums.a, lds, c);
+            const T sRD = (T) E::sum((double) sums.b, lds, c);
             clk.mark(PH_RES);
             // <r~, M r~> and <r~, M ds> from two adjoints (src/cache.cuh:1066,1080)
             const Cross2<T> cr = E::adjDots(Pp, RR, DS, lds, true);
@@ -494,10 +575,7 @@ __device__ void lockstepSolve(const LaneInst<T> *Pp, Out *outs, double *lds, lon
             clk.mark(PH_ELL);
             const bool takeK1 = ls && (w <= wSafe) && (wTilde <= c1 * w);
             if (anyLane(takeK1)) {  // K1: cand <- z
-                const VW cc = V(C), z = V(Z);
-                E::template pass<16>(n, c, [&](long e) { return z[e]; }, [&](long e, T v) {
-                    if (takeK1) cc[e] = v;
-                });
+                takePass<T, E>(n, C, Z, nullptr, T(0), takeK1);
                 __syncthreads();
             }
             if (takeK1) {
@@ -509,12 +587,7 @@ __device__ void lockstepSolve(const LaneInst<T> *Pp, Out *outs, double *lds, lon
             const bool takeK2 = still && (rho >= sigma * wTilde * w);
             if (anyLane(takeK2)) {  // K2: cand <- z_prev - f r
                 const T f = lambda * rho / (wTilde * wTilde);
-                const VW cc = V(C), rr = V(RR), zp = V(ZP);
-                E::template pass<16>(
-                    n, c, [&](long e) { return V2<T>{rr[e], zp[e]}; },
-                    [&](long e, const V2<T> &v) {
-                        if (takeK2) cc[e] = v.b - v.a * f;
-                    });
+                takePass<T, E>(n, C, ZP, RR, f, takeK2);
                 __syncthreads();
             }
             if (takeK2) k2++;
@@ -525,10 +598,7 @@ __device__ void lockstepSolve(const LaneInst<T> *Pp, Out *outs, double *lds, lon
             }
             const bool takeK3 = back && (in >= P.maxInner - 1);
             if (anyLane(takeK3)) {  // K3: restore the plain CP step
-                const VW cc = V(C), bk = V(BK);
-                E::template pass<16>(n, c, [&](long e) { return bk[e]; }, [&](long e, T v) {
-                    if (takeK3) cc[e] = v;
-                });
+                takePass<T, E>(n, C, BK, nullptr, T(0), takeK3);
                 __syncthreads();
             }
             if (takeK3) k3++;

@@ -6,7 +6,7 @@
 // and four consecutive rows of its 16 instances are 64 consecutive words.
 //
 // Lane l of a wave serves instance j = l % 16 and row group g = l / 16.  A node's product of a
-// factor M (r x c, column major) with the 16 instances' vectors X (c x 16) is a GEMM on
+// factor M (r x c, packed in operand order) with the 16 instances' vectors X (c x 16) is a GEMM on
 // v_mfma_{f32,f64}_16x16x4: the A operand is a 16 x 4 block of M (lane l holds M[r0 + l%16][k0 + l/16]),
 // the B operand four rows of X (lane l holds X[k0 + l/16][l%16], its own instance's entry) and each
 // lane receives four rows of its instance (RowMap: rows 4g .. 4g + 3 of each 16-row tile in FP32,
@@ -39,11 +39,6 @@
 #define SPK_TILE_KERNEL_CAT(a, b) SPK_TILE_KERNEL_CAT2(a, b)
 #define SPK_TILE_KERNEL(name) SPK_TILE_KERNEL_CAT(name, SPK_TILE_MAX_THREADS)
 #endif
-#ifndef SPK_TILE_KB
-#define SPK_TILE_KB 2  // k-steps of 4 columns whose operands are loaded together (2 measured
-                       // 2.5% faster than 4 on the 229-node problem; 8 spills)
-#endif
-
 namespace spk {
 namespace tile {
 using namespace ls;
@@ -98,7 +93,11 @@ template <typename T>
 struct TV {
     T *p;   // this workgroup's slab of the region
     int j;  // instance within the workgroup
-    __device__ __forceinline__ SPK_GLOBAL T &operator[](long e) const { return ((SPK_GLOBAL T *) p)[e * W + j]; }
+    // the lane's part of the address is a 32-bit byte offset from a scalar base: a workgroup's slab of a
+    // region stays below 4 GiB (a batch of larger ones, at least 64 instances and 19 regions, exceeds the card)
+    __device__ __forceinline__ SPK_GLOBAL T &operator[](long e) const {
+        return *(SPK_GLOBAL T *) ((SPK_GLOBAL char *) p + ((unsigned) e * W + j) * (unsigned) sizeof(T));
+    }
     __device__ __forceinline__ TV shift(long e0) const { return TV{p + e0 * W, j}; }
 };
 
@@ -153,78 +152,153 @@ __device__ __forceinline__ void forRows(int len, F f) {
     }
 }
 
-template <int RT, typename T>
-__device__ __forceinline__ void zeroAcc(Acc<T> (&a)[RT]) {
+template <typename T, int NT>
+__device__ __forceinline__ void zeroTiles(Acc<T> (&a)[NT]) {
 #pragma unroll
-    for (int t = 0; t < RT; t++) a[t] = Acc<T>{T(0), T(0), T(0), T(0)};
+    for (int t = 0; t < NT; t++) a[t] = Acc<T>{T(0), T(0), T(0), T(0)};
 }
 
-// acc[t] += M[16 t + i][c] x(c) summed over c < cols for the 16 t + i < rows of RT row tiles:
-// M is column major with leading dimension ld; x(c) is this lane's instance's entry c.  Every load
-// is clamped into the matrix and the vector, so none is conditional (a conditional load would be
-// waited for on its own): rows past the end compute outputs nobody reads, and columns past the end
-// enter with x multiplied by 0 against finite matrix entries.  The operands of KB k-steps are
-// loaded together before their products, so a wave keeps KB (RT + 1) loads in flight.
-template <int RT, typename T, typename XF>
-__device__ __forceinline__ void mma(Acc<T> (&acc)[RT], CP<T> M, int rows, int ld, int cols, XF x) {
-    constexpr int KB = SPK_TILE_KB;
-    const int i = instLane(), g = rowGroup();
-    int ri[RT];
+// Row block r0 .. (a multiple of 64) of node n's packed factor (PTab): 2 row tiles if it has up to 32
+// rows, else 4.
+template <typename T>
+__device__ __forceinline__ CP<T> packed(const SPK_CONST PTab<T> &t, int n, int r0) {
+    return cst(t.data) + (size_t) cst(t.idx)[n] * t.stride + (size_t) (r0 >> 6) * ((t.cols + 15) >> 4) * 1024;
+}
+
+// acc[t] += M[16 t + i][c] x(c) summed over c < cols for the row tiles of M; x(c) is this lane's instance's
+// entry c.  The factors are packed for this (PTab): 16 columns of a row tile are one run of 64 lanes x 4
+// entries, so an operand of four k-steps is one 16-byte load a lane (two in FP64) at a scalar base, with
+// no clamping (the padding is zero), where the column-major table took four 4-byte loads of four 64-byte
+// runs each, and their addresses.  16 columns are one step, and the next step's operands are requested
+// before a step's products.  Kept a small loop: unrolled over 64 columns at its 17 call
+// sites T grew to 300 KB of code and ran 3 times slower than before.  Columns past the end enter with a
+// valid entry of x against the packing's zeros.
+template <typename T, int NT, typename XF>
+__device__ __forceinline__ void mma(Acc<T> (&acc)[NT], CP<T> M, int cols, XF x) {
+    constexpr bool AHEAD = sizeof(T) == 4;
+    typedef T Vec4 __attribute__((ext_vector_type(4)));
+    const int g = rowGroup();
+    const SPK_CONST Vec4 *base = (const SPK_CONST Vec4 *) M;
+    const unsigned lane = threadIdx.x & 63;
+    Vec4 a[NT], an[NT];
+    T b[4], bn[4];
+    auto load = [&](int c0, Vec4 (&av)[NT], T (&bv)[4]) {
 #pragma unroll
-    for (int t = 0; t < RT; t++) ri[t] = min(16 * t + i, rows - 1);
-    for (int k0 = 0; k0 < cols; k0 += 4 * KB) {
-        T a[KB][RT], b[KB];
+        for (int s = 0; s < 4; s++) bv[s] = x(min(c0 + 4 * s + g, cols - 1));
 #pragma unroll
-        for (int s = 0; s < KB; s++) {
-            const int c = k0 + 4 * s + g;
-            const int cc = min(c, cols - 1);
-            b[s] = x(cc) * T(c < cols ? 1 : 0);
-            CP<T> col = M + (size_t) cc * ld;
+        for (int t = 0; t < NT; t++) av[t] = base[t * 64 + lane];
+        base += NT * 64;
+    };
+    if (AHEAD) load(0, a, b);
+#pragma unroll 1
+    for (int c0 = 0; c0 < cols; c0 += 16) {
+        if (!AHEAD) load(c0, a, b);
+        else if (c0 + 16 < cols) load(c0 + 16, an, bn);
 #pragma unroll
-            for (int t = 0; t < RT; t++) a[s][t] = col[ri[t]];
-        }
-        // steps past the end add zero products (b = 0); no early exit, so the loads above are
-        // all issued before the first product waits for them
+        for (int s = 0; s < 4; s++)
 #pragma unroll
-        for (int s = 0; s < KB; s++) {
+            for (int t = 0; t < NT; t++) acc[t] = mfma(a[t][s], b[s], acc[t]);
+        if (AHEAD) {
 #pragma unroll
-            for (int t = 0; t < RT; t++) acc[t] = mfma(a[s][t], b[s], acc[t]);
+            for (int t = 0; t < NT; t++) a[t] = an[t];
+#pragma unroll
+            for (int s = 0; s < 4; s++) b[s] = bn[s];
         }
     }
 }
 
-template <int RT, typename T, typename F>
-__device__ __forceinline__ void eachOut(const Acc<T> (&acc)[RT], int rows, F f) {
+// The wave's LDS slice: the accumulators of 64 rows, or two staged vectors of 32 rows.
+template <typename T>
+__device__ __forceinline__ SP<T> waveStage() {
+    __shared__ __align__(32) T stage[MAXW * 2 * STG];
+    return (SP<T>) (stage + (threadIdx.x >> 6) * 2 * STG);
+}
+
+// f(row, value) for the rows < `rows` of a row block that this lane owns, straight from the registers
+// (for few rows or a short f: the code of f is repeated for every one).
+template <int NT, typename T, typename F>
+__device__ __forceinline__ void eachOut(Acc<T> (&acc)[NT], int rows, F f) {
     const int g = rowGroup();
 #pragma unroll
-    for (int t = 0; t < RT; t++) {
+    for (int t = 0; t < NT; t++) {
+        if (16 * t < rows) {
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int r = RowMap<T>::row(t, g, q);
-            if (r < rows) f(r, acc[t][q]);
+            for (int q = 0; q < 4; q++) {
+                const int r = RowMap<T>::row(t, g, q);
+                T v = acc[t][q];
+                if (r < rows) f(r, v);
+                acc[t][q] = v;
+            }
         }
     }
 }
 
-template <int RT, typename T, typename Terms, typename F>
-__device__ __forceinline__ void rowGroupProduct(int r0, int rr, Terms &terms, F &out) {
-    Acc<T> a[RT];
-    zeroAcc<RT, T>(a);
-    terms(a, r0, rr);
-    eachOut<RT, T>(a, rr, [&](int r, T v) { out(r0 + r, v); });
+// The same through the lane's own words of the LDS slice, so that one loop over the row tiles serves
+// any number of them (each lane's four values of a tile are contiguous: no bank conflicts).  The
+// return value of f replaces the staged one; again(f) visits the rows once more.
+template <typename T>
+struct StagedOut {
+    typedef T Vec4 __attribute__((ext_vector_type(4)));
+    SPK_LDS Vec4 *st;
+    int rows;
+    template <int NT>
+    __device__ __forceinline__ StagedOut(const Acc<T> (&acc)[NT], int nrows) : rows(nrows) {
+        st = (SPK_LDS Vec4 *) waveStage<T>() + (threadIdx.x & 63);
+#pragma unroll
+        for (int t = 0; t < NT; t++) st[t * 64] = acc[t];
+    }
+    template <bool KEEP, typename F>
+    __device__ __forceinline__ void each(F f) {
+        const int g = rowGroup();
+#pragma unroll 1
+        for (int t = 0; 16 * t < rows; t++) {
+            Vec4 v = st[t * 64];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int r = RowMap<T>::row(t, g, q);
+                if (r < rows) v[q] = f(r, v[q]);
+            }
+            if (KEEP) st[t * 64] = v;
+        }
+    }
+};
+
+// out(r, y_r) for every row r < rows this lane owns, y = the sum of the products terms(acc, r0)
+// accumulates (calls of mma on the row block at r0 of each term's matrix), 64 rows at a time.
+// STAGED: the outputs pass through the LDS slice (which must be free), else straight from registers.
+template <int NT, bool STAGED, typename T, typename Terms, typename F>
+__device__ __forceinline__ void gemvBlock(int r0, int rows, Terms &terms, F &out) {
+    Acc<T> a[NT];
+    zeroTiles<T>(a);
+    terms(a, r0);
+    if constexpr (STAGED) {
+        StagedOut<T> s(a, rows);
+        s.template each<false>([&](int r, T v) {
+            out(r0 + r, v);
+            return v;
+        });
+    } else {
+        eachOut<NT, T>(a, rows, [&](int r, T v) { out(r0 + r, v); });
+    }
 }
 
-// out(r, y_r) for every row r < rows this lane owns, y = the sum of the products terms(acc, r0, rr)
-// accumulates (calls of mma on the row block r0 .. r0 + rr of each term's matrix), 64 rows at a time.
-template <typename T, typename Terms, typename F>
+template <typename T, bool STAGED = true, typename Terms, typename F>
 __device__ __forceinline__ void gemv(int rows, Terms terms, F out) {
+#pragma unroll 1
     for (int r0 = 0; r0 < rows; r0 += 64) {
         const int rr = min(64, rows - r0);
-        if (rr > 48) rowGroupProduct<4, T>(r0, rr, terms, out);
-        else if (rr > 32) rowGroupProduct<3, T>(r0, rr, terms, out);
-        else if (rr > 16) rowGroupProduct<2, T>(r0, rr, terms, out);
-        else rowGroupProduct<1, T>(r0, rr, terms, out);
+        if (rr > 32) gemvBlock<4, STAGED, T>(r0, rr, terms, out);
+        else gemvBlock<2, STAGED, T>(r0, rr, terms, out);
     }
+}
+
+// The same for up to 32 rows, from the registers.
+template <typename T, typename Terms, typename F>
+__device__ __forceinline__ void gemv32(int rows, Terms terms, F out) {
+    Acc<T> a[2];
+    zeroTiles<T>(a);
+    terms(a, 0);
+    eachOut<2, T>(a, rows, out);
 }
 
 template <typename T>
@@ -255,16 +329,13 @@ __device__ __forceinline__ void adjNode(LP<T> P, const TV<T> &d, int n, E emit) 
             const int rows = part == 0 ? nx : nu;
             gemv<T>(
                 rows,
-                [&](auto &acc, int r0, int rr) {
+                [&](auto &acc, int r0) {
                     if (P.ncon == CON_POLY_DEV)
-                        mma(acc, tab(P.nGT, n) + part * nx + r0, rr, nxu, P.con3, [&](int cc) { return d[b3 + cc]; });
+                        mma<T>(acc, packed(part == 0 ? P.pGTx : P.pGTu, n, r0), P.con3, [&](int cc) { return d[b3 + cc]; });
                     if (P.ncost == COST_LIN_DEV) return;  // elementwise below
                     for (int ci = 0; ci < nc; ci++) {  // children accumulate (src/costs.cuh:172-177)
-                        const long iv = P.oIV + (long) (c0 + ci) * d4;
-                        if (part == 0)
-                            mma(acc, tab(P.sQ, c0 + ci) + r0, rr, nx, nx, [&](int cc) { return d[iv + cc]; });
-                        else
-                            mma(acc, tab(P.sR, c0 + ci) + r0, rr, nu, nu, [&](int cc) { return d[iv + nx + cc]; });
+                        const long iv = P.oIV + (long) (c0 + ci) * d4 + part * nx;
+                        mma<T>(acc, packed(part == 0 ? P.psQ : P.psR, c0 + ci, r0), rows, [&](int cc) { return d[iv + cc]; });
                     }
                 },
                 [&](int r, T v) {
@@ -295,10 +366,9 @@ __device__ __forceinline__ void adjNode(LP<T> P, const TV<T> &d, int n, E emit) 
         const T a = lin ? T(0) : d[vi + nx], bb = lin ? T(0) : d[vi + nx + 1];
         gemv<T>(
             nx,
-            [&](auto &acc, int r0, int rr) {
-                if (P.lcon == CON_POLY_DEV)
-                    mma(acc, tab(P.lGT, l) + r0, rr, nx, P.con5, [&](int cc) { return d[b5 + cc]; });
-                if (!lin) mma(acc, tab(P.lsQ, l) + r0, rr, nx, nx, [&](int cc) { return d[vi + cc]; });
+            [&](auto &acc, int r0) {
+                if (P.lcon == CON_POLY_DEV) mma<T>(acc, packed(P.plGT, l, r0), P.con5, [&](int cc) { return d[b5 + cc]; });
+                if (!lin) mma<T>(acc, packed(P.plsQ, l, r0), nx, [&](int cc) { return d[vi + cc]; });
             },
             [&](int r, T v) {
                 if (P.lcon == CON_RECT_DEV) v += d[b5 + r];
@@ -349,11 +419,11 @@ __device__ __forceinline__ void opNode(LP<T> P, int n, PV pv, H &h) {
             forRows<T>(nx, [&](int k) { h.elemBox(base + k, pv(P.oX + (long) n * nx + k), lb[k], ub[k]); });
             forRows<T>(nu, [&](int k) { h.elemBox(base + nx + k, pv(P.oU + (long) n * nu + k), lb[nx + k], ub[nx + k]); });
         } else if (P.ncon == CON_POLY_DEV) {
-            CP<T> G = tab(P.nG, n), lb = tab(P.nLB, n), ub = tab(P.nUB, n);
+            CP<T> lb = tab(P.nLB, n), ub = tab(P.nUB, n);
             gemv<T>(
                 P.con3,
-                [&](auto &acc, int r0, int rr) {
-                    mma(acc, G + r0, rr, P.con3, nxu, [&](int cc) {
+                [&](auto &acc, int r0) {
+                    mma<T>(acc, packed(P.pG, n, r0), nxu, [&](int cc) {
                         return cc < nx ? pv(P.oX + (long) n * nx + cc) : pv(P.oU + (long) n * nu + cc - nx);
                     });
                 },
@@ -374,34 +444,47 @@ __device__ __forceinline__ void opNode(LP<T> P, int n, PV pv, H &h) {
     } else {  // IV
         const long base = P.oIV + (long) n * (nxu + 2);
         CP<T> tr = tab(P.trans, n);
-        h.socBegin();
         if (n >= 1) {
             const int a = cst(P.anc)[n];
-            gemv<T>(
-                nx,
-                [&](auto &acc, int r0, int rr) {
-                    mma(acc, tab(P.sQ, n) + r0, rr, nx, nx, [&](int cc) { return pv(P.oX + (long) a * nx + cc); });
-                },
-                [&](int r, T v) { h.socPart(base + r, v, tr[r]); });
-            gemv<T>(
-                nu,
-                [&](auto &acc, int r0, int rr) {
-                    mma(acc, tab(P.sR, n) + r0, rr, nu, nu, [&](int cc) { return pv(P.oU + (long) a * nu + cc); });
-                },
-                [&](int r, T v) { h.socPart(base + nx + r, v, tr[nx + r]); });
+            auto xa = [&](int cc) { return pv(P.oX + (long) a * nx + cc); };
+            auto ua = [&](int cc) { return pv(P.oU + (long) a * nu + cc); };
             T hv = pv(P.oT + n) * T(0.5);
             if (P.ncost == COST_QUADLIN_DEV) {
                 CP<T> qn = tab(P.q, n), rn = tab(P.r, n);
                 T pq = T(0), pr = T(0);
-                forRows<T>(nx, [&](int k) { pq += qn[k] * pv(P.oX + (long) a * nx + k); });
-                forRows<T>(nu, [&](int k) { pr += rn[k] * pv(P.oU + (long) a * nu + k); });
+                forRows<T>(nx, [&](int k) { pq += qn[k] * xa(k); });
+                forRows<T>(nu, [&](int k) { pr += rn[k] * ua(k); });
                 pq = sumG(pq);
                 pr = sumG(pr);
                 hv = hv + T(-0.5) * pq;
                 hv = hv + T(-0.5) * pr;
             }
-            h.socEnd(base, nx, nu, hv, tr);
+            auto soc = [&](auto &ax) {
+                zeroTiles<T>(ax);
+                Acc<T> au[2];
+                zeroTiles<T>(au);
+                mma<T>(ax, packed(P.psQ, n, 0), nx, xa);
+                mma<T>(au, packed(P.psR, n, 0), nu, ua);
+                h.socRegs(base, ax, nx, au, nu, hv, tr);
+            };
+            if (nx <= 32) {  // the block's entries stay with the wave (nu <= 32)
+                Acc<T> ax[2];
+                soc(ax);
+            } else if (nx <= 64) {
+                Acc<T> ax[4];
+                soc(ax);
+            } else {
+                h.socBegin();
+                gemv<T>(
+                    nx, [&](auto &acc, int r0) { mma<T>(acc, packed(P.psQ, n, r0), nx, xa); },
+                    [&](int r, T v) { h.socPart(base + r, v, tr[r]); });
+                gemv<T>(
+                    nu, [&](auto &acc, int r0) { mma<T>(acc, packed(P.psR, n, r0), nu, ua); },
+                    [&](int r, T v) { h.socPart(base + nx + r, v, tr[nx + r]); });
+                h.socEnd(base, nx, nu, hv, tr);
+            }
         } else {
+            h.socBegin();
             forRows<T>(nx, [&](int r) { h.socPart(base + r, T(0), tr[r]); });
             forRows<T>(nu, [&](int r) { h.socPart(base + nx + r, T(0), tr[nx + r]); });
             h.socEnd(base, nx, nu, T(0), tr);
@@ -417,9 +500,7 @@ __device__ __forceinline__ void opNode(LP<T> P, int n, PV pv, H &h) {
             CP<T> lb = tab(P.lLB, l), ub = tab(P.lUB, l);
             gemv<T>(
                 P.con5,
-                [&](auto &acc, int r0, int rr) {
-                    mma(acc, tab(P.lG, l) + r0, rr, P.con5, nx, [&](int cc) { return pv(P.oX + (long) n * nx + cc); });
-                },
+                [&](auto &acc, int r0) { mma<T>(acc, packed(P.plG, l, r0), nx, [&](int cc) { return pv(P.oX + (long) n * nx + cc); }); },
                 [&](int r, T v) { h.elemBox(b5 + r, v, lb[r], ub[r]); });
         }
         if (P.lcost == COST_LIN_DEV) {  // VI: (q' x_l, s_l) (src/costs.cuh:269-272)
@@ -432,29 +513,43 @@ __device__ __forceinline__ void opNode(LP<T> P, int n, PV pv, H &h) {
         }
         const long base = P.oVI + (long) l * (nx + 2);
         CP<T> tr = tab(P.ltrans, l);
-        h.socBegin();
-        gemv<T>(
-            nx,
-            [&](auto &acc, int r0, int rr) {
-                mma(acc, tab(P.lsQ, l) + r0, rr, nx, nx, [&](int cc) { return pv(P.oX + (long) n * nx + cc); });
-            },
-            [&](int r, T v) { h.socPart(base + r, v, tr[r]); });
+        auto xl = [&](int cc) { return pv(P.oX + (long) n * nx + cc); };
         T hs = pv(P.oS + n) * T(0.5);
         if (P.lcost == COST_QUADLIN_DEV) {
             CP<T> lq = tab(P.lq, l);
             T pq = T(0);
-            forRows<T>(nx, [&](int k) { pq += lq[k] * pv(P.oX + (long) n * nx + k); });
+            forRows<T>(nx, [&](int k) { pq += lq[k] * xl(k); });
             pq = sumG(pq);
             hs = hs + T(-0.5) * pq;
         }
-        h.socEnd(base, nx, 0, hs, tr);
+        auto soc = [&](auto &ax) {
+            zeroTiles<T>(ax);
+            Acc<T> au[2];
+            zeroTiles<T>(au);
+            mma<T>(ax, packed(P.plsQ, l, 0), nx, xl);
+            h.socRegs(base, ax, nx, au, 0, hs, tr);
+        };
+        if (nx <= 32) {
+            Acc<T> ax[2];
+            soc(ax);
+        } else if (nx <= 64) {
+            Acc<T> ax[4];
+            soc(ax);
+        } else {
+            h.socBegin();
+            gemv<T>(
+                nx, [&](auto &acc, int r0) { mma<T>(acc, packed(P.plsQ, l, r0), nx, xl); },
+                [&](int r, T v) { h.socPart(base + r, v, tr[r]); });
+            h.socEnd(base, nx, 0, hs, tr);
+        }
     }
 }
 
 // Dual prox of the CP step (src/cache.cuh:770-789): w = (L gamma + z_d)/gamma + c and
 // cand_d = gamma (w - Pi(w)), Pi the masked NNOC (src/risks.cuh:99-106), NNOC (src/cones.cuh:134-137),
-// box (src/constraints.cuh:70-74) or SOC (src/projections.cuh:102-128).  SOC blocks stage w in
-// cand_d (each lane its own rows), accumulate |w|^2 and rescale in socEnd.
+// box (src/constraints.cuh:70-74) or SOC (src/projections.cuh:102-128).  SOC blocks of up to 64 states
+// keep w in registers (socRegs); larger ones stage it in cand_d (each lane its own rows), accumulate
+// |w|^2 and rescale in socEnd.
 template <typename T>
 struct Prox {
     LP<T> P;
@@ -482,8 +577,8 @@ struct Prox {
         cd[e] = w;
         ss += w * w;
     }
-    __device__ __forceinline__ void socEnd(long base, int n1, int n2, T hv, CP<T> tr) {
-        const int dim = n1 + n2 + 2;
+    // the factor of the block's vector part; the last two entries are written
+    __device__ __forceinline__ T socScale(long base, int dim, T hv, CP<T> tr) {
         const long k1 = base + dim - 2, k2 = base + dim - 1;
         const T w1 = wOf(hv, k1, tr[dim - 2]);
         const T w2 = wOf(hv, k2, tr[dim - 1]);
@@ -494,12 +589,6 @@ struct Prox {
         const int i3 = !i1 && !i2;
         const T sc = (nrm + tl) / (T(2) * nrm + T(1 - i3));
         const T mult = T(1 - i2) * (T(i3) * sc + T(1 - i3));
-        auto rescale = [&](long e) {
-            const T w = cd[e];
-            cd[e] = (w - w * mult) * P.gamma;
-        };
-        forRows<T>(n1, [&](int r) { rescale(base + r); });
-        forRows<T>(n2, [&](int r) { rescale(base + n1 + r); });
         if (rowGroup() == 0) {
             const T p1 = w1 * mult;
             const int i1b = (1 - i2) * (1 - i3);
@@ -507,6 +596,36 @@ struct Prox {
             cd[k1] = (w1 - p1) * P.gamma;
             cd[k2] = (w2 - p2) * P.gamma;
         }
+        return mult;
+    }
+    template <int NT>
+    __device__ __forceinline__ void socRegs(long base, Acc<T> (&ax)[NT], int n1, Acc<T> (&au)[2], int n2, T hv, CP<T> tr) {
+        ss = T(0);
+        StagedOut<T> x(ax, n1);
+        x.template each<true>([&](int r, T v) {
+            const T w = wOf(v, base + r, tr[r]);
+            ss += w * w;
+            return w;
+        });
+        eachOut<2, T>(au, n2, [&](int r, T &v) {
+            v = wOf(v, base + n1 + r, tr[n1 + r]);
+            ss += v * v;
+        });
+        const T mult = socScale(base, n1 + n2 + 2, hv, tr);
+        x.template each<false>([&](int r, T w) {
+            cd[base + r] = (w - w * mult) * P.gamma;
+            return w;
+        });
+        eachOut<2, T>(au, n2, [&](int r, T &w) { cd[base + n1 + r] = (w - w * mult) * P.gamma; });
+    }
+    __device__ __forceinline__ void socEnd(long base, int n1, int n2, T hv, CP<T> tr) {
+        const T mult = socScale(base, n1 + n2 + 2, hv, tr);
+        auto rescale = [&](long e) {
+            const T w = cd[e];
+            cd[e] = (w - w * mult) * P.gamma;
+        };
+        forRows<T>(n1, [&](int r) { rescale(base + r); });
+        forRows<T>(n2, [&](int r) { rescale(base + n1 + r); });
     }
     __device__ __forceinline__ void lin(long eSum, long eSet, T sum, T set) {
         const T ws = wOf(sum, eSum, T(0)), wt = wOf(set, eSet, T(0));
@@ -538,6 +657,16 @@ struct Red {
         acc(P.sPrim + base + dim - 2, hv);
         acc(P.sPrim + base + dim - 1, hv);
     }
+    template <int NT>
+    __device__ __forceinline__ void socRegs(long base, Acc<T> (&ax)[NT], int n1, Acc<T> (&au)[2], int n2, T hv, CP<T> tr) {
+        StagedOut<T> x(ax, n1);
+        x.template each<false>([&](int r, T v) {
+            acc(P.sPrim + base + r, v);
+            return v;
+        });
+        eachOut<2, T>(au, n2, [&](int r, T v) { acc(P.sPrim + base + n1 + r, v); });
+        socEnd(base, n1, n2, hv, tr);
+    }
     __device__ __forceinline__ void lin(long eSum, long eSet, T sum, T set) {
         acc(P.sPrim + eSum, sum);
         acc(P.sPrim + eSet, set);
@@ -558,6 +687,12 @@ struct Store {
         const int dim = n1 + n2 + 2;
         out[base + dim - 2] = hv;
         out[base + dim - 1] = hv;
+    }
+    template <int NT>
+    __device__ __forceinline__ void socRegs(long base, Acc<T> (&ax)[NT], int n1, Acc<T> (&au)[2], int n2, T hv, CP<T> tr) {
+        eachOut<NT, T>(ax, n1, [&](int r, T v) { out[base + r] = v; });
+        eachOut<2, T>(au, n2, [&](int r, T v) { out[base + n1 + r] = v; });
+        socEnd(base, n1, n2, hv, tr);
     }
     __device__ __forceinline__ void lin(long eSum, long eSet, T sum, T set) {
         out[eSum] = sum;
@@ -605,20 +740,17 @@ __device__ __forceinline__ void dynBackward(LP<T> P, const TV<T> &cand, const TV
     const bool affine = P.affine != 0;
     auto qv = [&](int j, int cc) { return affine ? qd[(long) j * nx + cc] + tab(P.Pe, j)[cc] : qd[(long) j * nx + cc]; };
     // e = ubar - sum_j B_j' q_j
-    gemv<T>(
+    gemv32<T>(
         nu,
-        [&](auto &acc, int r0, int rr) {
-            for (int ci = 0; ci < nc; ci++)
-                mma(acc, tab(P.BTr, c0 + ci) + r0, rr, nu, nx, [&](int cc) { return qv(c0 + ci, cc); });
+        [&](auto &acc, int r0) {
+            for (int ci = 0; ci < nc; ci++) mma<T>(acc, packed(P.pBTr, c0 + ci, r0), nx, [&](int cc) { return qv(c0 + ci, cc); });
         },
         [&](int r, T v) { e1[r * W + jj] = -v + cand[P.oU + (long) i * nu + r]; });
     __builtin_amdgcn_wave_barrier();
     // d = R~^-1 e
-    gemv<T>(
+    gemv32<T>(
         nu,
-        [&](auto &acc, int r0, int rr) {
-            mma(acc, tab(P.RtInv, i) + r0, rr, nu, nu, [&](int cc) { return e1[cc * W + jj]; });
-        },
+        [&](auto &acc, int r0) { mma<T>(acc, packed(P.pRtInv, i, r0), nu, [&](int cc) -> T { return e1[cc * W + jj]; }); },
         [&](int r, T v) {
             dd[(long) i * nu + r] = v;
             d1[r * W + jj] = v;
@@ -628,14 +760,13 @@ __device__ __forceinline__ void dynBackward(LP<T> P, const TV<T> &cand, const TV
     // q_i = sum_j (APB_j d_i + ABKTr_j q_j) + K_i'(d_i - u_i) - x_i
     gemv<T>(
         nx,
-        [&](auto &acc, int r0, int rr) {
+        [&](auto &acc, int r0) {
             for (int ci = 0; ci < nc; ci++) {
                 const int j = c0 + ci;
-                mma(acc, tab(P.APB, j) + r0, rr, nx, nu, [&](int cc) { return d1[cc * W + jj]; });
-                mma(acc, tab(P.ABKTr, j) + r0, rr, nx, nx, [&](int cc) { return qv(j, cc); });
+                mma<T>(acc, packed(P.pAPB, j, r0), nu, [&](int cc) -> T { return d1[cc * W + jj]; });
+                mma<T>(acc, packed(P.pABKTr, j, r0), nx, [&](int cc) { return qv(j, cc); });
             }
-            mma(acc, tab(P.KTr, i) + r0, rr, nx, nu,
-                [&](int cc) { return d1[cc * W + jj] - cand[P.oU + (long) i * nu + cc]; });
+            mma<T>(acc, packed(P.pKTr, i, r0), nu, [&](int cc) -> T { return d1[cc * W + jj] - cand[P.oU + (long) i * nu + cc]; });
         },
         [&](int r, T v) { qd[(long) i * nx + r] = v - cand[P.oX + (long) i * nx + r]; });
 }
@@ -651,7 +782,7 @@ __device__ __forceinline__ void kernelProj(LP<T> P, const TV<T> &cand, int i) {
         return (k - yD - E < nc) ? cand[P.oS + c0 + (k - yD - E)] : T(0);
     };
     gemv<T>(
-        P.nD, [&](auto &acc, int r0, int rr) { mma(acc, tab(P.NN, i) + r0, rr, P.nD, P.nD, vin); },
+        P.nD, [&](auto &acc, int r0) { mma<T>(acc, packed(P.pNN, i, r0), P.nD, vin); },
         [&](int k, T v) {
             if (k < yD) cand[P.oY + (long) i * yD + k] = v;
             else if (k < yD + E) {
@@ -672,8 +803,8 @@ __device__ __forceinline__ void dynForward(LP<T> P, const TV<T> &cand, const TV<
     // x_0 is the (scaled) initial state; other nodes' x were written by their parent's step
     auto xv = [&](int cc) { return i == 0 ? x0s[cc] : cand[P.oX + (long) i * nx + cc]; };
     if (i == 0) forRows<T>(nx, [&](int r) { cand[P.oX + r] = x0s[r]; });
-    gemv<T>(
-        nu, [&](auto &acc, int r0, int rr) { mma(acc, tab(P.K, i) + r0, rr, nu, nx, xv); },
+    gemv32<T>(
+        nu, [&](auto &acc, int r0) { mma<T>(acc, packed(P.pK, i, r0), nx, xv); },
         [&](int r, T v) {
             const T u = v + dd[(long) i * nu + r];
             cand[P.oU + (long) i * nu + r] = u;
@@ -683,11 +814,10 @@ __device__ __forceinline__ void dynForward(LP<T> P, const TV<T> &cand, const TV<
     const int c0 = cst(P.chFrom)[i], nc = cst(P.numCh)[i];
     for (int ci = 0; ci < nc; ci++) {
         const int j = c0 + ci;
-        gemv<T>(
+        gemv<T, false>(  // u1 stays in the LDS slice for the next child
             nx,
-            [&](auto &acc, int r0, int rr) {
-                mma(acc, tab(P.AB, j) + r0, rr, nx, nx + nu,
-                    [&](int cc) { return cc < nx ? xv(cc) : u1[(cc - nx) * W + jj]; });
+            [&](auto &acc, int r0) {
+                mma<T>(acc, packed(P.pAB, j, r0), nx + nu, [&](int cc) -> T { return cc < nx ? xv(cc) : u1[(cc - nx) * W + jj]; });
             },
             [&](int r, T v) {
                 if (P.affine) v += tab(P.e, j)[r];
@@ -727,12 +857,6 @@ __device__ __forceinline__ void phaseDual(LP<T> P, const Ctx &c, const TV<T> &z,
     Prox<T> h{P, z.shift(P.sPrim), cand.shift(P.sPrim), T(0)};
     auto pv = [&](long e) { return cand[e] * T(2) - z[e]; };
     for (int n = c.wave; n < P.N; n += c.nw) opNode(P, n, pv, h);
-}
-
-template <typename T>
-__device__ __forceinline__ SP<T> waveStage() {
-    __shared__ __align__(16) T stage[MAXW * 2 * STG];
-    return (SP<T>) (stage + (threadIdx.x >> 6) * 2 * STG);
 }
 
 // The CP operator T (src/cache.cuh:796-801): cand = T(z).
@@ -839,19 +963,18 @@ __device__ __forceinline__ void pass(long n, const Ctx &c, Ld ld, St st) {
     using Vals = decltype(ld(0L));
     const long per = (((n + c.nw - 1) / c.nw) + 3) & ~3L;
     const long e0 = (long) c.wave * per, e1 = min(n, e0 + per);
-    for (long b = e0; b < e1; b += 4 * U) {
+    long b = e0;
+#pragma unroll 1
+    for (; b + 4 * U <= e1; b += 4 * U) {  // no conditions: all U loads are in flight together
         Vals v[U];
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const long e = b + 4 * u + c.g;
-            if (e < e1) v[u] = ld(e);
-        }
+        for (int u = 0; u < U; u++) v[u] = ld(b + 4 * u + c.g);
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const long e = b + 4 * u + c.g;
-            if (e < e1) st(e, v[u]);
-        }
+        for (int u = 0; u < U; u++) st(b + 4 * u + c.g, v[u]);
     }
+#pragma unroll 1
+    for (; b < e1; b += 4)
+        if (b + c.g < e1) st(b + c.g, ld(b + c.g));
 }
 
 // The tile engine as a policy of the lockstep solve.
