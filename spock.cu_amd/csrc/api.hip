@@ -232,6 +232,9 @@ void ensureUploaded(spk_problem *p) {
     X(lsQ, lsQ, 0, h.nx) X(G, nG, 0, h.con3) X(GTx, nGT, 0, h.nx) X(GTu, nGT, h.nx, h.nu) X(lG, lG, 0, h.con5) \
     X(lGT, lGT, 0, h.nx)
 
+// row tiles of a block with `rows` rows left, as the kernels unroll them
+int packedTiles(int rows) { return rows > 32 ? 4 : rows > 16 ? 2 : 1; }
+
 template <typename T>
 void uploadPacked(spk_problem *p, const std::string &name, const Table &t, int row0, int rows) {
     DevTableSet<T> s;
@@ -240,13 +243,13 @@ void uploadPacked(spk_problem *p, const std::string &name, const Table &t, int r
     const int kg = (t.cols + 15) / 16;
     const size_t sz = (size_t) t.rows * t.cols, count = sz && rows ? t.data.size() / sz : 0;
     size_t stride = 0;
-    for (int r0 = 0; r0 < rows; r0 += 64) stride += (size_t) kg * (rows - r0 > 32 ? 4 : 2) * 256;
+    for (int r0 = 0; r0 < rows; r0 += 64) stride += (size_t) kg * packedTiles(rows - r0) * 256;
     std::vector<T> d(std::max<size_t>(1, count * stride), T(0));
     for (size_t m = 0; m < count; m++) {
         T *out = d.data() + m * stride;
         const double *M = t.data.data() + m * sz + row0;
         for (int r0 = 0; r0 < rows; r0 += 64) {
-            const int tiles = rows - r0 > 32 ? 4 : 2;
+            const int tiles = packedTiles(rows - r0);
             for (int c = 0; c < t.cols; c++)
                 for (int r = r0; r < std::min(rows, r0 + 64); r++) {
                     const int tile = (r - r0) / 16, lane = (r & 15) + 16 * (c & 3);
@@ -689,7 +692,7 @@ size_t laneLayout(spk_batch *b) {
     off += (size_t) h.nu * h.nl * B;
     b->lRegion[LR_X0] = off;
     off += (size_t) h.nx * B;
-    return off;
+    return off + 64 * 64;  // the tile engine reads whole row blocks, up to 64 rows past a region's end
 }
 
 template <typename T>

@@ -45,7 +45,7 @@ __device__ __forceinline__ CP<T> tab(const SPK_CONST DTab<T> &t, int n) {
 
 // The same table packed for the tile engine's products: per distinct matrix and block of 64 rows,
 // [16-column group][16-row tile][lane][4], lane l holding M[16 t + l % 16][16 k + 4 s + l / 16] at
-// position s, zero past the matrix, with 2 row tiles in a block of up to 32 rows and 4 in a larger one.
+// position s, zero past the matrix, with 1, 2 or 4 row tiles in a block of up to 16, 32 or 64 rows.
 // `stride` entries per matrix.
 template <typename T>
 struct PTab {

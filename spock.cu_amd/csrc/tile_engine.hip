@@ -26,6 +26,8 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include <type_traits>
+
 // Launch bound of this compilation: 512 threads (two waves per SIMD, up to 256 registers each) or 1024
 // (four waves per SIMD, 128 registers each: more waves to hide memory latency, more spills).  The
 // library is built once per bound; the 1024 build's kernels carry the suffix _x1024.
@@ -158,8 +160,7 @@ __device__ __forceinline__ void zeroTiles(Acc<T> (&a)[NT]) {
     for (int t = 0; t < NT; t++) a[t] = Acc<T>{T(0), T(0), T(0), T(0)};
 }
 
-// Row block r0 .. (a multiple of 64) of node n's packed factor (PTab): 2 row tiles if it has up to 32
-// rows, else 4.
+// Row block r0 .. (a multiple of 64) of node n's packed factor (PTab): 1, 2 or 4 row tiles.
 template <typename T>
 __device__ __forceinline__ CP<T> packed(const SPK_CONST PTab<T> &t, int n, int r0) {
     return cst(t.data) + (size_t) cst(t.idx)[n] * t.stride + (size_t) (r0 >> 6) * ((t.cols + 15) >> 4) * 1024;
@@ -169,40 +170,48 @@ __device__ __forceinline__ CP<T> packed(const SPK_CONST PTab<T> &t, int n, int r
 // entry c.  The factors are packed for this (PTab): 16 columns of a row tile are one run of 64 lanes x 4
 // entries, so an operand of four k-steps is one 16-byte load a lane (two in FP64) at a scalar base, with
 // no clamping (the padding is zero), where the column-major table took four 4-byte loads of four 64-byte
-// runs each, and their addresses.  16 columns are one step, and the next step's operands are requested
-// before a step's products.  Kept a small loop: unrolled over 64 columns at its 17 call
-// sites T grew to 300 KB of code and ran 3 times slower than before.  Columns past the end enter with a
-// valid entry of x against the packing's zeros.
+// runs each, and their addresses.  The vector's entries of up to
+// 64 columns are requested together in FP32 (16 in FP64, whose registers they would take).  Code size
+// matters at 17 call sites: with the factor's loads and the products of 64 columns unrolled as well T was
+// 300 KB of code and 3 times slower.  Columns past the end enter with a valid entry of x against the
+// packing's zeros.
 template <typename T, int NT, typename XF>
 __device__ __forceinline__ void mma(Acc<T> (&acc)[NT], CP<T> M, int cols, XF x) {
-    constexpr bool AHEAD = sizeof(T) == 4;
     typedef T Vec4 __attribute__((ext_vector_type(4)));
     const int g = rowGroup();
     const SPK_CONST Vec4 *base = (const SPK_CONST Vec4 *) M;
     const unsigned lane = threadIdx.x & 63;
-    Vec4 a[NT], an[NT];
-    T b[4], bn[4];
-    auto load = [&](int c0, Vec4 (&av)[NT], T (&bv)[4]) {
+    auto loadX = [&](int c0, T *b) {
 #pragma unroll
-        for (int s = 0; s < 4; s++) bv[s] = x(min(c0 + 4 * s + g, cols - 1));
-#pragma unroll
-        for (int t = 0; t < NT; t++) av[t] = base[t * 64 + lane];
-        base += NT * 64;
+        for (int s = 0; s < 4; s++) b[s] = x(min(c0 + 4 * s + g, cols - 1));
     };
-    if (AHEAD) load(0, a, b);
-#pragma unroll 1
-    for (int c0 = 0; c0 < cols; c0 += 16) {
-        if (!AHEAD) load(c0, a, b);
-        else if (c0 + 16 < cols) load(c0 + 16, an, bn);
+    auto step = [&](const T *b) {
+        Vec4 a[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) a[t] = base[t * 64 + lane];
+        base += NT * 64;
 #pragma unroll
         for (int s = 0; s < 4; s++)
 #pragma unroll
             for (int t = 0; t < NT; t++) acc[t] = mfma(a[t][s], b[s], acc[t]);
-        if (AHEAD) {
+    };
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll 1
+        for (int c0 = 0; c0 < cols; c0 += 64) {
+            T b[16];
 #pragma unroll
-            for (int t = 0; t < NT; t++) a[t] = an[t];
+            for (int k = 0; k < 4; k++)
+                if (c0 + 16 * k < cols) loadX(c0 + 16 * k, b + 4 * k);
 #pragma unroll
-            for (int s = 0; s < 4; s++) b[s] = bn[s];
+            for (int k = 0; k < 4; k++)
+                if (c0 + 16 * k < cols) step(b + 4 * k);
+        }
+    } else {
+#pragma unroll 1
+        for (int c0 = 0; c0 < cols; c0 += 16) {
+            T b[4];
+            loadX(c0, b);
+            step(b);
         }
     }
 }
@@ -288,17 +297,9 @@ __device__ __forceinline__ void gemv(int rows, Terms terms, F out) {
     for (int r0 = 0; r0 < rows; r0 += 64) {
         const int rr = min(64, rows - r0);
         if (rr > 32) gemvBlock<4, STAGED, T>(r0, rr, terms, out);
+        else if (rr <= 16) gemvBlock<1, STAGED, T>(r0, rr, terms, out);
         else gemvBlock<2, STAGED, T>(r0, rr, terms, out);
     }
-}
-
-// The same for up to 32 rows, from the registers.
-template <typename T, typename Terms, typename F>
-__device__ __forceinline__ void gemv32(int rows, Terms terms, F out) {
-    Acc<T> a[2];
-    zeroTiles<T>(a);
-    terms(a, 0);
-    eachOut<2, T>(a, rows, out);
 }
 
 template <typename T>
@@ -309,26 +310,149 @@ __device__ __forceinline__ T projBox(T v, T lb, T ub) {  // src/definitions.cu:3
     return v * T(1 - lower) * T(1 - upper) + lbi + ubi;
 }
 
+// ------------------------------------------------------------------ rows of a node's block
+// Row (t, q) of the lane in a block of rows: a scalar base, the lane's own offset and an immediate, so a
+// block's loads are one instruction each and all in flight together.  They are not conditional: rows past
+// the block read what follows it in the region (the state buffer is padded by 64 rows) and are not used.
+template <typename T>
+__device__ __forceinline__ unsigned rowLane() {
+    return ((unsigned) RowMap<T>::row(0, rowGroup(), 0) * W + instLane()) * (unsigned) sizeof(T);
+}
+
+template <typename T>
+__device__ __forceinline__ SPK_GLOBAL T &rowAt(const TV<T> &v, long e0, unsigned lo, int t, int q) {
+    return *(SPK_GLOBAL T *) ((SPK_GLOBAL char *) (v.p + e0 * W) + lo + RowMap<T>::row(t, 0, q) * W * (int) sizeof(T));
+}
+
+template <typename T, int NT>
+__device__ __forceinline__ void loadRows(const TV<T> &v, long e0, unsigned lo, T (&out)[NT][4]) {
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) out[t][q] = rowAt(v, e0, lo, t, q);
+}
+
+// The same of a per-node vector of a table (padded by 64 entries).
+template <typename T, int NT>
+__device__ __forceinline__ void loadRows(CP<T> p, T (&out)[NT][4]) {
+    const int r0 = RowMap<T>::row(0, rowGroup(), 0);
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) out[t][q] = (p + RowMap<T>::row(t, 0, q))[r0];
+}
+
+// f(t, q, r) for the rows r < `rows` of a block of up to NT tiles.
+template <typename T, int NT, typename F>
+__device__ __forceinline__ void eachRow(int rows, F f) {
+    const int g = rowGroup();
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        if (16 * t < rows) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int r = RowMap<T>::row(t, g, q);
+                if (r < rows) f(t, q, r);
+            }
+        }
+    }
+}
+
+// What a handler reads of the rows of a block besides the products.  In FP32 it is requested before the
+// products, so that it arrives with their operands; in FP64 after them, two row tiles at a time (the
+// registers do not hold more).
+template <typename T, int NT>
+struct Pre {
+    T a[NT][4], b[NT][4];
+};
+template <typename T>
+constexpr bool EARLY = sizeof(T) == 4;
+
+// f(first tile, its accumulators) for the parts of NT row tiles that are handled together.
+template <typename T, int NT, typename F>
+__device__ __forceinline__ void eachPart(Acc<T> (&a)[NT], F f) {
+    constexpr int CH = EARLY<T> ? NT : (NT < 2 ? NT : 2);
+#pragma unroll
+    for (int t0 = 0; t0 < NT; t0 += CH) {
+        Acc<T> part[CH];
+#pragma unroll
+        for (int t = 0; t < CH; t++) part[t] = a[t0 + t];
+        f(t0, part);
+#pragma unroll
+        for (int t = 0; t < CH; t++) a[t0 + t] = part[t];
+    }
+}
+
 // ------------------------------------------------------------------ L* per node
 // src/operator.cuh:63-82; src/costs.cuh:162-195 (quadratic), :418-458 (quadratic+linear);
 // src/constraints.cuh:171-191 (rectangle), :265-286 (polyhedron).
-// emit(kind, k, value): kind 0 = x (k < nx), 1 = u (k < nu), 2 = y (k < yD), 3 = s, 4 = t; each
-// entry of this lane's instance is emitted by exactly one lane.
-template <typename T, typename E>
-__device__ __forceinline__ void adjNode(LP<T> P, const TV<T> &d, int n, E emit) {
+// The handler gets every entry of this lane's instance in exactly one lane: one(kind, k, value) with kind
+// 2 = y (k < yD), 3 = s, 4 = t, and for blocks of x (kind 0) and u (kind 1) rows, at element e0 of the
+// primal part, load(e0, lo, pre) and then rows(kind, k0, e0, lo, rows, values, pre).
+// A node is a chain of memory round trips (about 2 us each when all CUs are busy), so they are few: the
+// operands of up to 64 columns, the constraint's dual rows and the handler's rows go out together.
+template <int NT, typename T, typename H, typename Terms, typename Extra>
+__device__ __forceinline__ void adjBlock(const TV<T> &d, int kind, int k0, long e0, long ec, bool rect, int rows, Terms &terms,
+                                         Extra &extra, H &h) {
+    const unsigned lo = rowLane<T>();
+    Pre<T, NT> all;
+    T crAll[NT][4];
+    if (EARLY<T>) {
+        h.load(e0, lo, all);
+        if (rect) loadRows(d, ec, lo, crAll);
+    }
+    Acc<T> acc[NT];
+    zeroTiles<T>(acc);
+    terms(acc, k0);
+    eachPart<T, NT>(acc, [&](int t0, auto &a) {
+        constexpr int CH = std::extent_v<std::remove_reference_t<decltype(a)>>;
+        auto finish = [&](auto &pre, auto &cr) {
+            if (rect) {
+#pragma unroll
+                for (int t = 0; t < CH; t++)
+#pragma unroll
+                    for (int q = 0; q < 4; q++) a[t][q] += cr[t][q];
+            }
+            extra(a, k0 + 16 * t0, rows - 16 * t0);
+            h.rows(kind, k0 + 16 * t0, e0 + 16 * t0, lo, rows - 16 * t0, a, pre);
+        };
+        if constexpr (EARLY<T>) {
+            finish(all, crAll);
+        } else if (16 * t0 < rows) {
+            Pre<T, CH> pre;
+            T cr[CH][4];
+            h.load(e0 + 16 * t0, lo, pre);
+            if (rect) loadRows(d, ec + 16 * t0, lo, cr);
+            finish(pre, cr);
+        }
+    });
+}
+
+template <typename T, typename H>
+__device__ __forceinline__ void adjNode(LP<T> P, const TV<T> &d, int n, H &h) {
     const int nx = P.nx, nu = P.nu, nxu = nx + nu, d4 = nxu + 2;
     const bool first = rowGroup() == 0;
+    auto blocks = [&](int kind, long e0, long ec, bool rect, int rows, auto terms, auto extra) {
+#pragma unroll 1
+        for (int r0 = 0; r0 < rows; r0 += 64) {
+            const int rr = min(64, rows - r0);
+            if (rr > 32) adjBlock<4>(d, kind, r0, e0 + r0, ec + r0, rect, rr, terms, extra, h);
+            else if (rr <= 16) adjBlock<1>(d, kind, r0, e0 + r0, ec + r0, rect, rr, terms, extra, h);
+            else adjBlock<2>(d, kind, r0, e0 + r0, ec + r0, rect, rr, terms, extra, h);
+        }
+    };
     if (n < P.nl) {
         const T II = d[P.oII + n];
-        if (first) emit(3, 0, II);
+        if (first) h.one(3, 0, II);
         CP<T> bn = tab(P.b, n);
-        forRows<T>(P.yD, [&](int k) { emit(2, k, d[P.oI + (long) n * P.yD + k] - bn[k] * II); });
+        forRows<T>(P.yD, [&](int k) { h.one(2, k, d[P.oI + (long) n * P.yD + k] - bn[k] * II); });
         const long b3 = P.oIII + (long) n * P.con3;
         const int c0 = cst(P.chFrom)[n], nc = cst(P.numCh)[n];
+#pragma unroll 1
         for (int part = 0; part < 2; part++) {  // x rows, then u rows
             const int rows = part == 0 ? nx : nu;
-            gemv<T>(
-                rows,
+            blocks(
+                part, part == 0 ? P.oX + (long) n * nx : P.oU + (long) n * nu, b3 + part * nx, P.ncon == CON_RECT_DEV, rows,
                 [&](auto &acc, int r0) {
                     if (P.ncon == CON_POLY_DEV)
                         mma<T>(acc, packed(part == 0 ? P.pGTx : P.pGTu, n, r0), P.con3, [&](int cc) { return d[b3 + cc]; });
@@ -338,24 +462,27 @@ __device__ __forceinline__ void adjNode(LP<T> P, const TV<T> &d, int n, E emit) 
                         mma<T>(acc, packed(part == 0 ? P.psQ : P.psR, c0 + ci, r0), rows, [&](int cc) { return d[iv + cc]; });
                     }
                 },
-                [&](int r, T v) {
-                    if (P.ncon == CON_RECT_DEV) v += d[b3 + part * nx + r];
+                [&](auto &acc, int r0, int rr) {
                     if (P.ncost == COST_LIN_DEV) {  // q_j sum_j, r_j sum_j (src/costs.cuh:274-285)
                         for (int ci = 0; ci < nc; ci++) {
                             const int j = c0 + ci;
-                            v += (part == 0 ? tab(P.q, j) : tab(P.r, j))[r] * d[P.oIV + j];
+                            CP<T> qj = (part == 0 ? tab(P.q, j) : tab(P.r, j)) + r0;
+                            const T sj = d[P.oIV + j];
+                            eachOut<std::extent_v<std::remove_reference_t<decltype(acc)>>, T>(acc, rr,
+                                                                                             [&](int r, T &v) { v += qj[r] * sj; });
                         }
-                    }
-                    if (P.ncost == COST_QUADLIN_DEV) {
+                    } else if (P.ncost == COST_QUADLIN_DEV) {
                         for (int ci = 0; ci < nc; ci++) {
                             const int j = c0 + ci;
                             const long iv = P.oIV + (long) j * d4;
                             const T a = d[iv + nxu], bb = d[iv + nxu + 1];
-                            const T qr = (part == 0 ? tab(P.q, j) : tab(P.r, j))[r];
-                            v = v - T(0.5) * qr * a - T(0.5) * qr * bb;
+                            CP<T> qj = (part == 0 ? tab(P.q, j) : tab(P.r, j)) + r0;
+                            eachOut<std::extent_v<std::remove_reference_t<decltype(acc)>>, T>(acc, rr, [&](int r, T &v) {
+                                const T qr = qj[r];
+                                v = v - T(0.5) * qr * a - T(0.5) * qr * bb;
+                            });
                         }
                     }
-                    emit(part, r, v);
                 });
         }
     } else {
@@ -364,43 +491,118 @@ __device__ __forceinline__ void adjNode(LP<T> P, const TV<T> &d, int n, E emit) 
         const bool lin = P.lcost == COST_LIN_DEV;  // block VI = (sum of every leaf; set of every leaf)
         const long vi = P.oVI + (long) l * (lin ? 1 : nx + 2);
         const T a = lin ? T(0) : d[vi + nx], bb = lin ? T(0) : d[vi + nx + 1];
-        gemv<T>(
-            nx,
+        blocks(
+            0, P.oX + (long) n * nx, b5, P.lcon == CON_RECT_DEV, nx,
             [&](auto &acc, int r0) {
                 if (P.lcon == CON_POLY_DEV) mma<T>(acc, packed(P.plGT, l, r0), P.con5, [&](int cc) { return d[b5 + cc]; });
                 if (!lin) mma<T>(acc, packed(P.plsQ, l, r0), nx, [&](int cc) { return d[vi + cc]; });
             },
-            [&](int r, T v) {
-                if (P.lcon == CON_RECT_DEV) v += d[b5 + r];
-                if (lin) v += tab(P.lq, l)[r] * d[vi];  // q sum_l (src/costs.cuh:289-292)
-                if (P.lcost == COST_QUADLIN_DEV) {
-                    const T qr = tab(P.lq, l)[r];
-                    v = v - T(0.5) * qr * a - T(0.5) * qr * bb;
-                }
-                emit(0, r, v);
+            [&](auto &acc, int r0, int rr) {
+                if (!lin && P.lcost != COST_QUADLIN_DEV) return;
+                CP<T> lq = tab(P.lq, l) + r0;
+                const T sl = lin ? d[vi] : T(0);  // q sum_l (src/costs.cuh:289-292)
+                eachOut<std::extent_v<std::remove_reference_t<decltype(acc)>>, T>(acc, rr, [&](int r, T &v) {
+                    const T qr = lq[r];
+                    if (lin) v += qr * sl;
+                    else v = v - T(0.5) * qr * a - T(0.5) * qr * bb;
+                });
             });
-        if (first) emit(3, 0, lin ? d[P.oVI + P.nlf + l] : (a + bb) * T(0.5));
+        if (first) h.one(3, 0, lin ? d[P.oVI + P.nlf + l] : (a + bb) * T(0.5));
     }
     if (first) {
         if (P.ncost == COST_LIN_DEV) {
-            emit(4, 0, d[P.oIV + P.N + n]);  // t <- set, every node (src/costs.cuh:286)
+            h.one(4, 0, d[P.oIV + P.N + n]);  // t <- set, every node (src/costs.cuh:286)
         } else if (n >= 1) {
             const long iv = P.oIV + (long) n * d4;
-            emit(4, 0, (d[iv + nxu] + d[iv + nxu + 1]) * T(0.5));
+            h.one(4, 0, (d[iv + nxu] + d[iv + nxu + 1]) * T(0.5));
         } else {
-            emit(4, 0, T(0));
+            h.one(4, 0, T(0));
         }
     }
 }
 
 // ------------------------------------------------------------------ L per node
 // src/operator.cuh:41-60; src/costs.cuh:126-160, :379-416; src/constraints.cuh:158-169, :251-263.
-// Handler: elemI(n, k, v), elemII(n, v) (row group 0 only), elemBox(e, v, lb, ub) for III and V,
-// and for the SOC blocks IV and VI socBegin(), socPart(e, v, trans) for the owned rows of all but
-// the last two entries, then socEnd(base, n1, n2, h, trans) for a block of n1 + n2 + 2 entries
-// whose last two both carry h.
+// pv(e) is element e of the primal vector, pv.rows(e0, lo, v) the lane's rows of a block.
+// Handler: elemI(n, k, v), elemII(n, v) (row group 0 only), elemBox(e, v, lb, ub) for polyhedral rows;
+// load(e0, lo, pre) and boxRows(e0, lo, rows, v, lb, ub, pre) for the box blocks III and V.  SOC blocks
+// (IV and VI): socBegin(); with up to 64 states socIn(e0, lo, rows, values, pre, trans) for its row tiles,
+// m = socScale(base, dim, h, trans) for its last two entries, which both carry h, and socOut(e0, lo, rows,
+// values, m); with more, socPart(e, v, trans) for the owned rows of all but the last two entries and
+// socEnd(base, n1, n2, h, trans).
+template <int NT, typename T, typename PV, typename H>
+__device__ __forceinline__ void boxTiles(long e0, long eb, int rows, CP<T> lb, CP<T> ub, PV &pv, H &h) {
+    const unsigned lo = rowLane<T>();
+#pragma unroll 1
+    for (int r0 = 0; r0 < rows; r0 += 16 * NT) {
+        Pre<T, NT> pre;
+        T v[NT][4], l[NT][4], u[NT][4];
+        pv.rows(e0 + r0, lo, v);
+        h.load(eb + r0, lo, pre);
+        loadRows(lb + r0, l);
+        loadRows(ub + r0, u);
+        h.boxRows(eb + r0, lo, min(16 * NT, rows - r0), v, l, u, pre);
+    }
+}
+
 template <typename T, typename PV, typename H>
-__device__ __forceinline__ void opNode(LP<T> P, int n, PV pv, H &h) {
+__device__ __forceinline__ void boxRows(long e0, long eb, int rows, CP<T> lb, CP<T> ub, PV &pv, H &h) {
+    if (!EARLY<T> || rows <= 16) boxTiles<1>(e0, eb, rows, lb, ub, pv, h);
+    else boxTiles<2>(e0, eb, rows, lb, ub, pv, h);
+}
+
+template <int NX, int NU, typename T, typename XF, typename UF, typename H>
+__device__ __forceinline__ void socBlock(CP<T> MX, int nx, XF xf, CP<T> MU, int nu, UF uf, long base, T hv, CP<T> tr, H &h) {
+    const unsigned lo = rowLane<T>();
+    Pre<T, NX> px;
+    Pre<T, NU> pu;
+    if (EARLY<T>) {
+        h.load(base, lo, px);
+        if (nu > 0) h.load(base + nx, lo, pu);
+    }
+    Acc<T> ax[NX], au[NU];
+    zeroTiles<T>(ax);
+    zeroTiles<T>(au);
+    mma<T>(ax, MX, nx, xf);
+    if (nu > 0) mma<T>(au, MU, nu, uf);
+    h.socBegin();
+    auto in = [&](auto &acc, int n, long e0, CP<T> trn, auto &all) {
+        constexpr int NT = std::extent_v<std::remove_reference_t<decltype(acc)>>;
+        eachPart<T, NT>(acc, [&](int t0, auto &a) {
+            constexpr int CH = std::extent_v<std::remove_reference_t<decltype(a)>>;
+            if constexpr (EARLY<T>) {
+                h.socIn(e0, lo, n, a, all, trn);
+            } else if (16 * t0 < n) {
+                Pre<T, CH> pre;
+                h.load(e0 + 16 * t0, lo, pre);
+                h.socIn(e0 + 16 * t0, lo, n - 16 * t0, a, pre, trn + 16 * t0);
+            }
+        });
+    };
+    in(ax, nx, base, tr, px);
+    if (nu > 0) in(au, nu, base + nx, tr + nx, pu);
+    const T mult = h.socScale(base, nx + nu + 2, hv, tr);
+    h.socOut(base, lo, nx, ax, mult);
+    if (nu > 0) h.socOut(base + nx, lo, nu, au, mult);
+}
+
+// By the row tiles of the state and input parts (nx <= 64, nu <= 32).
+template <typename T, typename XF, typename UF, typename H>
+__device__ __forceinline__ void socTiles(CP<T> MX, int nx, XF xf, CP<T> MU, int nu, UF uf, long base, T hv, CP<T> tr, H &h) {
+    if (nx <= 16) {
+        if (nu <= 16) socBlock<1, 1, T>(MX, nx, xf, MU, nu, uf, base, hv, tr, h);
+        else socBlock<1, 2, T>(MX, nx, xf, MU, nu, uf, base, hv, tr, h);
+    } else if (nx <= 32) {
+        if (nu <= 16) socBlock<2, 1, T>(MX, nx, xf, MU, nu, uf, base, hv, tr, h);
+        else socBlock<2, 2, T>(MX, nx, xf, MU, nu, uf, base, hv, tr, h);
+    } else {
+        if (nu <= 16) socBlock<4, 1, T>(MX, nx, xf, MU, nu, uf, base, hv, tr, h);
+        else socBlock<4, 2, T>(MX, nx, xf, MU, nu, uf, base, hv, tr, h);
+    }
+}
+
+template <typename T, typename PV, typename H>
+__device__ __forceinline__ void opNode(LP<T> P, int n, PV &pv, H &h) {
     const int nx = P.nx, nu = P.nu, nxu = nx + nu;
     const int g = rowGroup();
     if (n < P.nl) {
@@ -416,8 +618,8 @@ __device__ __forceinline__ void opNode(LP<T> P, int n, PV pv, H &h) {
         const long base = P.oIII + (long) n * P.con3;
         if (P.ncon == CON_RECT_DEV) {
             CP<T> lb = tab(P.nLB, n), ub = tab(P.nUB, n);
-            forRows<T>(nx, [&](int k) { h.elemBox(base + k, pv(P.oX + (long) n * nx + k), lb[k], ub[k]); });
-            forRows<T>(nu, [&](int k) { h.elemBox(base + nx + k, pv(P.oU + (long) n * nu + k), lb[nx + k], ub[nx + k]); });
+            boxRows(P.oX + (long) n * nx, base, nx, lb, ub, pv, h);
+            boxRows(P.oU + (long) n * nu, base + nx, nu, lb + nx, ub + nx, pv, h);
         } else if (P.ncon == CON_POLY_DEV) {
             CP<T> lb = tab(P.nLB, n), ub = tab(P.nUB, n);
             gemv<T>(
@@ -459,20 +661,8 @@ __device__ __forceinline__ void opNode(LP<T> P, int n, PV pv, H &h) {
                 hv = hv + T(-0.5) * pq;
                 hv = hv + T(-0.5) * pr;
             }
-            auto soc = [&](auto &ax) {
-                zeroTiles<T>(ax);
-                Acc<T> au[2];
-                zeroTiles<T>(au);
-                mma<T>(ax, packed(P.psQ, n, 0), nx, xa);
-                mma<T>(au, packed(P.psR, n, 0), nu, ua);
-                h.socRegs(base, ax, nx, au, nu, hv, tr);
-            };
-            if (nx <= 32) {  // the block's entries stay with the wave (nu <= 32)
-                Acc<T> ax[2];
-                soc(ax);
-            } else if (nx <= 64) {
-                Acc<T> ax[4];
-                soc(ax);
+            if (nx <= 64) {  // the block's entries stay in registers
+                socTiles<T>(packed(P.psQ, n, 0), nx, xa, packed(P.psR, n, 0), nu, ua, base, hv, tr, h);
             } else {
                 h.socBegin();
                 gemv<T>(
@@ -494,8 +684,7 @@ __device__ __forceinline__ void opNode(LP<T> P, int n, PV pv, H &h) {
         const int l = n - P.nl;
         const long b5 = P.oV + (long) l * P.con5;
         if (P.lcon == CON_RECT_DEV) {
-            CP<T> lb = tab(P.lLB, l), ub = tab(P.lUB, l);
-            forRows<T>(nx, [&](int k) { h.elemBox(b5 + k, pv(P.oX + (long) n * nx + k), lb[k], ub[k]); });
+            boxRows(P.oX + (long) n * nx, b5, nx, tab(P.lLB, l), tab(P.lUB, l), pv, h);
         } else if (P.lcon == CON_POLY_DEV) {
             CP<T> lb = tab(P.lLB, l), ub = tab(P.lUB, l);
             gemv<T>(
@@ -522,19 +711,12 @@ __device__ __forceinline__ void opNode(LP<T> P, int n, PV pv, H &h) {
             pq = sumG(pq);
             hs = hs + T(-0.5) * pq;
         }
-        auto soc = [&](auto &ax) {
-            zeroTiles<T>(ax);
-            Acc<T> au[2];
-            zeroTiles<T>(au);
-            mma<T>(ax, packed(P.plsQ, l, 0), nx, xl);
-            h.socRegs(base, ax, nx, au, 0, hs, tr);
-        };
-        if (nx <= 32) {
-            Acc<T> ax[2];
-            soc(ax);
+        if (nx <= 16) {
+            socBlock<1, 1, T>(packed(P.plsQ, l, 0), nx, xl, (CP<T>) nullptr, 0, xl, base, hs, tr, h);
+        } else if (nx <= 32) {
+            socBlock<2, 1, T>(packed(P.plsQ, l, 0), nx, xl, (CP<T>) nullptr, 0, xl, base, hs, tr, h);
         } else if (nx <= 64) {
-            Acc<T> ax[4];
-            soc(ax);
+            socBlock<4, 1, T>(packed(P.plsQ, l, 0), nx, xl, (CP<T>) nullptr, 0, xl, base, hs, tr, h);
         } else {
             h.socBegin();
             gemv<T>(
@@ -544,6 +726,30 @@ __device__ __forceinline__ void opNode(LP<T> P, int n, PV pv, H &h) {
         }
     }
 }
+
+// Primal vectors of opNode: 2 xbar - z, and one vector.
+template <typename T>
+struct Reflected {
+    TV<T> cand, z;
+    __device__ __forceinline__ T operator()(long e) const { return cand[e] * T(2) - z[e]; }
+    template <int NT>
+    __device__ __forceinline__ void rows(long e0, unsigned lo, T (&v)[NT][4]) const {
+        T c[NT][4];
+        loadRows(cand, e0, lo, c);
+        loadRows(z, e0, lo, v);
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[t][q] = c[t][q] * T(2) - v[t][q];
+    }
+};
+template <typename T>
+struct Plain {
+    TV<T> y;
+    __device__ __forceinline__ T operator()(long e) const { return y[e]; }
+    template <int NT>
+    __device__ __forceinline__ void rows(long e0, unsigned lo, T (&v)[NT][4]) const { loadRows(y, e0, lo, v); }
+};
 
 // Dual prox of the CP step (src/cache.cuh:770-789): w = (L gamma + z_d)/gamma + c and
 // cand_d = gamma (w - Pi(w)), Pi the masked NNOC (src/risks.cuh:99-106), NNOC (src/cones.cuh:134-137),
@@ -555,7 +761,8 @@ struct Prox {
     LP<T> P;
     TV<T> zd, cd;
     T ss;
-    __device__ __forceinline__ T wOf(T Lv, long e, T tr) const { return (Lv * P.gamma + zd[e]) * P.gammaRecip + tr; }
+    __device__ __forceinline__ T wAt(T Lv, T z, T tr) const { return (Lv * P.gamma + z) * P.gammaRecip + tr; }
+    __device__ __forceinline__ T wOf(T Lv, long e, T tr) const { return wAt(Lv, zd[e], tr); }
     __device__ __forceinline__ void elemI(int n, int k, T v) {
         const long e = P.oI + (long) n * P.yD + k;
         const T w = wOf(v, e, T(0));
@@ -570,6 +777,16 @@ struct Prox {
     __device__ __forceinline__ void elemBox(long e, T v, T lb, T ub) {
         const T w = wOf(v, e, T(0));
         cd[e] = (w - projBox(w, lb, ub)) * P.gamma;
+    }
+    template <int NT>
+    __device__ __forceinline__ void load(long e0, unsigned lo, Pre<T, NT> &p) const { loadRows(zd, e0, lo, p.a); }
+    template <int NT>
+    __device__ __forceinline__ void boxRows(long e0, unsigned lo, int rows, T (&v)[NT][4], T (&lb)[NT][4], T (&ub)[NT][4],
+                                            Pre<T, NT> &p) {
+        eachRow<T, NT>(rows, [&](int t, int q, int) {
+            const T w = wAt(v[t][q], p.a[t][q], T(0));
+            rowAt(cd, e0, lo, t, q) = (w - projBox(w, lb[t][q], ub[t][q])) * P.gamma;
+        });
     }
     __device__ __forceinline__ void socBegin() { ss = T(0); }
     __device__ __forceinline__ void socPart(long e, T v, T tr) {
@@ -599,24 +816,21 @@ struct Prox {
         return mult;
     }
     template <int NT>
-    __device__ __forceinline__ void socRegs(long base, Acc<T> (&ax)[NT], int n1, Acc<T> (&au)[2], int n2, T hv, CP<T> tr) {
-        ss = T(0);
-        StagedOut<T> x(ax, n1);
-        x.template each<true>([&](int r, T v) {
-            const T w = wOf(v, base + r, tr[r]);
+    __device__ __forceinline__ void socIn(long, unsigned, int rows, Acc<T> (&a)[NT], Pre<T, NT> &p, CP<T> tr) {
+        T tx[NT][4];
+        loadRows(tr, tx);
+        eachRow<T, NT>(rows, [&](int t, int q, int) {
+            const T w = wAt(a[t][q], p.a[t][q], tx[t][q]);
+            a[t][q] = w;
             ss += w * w;
-            return w;
         });
-        eachOut<2, T>(au, n2, [&](int r, T &v) {
-            v = wOf(v, base + n1 + r, tr[n1 + r]);
-            ss += v * v;
+    }
+    template <int NT>
+    __device__ __forceinline__ void socOut(long e0, unsigned lo, int rows, Acc<T> (&a)[NT], T mult) {
+        eachRow<T, NT>(rows, [&](int t, int q, int) {
+            const T w = a[t][q];
+            rowAt(cd, e0, lo, t, q) = (w - w * mult) * P.gamma;
         });
-        const T mult = socScale(base, n1 + n2 + 2, hv, tr);
-        x.template each<false>([&](int r, T w) {
-            cd[base + r] = (w - w * mult) * P.gamma;
-            return w;
-        });
-        eachOut<2, T>(au, n2, [&](int r, T &w) { cd[base + n1 + r] = (w - w * mult) * P.gamma; });
     }
     __device__ __forceinline__ void socEnd(long base, int n1, int n2, T hv, CP<T> tr) {
         const T mult = socScale(base, n1 + n2 + 2, hv, tr);
@@ -634,72 +848,6 @@ struct Prox {
     }
 };
 
-// ell(y) = [L* y_d; L y_p] reductions: sum x.(y - gamma ell) and max |y/gamma - ell|
-// (src/cache.cuh:722-734, 917-931), per lane over its own entries.
-template <typename T>
-struct Red {
-    LP<T> P;
-    TV<T> x, y;
-    T dot, mx;
-    __device__ __forceinline__ void acc(long e, T ell) {
-        const T yk = y[e];
-        dot += x[e] * (ell * (-P.gamma) + yk);
-        mx = fmax(mx, fabs(yk * P.gammaRecip - ell));
-    }
-    __device__ __forceinline__ void elemI(int n, int k, T v) { acc(P.sPrim + P.oI + (long) n * P.yD + k, v); }
-    __device__ __forceinline__ void elemII(int n, T v) { acc(P.sPrim + P.oII + n, v); }
-    __device__ __forceinline__ void elemBox(long e, T v, T, T) { acc(P.sPrim + e, v); }
-    __device__ __forceinline__ void socBegin() {}
-    __device__ __forceinline__ void socPart(long e, T v, T) { acc(P.sPrim + e, v); }
-    __device__ __forceinline__ void socEnd(long base, int n1, int n2, T hv, CP<T>) {
-        if (rowGroup() != 0) return;
-        const int dim = n1 + n2 + 2;
-        acc(P.sPrim + base + dim - 2, hv);
-        acc(P.sPrim + base + dim - 1, hv);
-    }
-    template <int NT>
-    __device__ __forceinline__ void socRegs(long base, Acc<T> (&ax)[NT], int n1, Acc<T> (&au)[2], int n2, T hv, CP<T> tr) {
-        StagedOut<T> x(ax, n1);
-        x.template each<false>([&](int r, T v) {
-            acc(P.sPrim + base + r, v);
-            return v;
-        });
-        eachOut<2, T>(au, n2, [&](int r, T v) { acc(P.sPrim + base + n1 + r, v); });
-        socEnd(base, n1, n2, hv, tr);
-    }
-    __device__ __forceinline__ void lin(long eSum, long eSet, T sum, T set) {
-        acc(P.sPrim + eSum, sum);
-        acc(P.sPrim + eSet, set);
-    }
-};
-
-template <typename T>
-struct Store {
-    LP<T> P;
-    TV<T> out;  // dual part
-    __device__ __forceinline__ void elemI(int n, int k, T v) { out[P.oI + (long) n * P.yD + k] = v; }
-    __device__ __forceinline__ void elemII(int n, T v) { out[P.oII + n] = v; }
-    __device__ __forceinline__ void elemBox(long e, T v, T, T) { out[e] = v; }
-    __device__ __forceinline__ void socBegin() {}
-    __device__ __forceinline__ void socPart(long e, T v, T) { out[e] = v; }
-    __device__ __forceinline__ void socEnd(long base, int n1, int n2, T hv, CP<T>) {
-        if (rowGroup() != 0) return;
-        const int dim = n1 + n2 + 2;
-        out[base + dim - 2] = hv;
-        out[base + dim - 1] = hv;
-    }
-    template <int NT>
-    __device__ __forceinline__ void socRegs(long base, Acc<T> (&ax)[NT], int n1, Acc<T> (&au)[2], int n2, T hv, CP<T> tr) {
-        eachOut<NT, T>(ax, n1, [&](int r, T v) { out[base + r] = v; });
-        eachOut<2, T>(au, n2, [&](int r, T v) { out[base + n1 + r] = v; });
-        socEnd(base, n1, n2, hv, tr);
-    }
-    __device__ __forceinline__ void lin(long eSum, long eSet, T sum, T set) {
-        out[eSum] = sum;
-        out[eSet] = set;
-    }
-};
-
 template <typename T>
 __device__ __forceinline__ long primIndex(LP<T> P, int n, int kind, int k) {
     if (kind == 0) return P.oX + (long) n * P.nx + k;
@@ -709,66 +857,216 @@ __device__ __forceinline__ long primIndex(LP<T> P, int n, int kind, int k) {
     return P.oT + n;
 }
 
+// ell(y) = [L* y_d; L y_p] reductions: sum x.(y - gamma ell) and max |y/gamma - ell|
+// (src/cache.cuh:722-734, 917-931), per lane over its own entries; elements are counted from the
+// iterate's start in adjNode and from its dual part in opNode.
+template <typename T>
+struct Red {
+    LP<T> P;
+    TV<T> x, y;
+    T dot, mx;
+    long off;  // of the elements the handler is given
+    T cross;   // adjoint part: sum of x_p . (L* y_d)
+    int n;
+    __device__ __forceinline__ void accV(T xk, T yk, T ell) {
+        dot += xk * (ell * (-P.gamma) + yk);
+        mx = fmax(mx, fabs(yk * P.gammaRecip - ell));
+    }
+    __device__ __forceinline__ void acc(long e, T ell) { accV(x[e], y[e], ell); }
+    template <int NT>
+    __device__ __forceinline__ void load(long e0, unsigned lo, Pre<T, NT> &p) const {
+        loadRows(x, off + e0, lo, p.a);
+        loadRows(y, off + e0, lo, p.b);
+    }
+    // adjoint
+    __device__ __forceinline__ void one(int kind, int k, T v) {
+        const long e = primIndex(P, n, kind, k);
+        cross += x[e] * v;
+        acc(e, v);
+    }
+    template <int NT>
+    __device__ __forceinline__ void rows(int, int, long, unsigned, int rows, Acc<T> (&a)[NT], Pre<T, NT> &p) {
+        eachRow<T, NT>(rows, [&](int t, int q, int) {
+            cross += p.a[t][q] * a[t][q];
+            accV(p.a[t][q], p.b[t][q], a[t][q]);
+        });
+    }
+    // operator
+    __device__ __forceinline__ void elemI(int n, int k, T v) { acc(off + P.oI + (long) n * P.yD + k, v); }
+    __device__ __forceinline__ void elemII(int n, T v) { acc(off + P.oII + n, v); }
+    __device__ __forceinline__ void elemBox(long e, T v, T, T) { acc(off + e, v); }
+    template <int NT>
+    __device__ __forceinline__ void boxRows(long, unsigned, int rows, T (&v)[NT][4], T (&)[NT][4], T (&)[NT][4], Pre<T, NT> &p) {
+        eachRow<T, NT>(rows, [&](int t, int q, int) { accV(p.a[t][q], p.b[t][q], v[t][q]); });
+    }
+    __device__ __forceinline__ void socBegin() {}
+    __device__ __forceinline__ void socPart(long e, T v, T) { acc(off + e, v); }
+    template <int NT>
+    __device__ __forceinline__ void socIn(long, unsigned, int rows, Acc<T> (&a)[NT], Pre<T, NT> &p, CP<T>) {
+        eachRow<T, NT>(rows, [&](int t, int q, int) { accV(p.a[t][q], p.b[t][q], a[t][q]); });
+    }
+    template <int NT>
+    __device__ __forceinline__ void socOut(long, unsigned, int, Acc<T> (&)[NT], T) {}
+    __device__ __forceinline__ T socScale(long base, int dim, T hv, CP<T> tr) {
+        socEnd(base, dim - 2, 0, hv, tr);
+        return T(0);
+    }
+    __device__ __forceinline__ void socEnd(long base, int n1, int n2, T hv, CP<T>) {
+        if (rowGroup() != 0) return;
+        const int dim = n1 + n2 + 2;
+        acc(off + base + dim - 2, hv);
+        acc(off + base + dim - 1, hv);
+    }
+    __device__ __forceinline__ void lin(long eSum, long eSet, T sum, T set) {
+        acc(off + eSum, sum);
+        acc(off + eSet, set);
+    }
+};
+
+// Raw values of L (opNode) and L* (adjNode) into `out` (its dual or primal part).
+template <typename T>
+struct Store {
+    LP<T> P;
+    TV<T> out;
+    int n;
+    template <int NT>
+    __device__ __forceinline__ void load(long, unsigned, Pre<T, NT> &) const {}
+    __device__ __forceinline__ void one(int kind, int k, T v) { out[primIndex(P, n, kind, k)] = v; }
+    template <int NT>
+    __device__ __forceinline__ void rows(int, int, long e0, unsigned lo, int rows, Acc<T> (&a)[NT], Pre<T, NT> &) {
+        eachRow<T, NT>(rows, [&](int t, int q, int) { rowAt(out, e0, lo, t, q) = a[t][q]; });
+    }
+    __device__ __forceinline__ void elemI(int n, int k, T v) { out[P.oI + (long) n * P.yD + k] = v; }
+    __device__ __forceinline__ void elemII(int n, T v) { out[P.oII + n] = v; }
+    __device__ __forceinline__ void elemBox(long e, T v, T, T) { out[e] = v; }
+    template <int NT>
+    __device__ __forceinline__ void boxRows(long e0, unsigned lo, int rows, T (&v)[NT][4], T (&)[NT][4], T (&)[NT][4], Pre<T, NT> &) {
+        eachRow<T, NT>(rows, [&](int t, int q, int) { rowAt(out, e0, lo, t, q) = v[t][q]; });
+    }
+    __device__ __forceinline__ void socBegin() {}
+    __device__ __forceinline__ void socPart(long e, T v, T) { out[e] = v; }
+    template <int NT>
+    __device__ __forceinline__ void socIn(long e0, unsigned lo, int rows, Acc<T> (&a)[NT], Pre<T, NT> &, CP<T>) {
+        eachRow<T, NT>(rows, [&](int t, int q, int) { rowAt(out, e0, lo, t, q) = a[t][q]; });
+    }
+    template <int NT>
+    __device__ __forceinline__ void socOut(long, unsigned, int, Acc<T> (&)[NT], T) {}
+    __device__ __forceinline__ T socScale(long base, int dim, T hv, CP<T> tr) {
+        socEnd(base, dim - 2, 0, hv, tr);
+        return T(0);
+    }
+    __device__ __forceinline__ void socEnd(long base, int n1, int n2, T hv, CP<T>) {
+        if (rowGroup() != 0) return;
+        const int dim = n1 + n2 + 2;
+        out[base + dim - 2] = hv;
+        out[base + dim - 1] = hv;
+    }
+    __device__ __forceinline__ void lin(long eSum, long eSet, T sum, T set) {
+        out[eSum] = sum;
+        out[eSet] = set;
+    }
+};
+
 // ------------------------------------------------------------------ T phases
 // modifyPrimal + proxRootS (src/cache.cuh:748-753, 639-642); leaves seed q = -xbar (src/dynamics.cuh:79-81).
 template <typename T>
+struct Axpy {
+    LP<T> P;
+    TV<T> z, cand, qd;
+    int n;
+    template <int NT>
+    __device__ __forceinline__ void load(long e0, unsigned lo, Pre<T, NT> &p) const { loadRows(z, e0, lo, p.a); }
+    __device__ __forceinline__ void one(int kind, int k, T v) {
+        const long e = primIndex(P, n, kind, k);
+        T val = v * (-P.gamma) + z[e];
+        if (kind == 3 && n == 0) val -= P.gamma;
+        cand[e] = val;
+    }
+    template <int NT>
+    __device__ __forceinline__ void rows(int, int k0, long e0, unsigned lo, int rows, Acc<T> (&a)[NT], Pre<T, NT> &p) {
+        const bool leaf = n >= P.nl;
+        eachRow<T, NT>(rows, [&](int t, int q, int) {
+            const T val = a[t][q] * (-P.gamma) + p.a[t][q];
+            rowAt(cand, e0, lo, t, q) = val;
+            if (leaf) rowAt(qd, (long) n * P.nx + k0, lo, t, q) = -val;
+        });
+    }
+};
+
+template <typename T>
 __device__ __forceinline__ void phaseAdj(LP<T> P, const Ctx &c, const TV<T> &z, const TV<T> &cand,
                                          const TV<T> &qd) {
-    const T g = -P.gamma;
     const TV<T> zd = z.shift(P.sPrim);
     for (int n = c.wave; n < P.N; n += c.nw) {
-        adjNode(P, zd, n, [&](int kind, int k, T v) {
-            const long e = primIndex(P, n, kind, k);
-            T val = v * g + z[e];
-            if (kind == 3 && n == 0) val -= P.gamma;
-            cand[e] = val;
-            if (kind == 0 && n >= P.nl) qd[(long) n * P.nx + k] = -val;
-        });
+        Axpy<T> h{P, z, cand, qd, n};
+        adjNode(P, zd, n, h);
     }
 }
 
 // Backward sweep step for node i (src/dynamics.cuh:85-139) with R~^-1 applied as one product.
-// stg: this wave's two LDS slices of 32 rows x 16 instances.
-template <typename T>
+// stg: this wave's two LDS slices of 32 rows x 16 instances.  NU: row tiles of the inputs (nu <= 32).
+template <int NT, typename T, typename Terms>
+__device__ __forceinline__ void dynBackRows(const TV<T> &cand, const TV<T> &qd, long ex, long eq, int r0, int rows, Terms &terms) {
+    const unsigned lo = rowLane<T>();
+    T xb[NT][4];
+    if (EARLY<T>) loadRows(cand, ex + r0, lo, xb);
+    Acc<T> acc[NT];
+    zeroTiles<T>(acc);
+    terms(acc, r0);
+    if (!EARLY<T>) loadRows(cand, ex + r0, lo, xb);
+    eachRow<T, NT>(rows, [&](int t, int q, int) { rowAt(qd, eq + r0, lo, t, q) = acc[t][q] - xb[t][q]; });
+}
+
+template <int NU, typename T>
 __device__ __forceinline__ void dynBackward(LP<T> P, const TV<T> &cand, const TV<T> &qd, const TV<T> &dd, int i,
                                             int stage, SP<T> stg) {
-    const int nx = P.nx, nu = P.nu;  // nu <= 32 (checked on the host)
+    const int nx = P.nx, nu = P.nu;
     const int c0 = cst(P.chFrom)[i], nc = cst(P.numCh)[i];
-    const int jj = instLane();
+    const int jj = instLane(), g = rowGroup();
+    const unsigned lo = rowLane<T>();
     SP<T> e1 = stg, d1 = stg + STG;
+    const long ub0 = P.oU + (long) i * nu;
+    T ub[NU][4];
+    loadRows(cand, ub0, lo, ub);
     // affine dynamics: the children's q enter as q_j + P_j e_j (src/dynamics.cuh:93-97)
     const bool affine = P.affine != 0;
     auto qv = [&](int j, int cc) { return affine ? qd[(long) j * nx + cc] + tab(P.Pe, j)[cc] : qd[(long) j * nx + cc]; };
     // e = ubar - sum_j B_j' q_j
-    gemv32<T>(
-        nu,
-        [&](auto &acc, int r0) {
-            for (int ci = 0; ci < nc; ci++) mma<T>(acc, packed(P.pBTr, c0 + ci, r0), nx, [&](int cc) { return qv(c0 + ci, cc); });
-        },
-        [&](int r, T v) { e1[r * W + jj] = -v + cand[P.oU + (long) i * nu + r]; });
+    Acc<T> au[NU];
+    zeroTiles<T>(au);
+#pragma unroll 1
+    for (int ci = 0; ci < nc; ci++) mma<T>(au, packed(P.pBTr, c0 + ci, 0), nx, [&](int cc) { return qv(c0 + ci, cc); });
+    eachRow<T, NU>(nu, [&](int t, int q, int r) { e1[r * W + jj] = -au[t][q] + ub[t][q]; });
     __builtin_amdgcn_wave_barrier();
     // d = R~^-1 e
-    gemv32<T>(
-        nu,
-        [&](auto &acc, int r0) { mma<T>(acc, packed(P.pRtInv, i, r0), nu, [&](int cc) -> T { return e1[cc * W + jj]; }); },
-        [&](int r, T v) {
-            dd[(long) i * nu + r] = v;
-            d1[r * W + jj] = v;
-        });
+    zeroTiles<T>(au);
+    mma<T>(au, packed(P.pRtInv, i, 0), nu, [&](int cc) -> T { return e1[cc * W + jj]; });
+    __builtin_amdgcn_wave_barrier();
+    eachRow<T, NU>(nu, [&](int t, int q, int r) {
+        rowAt(dd, (long) i * nu, lo, t, q) = au[t][q];
+        d1[r * W + jj] = au[t][q];
+        e1[r * W + jj] = au[t][q] - ub[t][q];
+    });
     __builtin_amdgcn_wave_barrier();
     if (stage == 0) return;
     // q_i = sum_j (APB_j d_i + ABKTr_j q_j) + K_i'(d_i - u_i) - x_i
-    gemv<T>(
-        nx,
-        [&](auto &acc, int r0) {
-            for (int ci = 0; ci < nc; ci++) {
-                const int j = c0 + ci;
-                mma<T>(acc, packed(P.pAPB, j, r0), nu, [&](int cc) -> T { return d1[cc * W + jj]; });
-                mma<T>(acc, packed(P.pABKTr, j, r0), nx, [&](int cc) { return qv(j, cc); });
-            }
-            mma<T>(acc, packed(P.pKTr, i, r0), nu, [&](int cc) -> T { return d1[cc * W + jj] - cand[P.oU + (long) i * nu + cc]; });
-        },
-        [&](int r, T v) { qd[(long) i * nx + r] = v - cand[P.oX + (long) i * nx + r]; });
+    auto terms = [&](auto &acc, int r0) {
+#pragma unroll 1
+        for (int ci = 0; ci < nc; ci++) {
+            const int j = c0 + ci;
+            mma<T>(acc, packed(P.pAPB, j, r0), nu, [&](int cc) -> T { return d1[cc * W + jj]; });
+            mma<T>(acc, packed(P.pABKTr, j, r0), nx, [&](int cc) { return qv(j, cc); });
+        }
+        mma<T>(acc, packed(P.pKTr, i, r0), nu, [&](int cc) -> T { return e1[cc * W + jj]; });
+    };
+    const long ex = P.oX + (long) i * nx, eq = (long) i * nx;
+#pragma unroll 1
+    for (int r0 = 0; r0 < nx; r0 += 64) {
+        const int rr = min(64, nx - r0);
+        if (rr > 32) dynBackRows<4>(cand, qd, ex, eq, r0, rr, terms);
+        else if (rr <= 16) dynBackRows<1>(cand, qd, ex, eq, r0, rr, terms);
+        else dynBackRows<2>(cand, qd, ex, eq, r0, rr, terms);
+    }
 }
 
 // Kernel projection for nonleaf node i (src/cache.cuh:650-676); padded child slots enter as 0.
@@ -794,26 +1092,32 @@ __device__ __forceinline__ void kernelProj(LP<T> P, const TV<T> &cand, int i) {
 }
 
 // Forward rollout for node i (src/dynamics.cuh:144-173); affine dynamics add e_j to each child.
-template <typename T>
+template <int NU, typename T>
 __device__ __forceinline__ void dynForward(LP<T> P, const TV<T> &cand, const TV<T> &x0s, const TV<T> &dd, int i,
                                            SP<T> stg) {
     const int nx = P.nx, nu = P.nu;
     const int jj = instLane();
+    const unsigned lo = rowLane<T>();
     SP<T> u1 = stg;
+    T db[NU][4];
+    loadRows(dd, (long) i * nu, lo, db);
     // x_0 is the (scaled) initial state; other nodes' x were written by their parent's step
     auto xv = [&](int cc) { return i == 0 ? x0s[cc] : cand[P.oX + (long) i * nx + cc]; };
     if (i == 0) forRows<T>(nx, [&](int r) { cand[P.oX + r] = x0s[r]; });
-    gemv32<T>(
-        nu, [&](auto &acc, int r0) { mma<T>(acc, packed(P.pK, i, r0), nx, xv); },
-        [&](int r, T v) {
-            const T u = v + dd[(long) i * nu + r];
-            cand[P.oU + (long) i * nu + r] = u;
-            u1[r * W + jj] = u;
-        });
+    Acc<T> au[NU];
+    zeroTiles<T>(au);
+    mma<T>(au, packed(P.pK, i, 0), nx, xv);
+    eachRow<T, NU>(nu, [&](int t, int q, int r) {
+        const T u = au[t][q] + db[t][q];
+        rowAt(cand, P.oU + (long) i * nu, lo, t, q) = u;
+        u1[r * W + jj] = u;
+    });
     __builtin_amdgcn_wave_barrier();
     const int c0 = cst(P.chFrom)[i], nc = cst(P.numCh)[i];
+#pragma unroll 1
     for (int ci = 0; ci < nc; ci++) {
         const int j = c0 + ci;
+        const long ex = P.oX + (long) j * nx;
         gemv<T, false>(  // u1 stays in the LDS slice for the next child
             nx,
             [&](auto &acc, int r0) {
@@ -821,28 +1125,28 @@ __device__ __forceinline__ void dynForward(LP<T> P, const TV<T> &cand, const TV<
             },
             [&](int r, T v) {
                 if (P.affine) v += tab(P.e, j)[r];
-                cand[P.oX + (long) j * nx + r] = v;
+                cand[ex + r] = v;
             });
     }
     __builtin_amdgcn_wave_barrier();
 }
 
-template <typename T>
-__device__ __forceinline__ void phaseProj(LP<T> P, const Ctx &c, const TV<T> &cand, const TV<T> &qd, const TV<T> &dd,
-                                          const TV<T> &x0s, bool doDyn, bool doKernel, SP<T> stg) {
+template <int NU, typename T>
+__device__ __forceinline__ void phaseProjTiles(LP<T> P, const Ctx &c, const TV<T> &cand, const TV<T> &qd, const TV<T> &dd,
+                                               const TV<T> &x0s, bool doDyn, bool doKernel, SP<T> stg) {
     if (doDyn) {
         for (int stage = P.S - 2; stage >= 0; stage--) {
             const int f = cst(P.stageFrom)[stage], nStage = cst(P.stageTo)[stage] - f + 1;
             const int extra = (doKernel && stage == P.S - 2) ? P.nl : 0;
             for (int task = c.wave; task < nStage + extra; task += c.nw) {
-                if (task < nStage) dynBackward(P, cand, qd, dd, f + task, stage, stg);
+                if (task < nStage) dynBackward<NU>(P, cand, qd, dd, f + task, stage, stg);
                 else kernelProj(P, cand, task - nStage);
             }
             __syncthreads();
         }
         for (int stage = 0; stage <= P.S - 2; stage++) {
             const int f = cst(P.stageFrom)[stage], nStage = cst(P.stageTo)[stage] - f + 1;
-            for (int task = c.wave; task < nStage; task += c.nw) dynForward(P, cand, x0s, dd, f + task, stg);
+            for (int task = c.wave; task < nStage; task += c.nw) dynForward<NU>(P, cand, x0s, dd, f + task, stg);
             __syncthreads();
         }
     } else if (doKernel) {
@@ -851,11 +1155,18 @@ __device__ __forceinline__ void phaseProj(LP<T> P, const Ctx &c, const TV<T> &ca
     }
 }
 
+template <typename T>
+__device__ __forceinline__ void phaseProj(LP<T> P, const Ctx &c, const TV<T> &cand, const TV<T> &qd, const TV<T> &dd,
+                                          const TV<T> &x0s, bool doDyn, bool doKernel, SP<T> stg) {
+    if (P.nu <= 16) phaseProjTiles<1>(P, c, cand, qd, dd, x0s, doDyn, doKernel, stg);
+    else phaseProjTiles<2>(P, c, cand, qd, dd, x0s, doDyn, doKernel, stg);  // nu <= 32 (checked on the host)
+}
+
 // modifyDual + proximalDual (src/cache.cuh:770-789) on 2 xbar - z_p.
 template <typename T>
 __device__ __forceinline__ void phaseDual(LP<T> P, const Ctx &c, const TV<T> &z, const TV<T> &cand) {
     Prox<T> h{P, z.shift(P.sPrim), cand.shift(P.sPrim), T(0)};
-    auto pv = [&](long e) { return cand[e] * T(2) - z[e]; };
+    Reflected<T> pv{cand, z};
     for (int n = c.wave; n < P.N; n += c.nw) opNode(P, n, pv, h);
 }
 
@@ -910,26 +1221,48 @@ __device__ __noinline__ DotMax<T> reduceEll(const LaneInst<T> *Pp, T *x, T *y, d
     const Ctx c = ctx();
     const TV<T> xv = tview(x, P.sIter, c.j), yv = tview(y, P.sIter, c.j);
     const TV<T> yd = yv.shift(P.sPrim);
-    Red<T> h{P, xv, yv, T(0), T(0)};
-    T dot = T(0), mx = T(0);
-    T cross = T(0);
-    auto pv = [&](long e) { return yv[e]; };
+    Red<T> h{P, xv, yv, T(0), T(0), 0, T(0), 0};
+    Plain<T> pv{yv};
     for (int n = c.wave; n < P.N; n += c.nw) {
-        adjNode(P, yd, n, [&](int kind, int k, T v) {
-            const long e = primIndex(P, n, kind, k);
-            const T yk = yv[e], xk = xv[e];
-            dot += xk * (v * (-P.gamma) + yk);
-            cross += xk * v;
-            mx = fmax(mx, fabs(yk * P.gammaRecip - v));
-        });
+        h.n = n;
+        h.off = 0;
+        adjNode(P, yd, n, h);
+        h.off = P.sPrim;
         opNode(P, n, pv, h);
     }
     DotMax<T> r;
-    r.dot = (T) tileSum((double) (dot + h.dot), lds, c);
-    r.mx = (T) tileMax((double) fmax(mx, h.mx), lds, c);
-    r.cross = (T) tileSum((double) cross, lds, c);
+    r.dot = (T) tileSum((double) h.dot, lds, c);
+    r.mx = (T) tileMax((double) h.mx, lds, c);
+    r.cross = (T) tileSum((double) h.cross, lds, c);
     return r;
 }
+
+// c1 += x_p . (adjoint), c2 += (adjoint) . y_p.
+template <typename T>
+struct Dots {
+    LP<T> P;
+    TV<T> x, y;
+    bool withY;
+    int n;
+    T c1, c2;
+    template <int NT>
+    __device__ __forceinline__ void load(long e0, unsigned lo, Pre<T, NT> &p) const {
+        loadRows(x, e0, lo, p.a);
+        if (withY) loadRows(y, e0, lo, p.b);
+    }
+    __device__ __forceinline__ void one(int kind, int k, T v) {
+        const long e = primIndex(P, n, kind, k);
+        c1 += x[e] * v;
+        if (withY) c2 += v * y[e];
+    }
+    template <int NT>
+    __device__ __forceinline__ void rows(int, int, long, unsigned, int rows, Acc<T> (&a)[NT], Pre<T, NT> &p) {
+        eachRow<T, NT>(rows, [&](int t, int q, int) {
+            c1 += p.a[t][q] * a[t][q];
+            if (withY) c2 += a[t][q] * p.b[t][q];
+        });
+    }
+};
 
 // c1 = sum_p x_p . (L* x_d),  c2 = sum_p x_p . (L* y_d) + (L* x_d) . y_p (see the lane engine).
 template <typename T>
@@ -942,12 +1275,15 @@ __device__ __noinline__ Cross2<T> adjDots(const LaneInst<T> *Pp, T *x, T *y, dou
     const TV<T> xd = xv.shift(P.sPrim), yd = yv.shift(P.sPrim);
     T c1 = T(0), c2 = T(0);
     for (int n = c.wave; n < P.N; n += c.nw) {
-        adjNode(P, xd, n, [&](int kind, int k, T v) {
-            const long e = primIndex(P, n, kind, k);
-            c1 += xv[e] * v;
-            if (withY) c2 += v * yv[e];
-        });
-        if (withY) adjNode(P, yd, n, [&](int kind, int k, T v) { c2 += xv[primIndex(P, n, kind, k)] * v; });
+        Dots<T> h{P, xv, yv, withY, n, c1, c2};
+        adjNode(P, xd, n, h);
+        c1 = h.c1;
+        c2 = h.c2;
+        if (withY) {
+            Dots<T> hy{P, xv, yv, false, n, c2, T(0)};
+            adjNode(P, yd, n, hy);
+            c2 = hy.c1;
+        }
     }
     Cross2<T> r;
     r.c1 = (T) tileSum((double) c1, lds, c);
@@ -1018,13 +1354,15 @@ __global__ void __launch_bounds__(SPK_TILE_MAX_THREADS) SPK_TILE_KERNEL(k_tile_d
     T *z = P.zio, *cand = P.work[1];
     const TV<T> zv = tview(z, P.sIter, c.j), cv = tview(cand, P.sIter, c.j);
     if (op == 0) {  // L
-        Store<T> h{P, cv.shift(P.sPrim)};
-        auto pv = [&](long e) { return zv[e]; };
+        Store<T> h{P, cv.shift(P.sPrim), 0};
+        Plain<T> pv{zv};
         for (int n = c.wave; n < P.N; n += c.nw) opNode(P, n, pv, h);
     } else if (op == 1) {  // L*
         const TV<T> zd = zv.shift(P.sPrim);
-        for (int n = c.wave; n < P.N; n += c.nw)
-            adjNode(P, zd, n, [&](int kind, int k, T v) { cv[primIndex(P, n, kind, k)] = v; });
+        for (int n = c.wave; n < P.N; n += c.nw) {
+            Store<T> h{P, cv, n};
+            adjNode(P, zd, n, h);
+        }
     } else if (op == 2 || op == 3) {  // dynamics / kernel projection of the primal part
         tile::pass<16>(P.sPrim, c, [&](long e) { return zv[e]; }, [&](long e, T v) { cv[e] = v; });
         __syncthreads();
