@@ -1003,6 +1003,13 @@ void gatherLanes(spk_batch *b, int count, T *dst, long ld) {
 
 }  // namespace
 
+float *spk::laneIterates(spk_batch *b, const spk_ctx *c, long n) {
+    if (!b->lanes || b->dtype != SPK_F32 || b->laneW != 16 || b->ctx != c || (long) b->probs[0]->hp.sIter != n) return nullptr;
+    check(hipSetDevice(c->device), "hipSetDevice");
+    fillDevice<float>(b, lanePtr<float>(b, LR_RIO), (size_t) n * b->Bpad);
+    return lanePtr<float>(b, LR_ZIO);
+}
+
 extern "C" {
 
 void spk_default_options(spk_options *o) {

@@ -71,4 +71,8 @@ inline int fail(spk_ctx *ctx, const std::exception &e) {
     return dynamic_cast<const CoopRefused *>(&e) ? -2 : -1;
 }
 
+// For a writer of all of a batch's iterates on context c's stream: where a shared FP32 batch of c holds them
+// (16 instances to a block, instance fastest) if an iterate has n words, its residuals cleared; else null.
+float *laneIterates(spk_batch *b, const spk_ctx *c, long n);
+
 }  // namespace spk
