@@ -139,6 +139,7 @@ struct spk_batch {
     DevBuf core, anders, x0buf, dInst, dOut;  // x0buf: scaled initial states (inputs, kept by reset)
     int wgs = 0;    // workgroups per instance (0 or 1: one; see gridWorkgroups)
     DevBuf gpart;   // grid-mode reduction partials (single-instance batches)
+    DevBuf gbar;    // grid-mode barrier (single-instance batches)
     std::vector<char> hInst;  // array of Inst<T>
     std::vector<double> tolFixed;  // per-instance given tolerance (0 = calibrate at the first check)
     // shared-problem batch in the instance-interleaved layout (lane engine)
@@ -394,6 +395,7 @@ void fillInsts(spk_batch *b, const spk_options &o, int warm, T *anders, const st
         I.dynInverse = o.dyn_inverse;
         I.maxTicks = o.max_time_secs > 0 ? o.max_time_secs * b->ctx->tickRateHz : 0.;
         I.gpart = gpart;
+        I.gbar = static_cast<unsigned *>(b->gbar.p);
         I.slot = k;
         if (b->dbgCap > 0) {
             I.dbg = static_cast<double *>(b->dbgRec.p) + (size_t) k * b->dbgCap * spk::DBG_WORDS;
@@ -1132,6 +1134,10 @@ int spk_batch_create(spk_ctx *ctx, int count, spk_problem *const *problems, int 
             off += coreCount(b->probs[k]->hp);
         }
         b->coreElems = off;
+        if (count == 1) {
+            b->gbar.alloc(spk::GRID_BAR_WORDS * sizeof(unsigned));
+            check(hipMemsetAsync(b->gbar.p, 0, spk::GRID_BAR_WORDS * sizeof(unsigned), ctx->stream), "zero barrier");
+        }
         b->core.alloc(off * b->elSize());
         check(hipMemsetAsync(b->core.p, 0, off * b->elSize(), ctx->stream), "zero state");
         b->x0Off.resize(count);

@@ -77,6 +77,7 @@ struct Inst {
     int maxInner, andBuff, checkPeriod, method, warm, lsMethod, dynInverse;
     double maxTicks;  // wall-clock cap in device ticks (0 = none)
     T *gpart;         // grid mode: 2 x GRID_MAXK x GRID_MAXWG reduction partials
+    unsigned *gbar;   // grid mode: the barrier's GRID_BAR_WORDS words, zero before the first launch
     // debug trace (enableDebug, src/cache.cuh:947-959); dbg == nullptr: off.  One record of
     // DBG_WORDS doubles per error check, at most dbgCap; dbgE (sPrim) carries err0's running
     // vector from check to check and from solve to solve
@@ -92,6 +93,11 @@ constexpr int DBG_WORDS = 6;
 // Grid mode limits: values per grid reduction and workgroups per cooperative launch.
 constexpr int GRID_MAXK = 16;
 constexpr int GRID_MAXWG = 1024;
+// The grid barrier: a counter for each of up to GRID_GROUPS groups of workgroups, one for the groups and a
+// release flag for each group, every one in a 256-byte piece of its own.
+constexpr int GRID_GROUPS = 8;
+constexpr int GRID_BAR_STEP = 64;
+constexpr int GRID_BAR_WORDS = GRID_BAR_STEP * (2 * GRID_GROUPS + 1);
 
 // Block-interleaved layout of a region of `rows` rows: instances are grouped in blocks of w (64
 // for the lane engine, 16 for the tile engine) and each block stores rows x w words contiguously,
