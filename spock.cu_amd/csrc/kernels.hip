@@ -950,15 +950,16 @@ __device__ __forceinline__ void kernelNode(IP<T> P, GP<T> cand, int i, unsigned 
     if (any) cand[at] = w[0];
 }
 
-// Forward rollout for node i (src/dynamics.cuh:144-173); affine dynamics add e_j to each child.
+// Forward rollout for node i (src/dynamics.cuh:144-173); affine dynamics add e_j to each child.  Member m of a
+// team of g waves takes every g-th child; u is computed by all of them.
 template <typename T, int R, int V>
-__device__ __forceinline__ void dynForwardNode(IP<T> P, GP<T> cand, int i, unsigned row) {
+__device__ __forceinline__ void dynForwardNode(IP<T> P, GP<T> cand, int i, unsigned row, int m = 0, int g = 1) {
     const int nx = P.nx, nu = P.nu;
     T xv[V], uv[V], w[R];
     GP<T> xi = cand + (P.oX + (long) i * nx);
     if (i == 0) {
         loadPtr(xv, cst(P.x0s), nx, row);
-        eachRow<V>(nx, row, [&](int c, unsigned k) { xi[k] = xv[c]; });
+        if (m == 0) eachRow<V>(nx, row, [&](int c, unsigned k) { xi[k] = xv[c]; });
     } else {
         loadPtr(xv, xi, nx, row);
     }
@@ -967,12 +968,12 @@ __device__ __forceinline__ void dynForwardNode(IP<T> P, GP<T> cand, int i, unsig
     zero(w);
     mvAcc(w, tab(P.K, i), nu, nu, nx, xv);
     const T u = mine ? w[0] + di : T(0);
-    if (mine) (cand + (P.oU + (long) i * nu))[row] = u;
+    if (m == 0 && mine) (cand + (P.oU + (long) i * nu))[row] = u;
     zero(uv);
     uv[0] = u;
     const int c0 = cst(P.chFrom)[i], nc = cst(P.numCh)[i];
 #pragma unroll 1
-    for (int ci = 0; ci < nc; ci++) {
+    for (int ci = m; ci < nc; ci += g) {
         const int j = c0 + ci;
         CP<T> AB = tab(P.AB, j);
         zero(w);
@@ -984,6 +985,135 @@ __device__ __forceinline__ void dynForwardNode(IP<T> P, GP<T> cand, int i, unsig
     }
 }
 
+// Stages with fewer nodes than half the waves (near the root, and all of them when a tree is spread over
+// the device) give each node to a team of waves of one workgroup: a node's products are a chain of trips to memory,
+// and a team takes its children side by side.  Team size: the largest power of two that fits the waves (and the
+// slots below), or 1.  Projections of one T: 341 nodes, nx = 100, 4 children, FP64, 128 workgroups 253 -> 121 us;
+// 1,365 nodes FP32, 256 workgroups 254 -> 138; 229 nodes, 9 of 11 stages without branching, 32 workgroups 167 -> 131.
+template <int R>
+constexpr int TEAM_ROUNDS = R == 1 ? 2 : 1;  // children of a member; wider nodes need fewer and keep LDS small
+
+template <typename T, int R>
+struct TeamLds {
+    T bq[8][TEAM_ROUNDS<R>][64];      // B'q of a member's children
+    T xq[8][TEAM_ROUNDS<R>][64 * R];  // their parts of q
+};
+
+template <int R>
+__device__ __forceinline__ int teamSize(const Tc &c, int nodes, int children) {
+    int g = 1;
+    while (2 * g <= c.lnw && c.lnw % (2 * g) == 0 && nodes * 2 * g <= c.nw) g *= 2;
+    return children <= TEAM_ROUNDS<R> * g ? g : 1;
+}
+
+// dynBackwardNode by member m of a team of g waves whose first is wave w0 of the workgroup: the same sums in the
+// same order.  With waves to spare (2 nc <= g) member nc + c takes the product with q of child c.  All waves
+// of the workgroup come here together; i < 0: no node.
+template <typename T, int R, int V>
+__device__ __forceinline__ void dynBackwardTeam(IP<T> P, GP<T> cand, int i, int stage, unsigned row, int m, int g, int w0,
+                                                SPK_LDS TeamLds<T, R> *lds) {
+    constexpr int K = TEAM_ROUNDS<R>;
+    const int nx = P.nx, nu = P.nu;
+    const bool mine = row < (unsigned) nu;
+    const int c0 = i < 0 ? 0 : cst(P.chFrom)[i], nc = i < 0 ? 0 : cst(P.numCh)[i];
+    const bool split = 2 * nc <= g;
+    GP<T> qd = (GP<T>) P.qd;
+    T rq[K][R], w[R];
+    const T ub = i >= 0 && mine ? (cand + (P.oU + (long) i * nu))[row] : T(0);
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        zero(rq[k]);
+        const int ci = split && m >= nc ? m - nc : m + k * g;
+        if (ci >= nc || (split && k > 0)) continue;
+        const int j = c0 + ci;
+        GP<T> qj = qd + (long) j * nx;
+        T v[V];
+        if (P.affine) {
+            CP<T> pe = tab(P.Pe, j);
+            loadV(v, nx, row, [&](unsigned k) -> T { return qj[k] + pe[k]; });
+        } else {
+            loadPtr(v, qj, nx, row);
+        }
+        if (m < nc || !split) {
+            zero(w);
+            mvAcc(w, tab(P.BTr, j), nu, nu, nx, v);
+            lds->bq[w0 + m][k][row] = w[0];
+        }
+        if (stage > 0 && (m >= nc || !split)) {
+            mvAcc(rq[k], tab(P.ABKTr, j), nx, nx, nx, v);
+            if (split) {
+#pragma unroll
+                for (int rc = 0; rc < R; rc++) lds->xq[w0 + m][0][row + 64 * rc] = rq[k][rc];
+            }
+        }
+    }
+    __syncthreads();
+    T d = T(0);
+    if (i >= 0 && !(split && stage > 0 && m >= nc && m > 2 * nc)) {
+        T acc = T(0);
+        for (int ci = 0; ci < nc; ci++) {
+            const T b = lds->bq[w0 + ci % g][ci / g][row];
+            acc = ci == 0 ? b : acc + b;
+        }
+        d = mine ? (-acc + ub) : T(0);
+        if (P.dynInverse) {
+            T dvin[V], dout[R];
+            zero(dvin);
+            dvin[0] = d;
+            zero(dout);
+            mvAcc(dout, tab(P.RtInv, i), nu, nu, nu, dvin);
+            d = mine ? dout[0] : T(0);
+        } else {
+            CP<T> L = tab(P.cholL, i);
+            for (int k = 0; k < nu; k++) {
+                const T dk = bcastLane(d, laneOf(k)) / L[k + (size_t) k * nu];
+                if ((int) row == k) d = dk;
+                else if ((int) row > k && mine) d -= L[row + (size_t) k * nu] * dk;
+            }
+            CP<T> U = tab(P.cholU, i);
+            for (int k = nu - 1; k >= 0; k--) {
+                const T dk = bcastLane(d, laneOf(k)) / U[k + (size_t) k * nu];
+                if ((int) row == k) d = dk;
+                else if ((int) row < k) d -= U[row + (size_t) k * nu] * dk;
+            }
+        }
+        if (m == 0 && mine) ((GP<T>) P.dd + (long) i * nu)[row] = d;
+    }
+    if (stage == 0) return;
+    T dv[V];
+    zero(dv);
+    dv[0] = d;
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const int ci = m + k * g;
+        if (ci >= nc) continue;
+        zero(w);
+        mvAcc(w, tab(P.APB, c0 + ci), nx, nx, nu, dv);
+#pragma unroll
+        for (int rc = 0; rc < R; rc++) lds->xq[w0 + m][k][row + 64 * rc] = w[rc] + rq[k][rc];
+    }
+    // the member that finishes the node: one without children if there is one
+    const int last = split ? min(2 * nc, g - 1) : nc < g ? nc : 0;
+    zero(w);
+    if (i >= 0 && m == last) {
+        dv[0] = mine ? d - ub : T(0);
+        mvAcc(w, tab(P.KTr, i), nx, nx, nu, dv);
+    }
+    __syncthreads();
+    if (i >= 0 && m == last) {
+        GP<T> xbar = cand + (P.oX + (long) i * nx);
+        eachRow<R>(nx, row, [&](int rc, unsigned r) {
+            T acc = T(0);
+            for (int ci = 0; ci < nc; ci++) {
+                T x = lds->xq[w0 + ci % g][ci / g][r];
+                if (split) x += lds->xq[w0 + nc + ci][0][r];
+                acc = ci == 0 ? x : acc + x;
+            }
+            (qd + (long) i * nx)[r] = (acc + w[rc]) - xbar[r];
+        });
+    }
+}
+
 // Dynamics projection + kernel projection on cand (in place).  The kernel projection touches
 // (y, t, s) only, so it shares the first backward stage's barrier interval.
 template <typename T, int R, int V>
@@ -991,19 +1121,31 @@ __device__ __noinline__ void phaseProjections(const Inst<T> *Pp, int grid, T *ca
     IP<T> P = *cst(uniformPtr(Pp));
     const Tc c = threadCtx(grid);
     GP<T> cand = glb(candIn);
+    __shared__ TeamLds<T, R> teamLds;
+    SPK_LDS TeamLds<T, R> *team = (SPK_LDS TeamLds<T, R> *) &teamLds;
     if (doDyn) {
         for (int stage = P.S - 2; stage >= 0; stage--) {
             const int f = cst(P.stageFrom)[stage], nStage = cst(P.stageTo)[stage] - f + 1;
             const int extra = (doKernel && stage == P.S - 2) ? P.nl : 0;
-            for (int task = c.wave; task < nStage + extra; task += c.nw) {
-                if (task < nStage) dynBackwardNode<T, R, V>(P, cand, f + task, stage, c.row);
-                else kernelNode<T, R, V>(P, cand, task - nStage, c.row);
+            const int g = teamSize<R>(c, nStage, P.E);
+            if (g > 1) {
+                const int m = c.lw % g, w0 = c.lw - m, node = c.wave / g;
+                if ((c.wave - c.lw) / g < nStage)
+                    dynBackwardTeam<T, R, V>(P, cand, node < nStage ? f + node : -1, stage, c.row, m, g, w0, team);
+                for (int task = c.wave; task < extra; task += c.nw) kernelNode<T, R, V>(P, cand, task, c.row);
+            } else {
+                for (int task = c.wave; task < nStage + extra; task += c.nw) {
+                    if (task < nStage) dynBackwardNode<T, R, V>(P, cand, f + task, stage, c.row);
+                    else kernelNode<T, R, V>(P, cand, task - nStage, c.row);
+                }
             }
             sync(c);
         }
         for (int stage = 0; stage <= P.S - 2; stage++) {
             const int f = cst(P.stageFrom)[stage], nStage = cst(P.stageTo)[stage] - f + 1;
-            for (int task = c.wave; task < nStage; task += c.nw) dynForwardNode<T, R, V>(P, cand, f + task, c.row);
+            const int g = teamSize<R>(c, nStage, 0);
+            for (int task = c.wave / g; task < nStage; task += c.nw / g)
+                dynForwardNode<T, R, V>(P, cand, f + task, c.row, c.lw % g, g);
             sync(c);
         }
     } else if (doKernel) {
