@@ -340,6 +340,18 @@ double tolScaleOf(const HostProblem &h) {
     return h.precond ? *std::min_element(h.scaling.begin(), h.scaling.end()) : 1.;
 }
 
+// The first stage from which on the tree does not branch: node k of each later nonleaf stage is the only child
+// of node k of the stage before.
+int chainStage(const HostProblem &h) {
+    for (int s = h.S - 2; s > 0; s--) {
+        const int f = h.stageFrom[s - 1], n = h.stageTo[s - 1] - f + 1;
+        if (h.stageTo[s] - h.stageFrom[s] + 1 != n) return s;
+        for (int k = 0; k < n; k++)
+            if (h.numCh[f + k] != 1 || h.chFrom[f + k] != h.stageFrom[s] + k) return s;
+    }
+    return 0;
+}
+
 // The instance descriptors of a per-instance solve in b->hInst: Anderson rings of instance k at
 // anders + andOff[k], grid-mode partials at gpart.
 template <typename T>
@@ -396,6 +408,7 @@ void fillInsts(spk_batch *b, const spk_options &o, int warm, T *anders, const st
         I.maxTicks = o.max_time_secs > 0 ? o.max_time_secs * b->ctx->tickRateHz : 0.;
         I.gpart = gpart;
         I.gbar = static_cast<unsigned *>(b->gbar.p);
+        I.chain = b->count == 1 && b->wgs > 1 ? chainStage(b->probs[k]->hp) : b->probs[k]->hp.S - 2;
         I.slot = k;
         if (b->dbgCap > 0) {
             I.dbg = static_cast<double *>(b->dbgRec.p) + (size_t) k * b->dbgCap * spk::DBG_WORDS;

@@ -77,6 +77,7 @@ struct Inst {
     int maxInner, andBuff, checkPeriod, method, warm, lsMethod, dynInverse;
     double maxTicks;  // wall-clock cap in device ticks (0 = none)
     T *gpart;         // grid mode: 2 x GRID_MAXK x GRID_MAXWG reduction partials
+    int chain;        // grid mode: from this stage on node k of a stage is the only child of node k of the one before
     unsigned *gbar;   // grid mode: the barrier's GRID_BAR_WORDS words, zero before the first launch
     // debug trace (enableDebug, src/cache.cuh:947-959); dbg == nullptr: off.  One record of
     // DBG_WORDS doubles per error check, at most dbgCap; dbgE (sPrim) carries err0's running
