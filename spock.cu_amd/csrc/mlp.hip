@@ -987,7 +987,7 @@ long spk_mlp_num_params(const spk_mlp *m) { return m ? m->nParams : -1; }
 int spk_mlp_get_params(spk_mlp *m, float *p) {
     try {
         check(hipStreamSynchronize(m->ctx->stream), "sync");
-        check(hipMemcpy(p, m->w.p, m->nParams * 4, hipMemcpyDeviceToHost), "params");
+        spk::readBack(m->ctx, p, m->w.as<float>(), m->nParams);
         return 0;
     } catch (const std::exception &e) {
         return fail(m->ctx, e);
@@ -1009,7 +1009,7 @@ int spk_mlp_set_params(spk_mlp *m, const float *p) {
 int spk_mlp_get_grads(spk_mlp *m, float *p) {
     try {
         check(hipStreamSynchronize(m->ctx->stream), "sync");
-        check(hipMemcpy(p, m->g.p, m->nParams * 4, hipMemcpyDeviceToHost), "grads");
+        spk::readBack(m->ctx, p, m->g.as<float>(), m->nParams);
         return 0;
     } catch (const std::exception &e) {
         return fail(m->ctx, e);
