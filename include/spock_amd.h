@@ -76,7 +76,7 @@ typedef struct spk_options {
     int check_period;
     int method;
     int block_size;  /* threads per workgroup; 0 (default): for per-instance batches the size chosen by
-                        spk_batch_autotune_uneven, else 512 (256 in grid mode); for shared batches the
+                        spk_batch_autotune_uneven, else 512 (256 in grid mode up to 16 nodes a workgroup); for shared batches the
                         size chosen by spk_batch_autotune, else 1024 */
     int ls_method;   /* enum spk_ls_method */
     int dyn_inverse; /* 1: apply (L L')^-1 as one matvec; 0: two triangular solves as the reference */

@@ -574,13 +574,26 @@ void launchKernel(spk_batch *b, int bs, bool debug, int op, const void *insDev =
     }
 }
 
-// Threads per workgroup of a per-instance solve: the option, else the autotuned size, else 512
-// (one workgroup per instance) or 256 (grid mode).  Measured on the 229-node problem (FP64, one
-// instance): 7.3 ms per outer iteration with 512 threads against 11.4 with 256; in grid mode with
-// 64 workgroups 1.6 ms with 256 against 1.9 with 512.
+// Grid mode: 512 threads where 256 would leave each wave more than 4 nodes and a compute unit takes one such
+// workgroup each.  Milliseconds with 256 / 512 threads by nodes per wave (256): 229 nodes FP64, 50 iterations, 2, 8,
+// 32, 64 workgroups (29, 7, 1.8, 0.9 nodes) 60 / 41, 20.4 / 18.6, 12.1 / 12.2, 11.6 / 13.0; 341 nodes, 15 iterations, 4, 32,
+// 128 workgroups (21, 2.7, 0.7) 51 / 42, 10.6 / 11.2, 7.4 / 9.1; 1,365 nodes FP32, 8 and 64 workgroups (43, 5.3) 21.4 / 14.1,
+// 4.0 / 3.2.
+bool manyNodesPerWave(const spk_batch *b) {
+    if (b->probs[0]->hp.N <= 16 * b->wgs) return false;
+    int cus = 0;
+    check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->ctx->device), "device attribute");
+    return b->wgs <= cus;
+}
+
+// Threads per workgroup of a per-instance solve: the option, else the autotuned size, else 512 (in grid mode 256
+// or 512).  Measured on the 229-node problem (FP64, one instance and workgroup, the matrix-vector products lane per
+// row): 7.3 ms per outer iteration with 512 threads against 11.4 with 256.
 int solveBlock(const spk_options &o, const spk_batch *b = nullptr) {
     const bool grid = b && b->count == 1 && b->wgs > 1;
-    const int bs = o.block_size > 0 ? o.block_size : (b && b->fusedBlock > 0 ? b->fusedBlock : (grid ? 256 : 512));
+    const int bs = o.block_size > 0 ? o.block_size
+        : b && b->fusedBlock > 0    ? b->fusedBlock
+        : grid && !manyNodesPerWave(b) ? 256 : 512;
     return std::max(64, std::min(512, bs / 64 * 64));
 }
 
