@@ -1049,6 +1049,10 @@ void gatherLanes(spk_batch *b, int count, T *dst, long ld) {
 // one (256 FP32 instances, solved and read back: 12.0 ms a pass, now 10.3).
 template <typename T>
 void readIterates(spk_batch *b, double *z) {
+    if (b->count == 1) {
+        spk::readBack(b->ctx, z, static_cast<const T *>(corePtr<T>(b, 0)), (size_t) b->probs[0]->hp.sIter);
+        return;
+    }
     std::vector<long> idx(2 * b->count + 1);
     long *from = idx.data(), *at = from + b->count;
     at[0] = 0;

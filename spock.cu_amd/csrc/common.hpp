@@ -140,9 +140,15 @@ void readBack(spk_ctx *c, D *dst, size_t n, F put) {
     end(pieces);
 }
 
-// The same from one device array.
+// The same from one device array; a small one needs no pinned memory.
 template <typename S, typename D>
 void readBack(spk_ctx *c, D *dst, const S *src, size_t n) {
+    if (n * sizeof(S) <= STAGE_BYTES / 4) {
+        std::vector<S> tmp(n);
+        check(hipMemcpy(tmp.data(), src, n * sizeof(S), hipMemcpyDeviceToHost), "read back");
+        std::copy(tmp.begin(), tmp.end(), dst);
+        return;
+    }
     readBack<S>(c, dst, n, [&](size_t first, size_t count, S *to) {
         check(hipMemcpyAsync(to, src + first, count * sizeof(S), hipMemcpyDeviceToHost, c->stream), "read back");
     });
