@@ -2,6 +2,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "gridbar.hpp"
+
 namespace spk {
 
 // Per-node factor table on the device: entry for node n starts at data + idx[n] * rows * cols (tab()).
@@ -94,11 +96,7 @@ constexpr int DBG_WORDS = 6;
 // Grid mode limits: values per grid reduction and workgroups per cooperative launch.
 constexpr int GRID_MAXK = 16;
 constexpr int GRID_MAXWG = 1024;
-// The grid barrier: a counter for each of up to GRID_GROUPS groups of workgroups, one for the groups and a
-// release flag for each group, every one in a 256-byte piece of its own.
-constexpr int GRID_GROUPS = 8;
-constexpr int GRID_BAR_STEP = 64;
-constexpr int GRID_BAR_WORDS = GRID_BAR_STEP * (2 * GRID_GROUPS + 1);
+static_assert(GRID_MAXWG / GRID_GROUPS < GRID_BAR_ROUND, "arrivals at one counter of the grid barrier");
 
 // Block-interleaved layout of a region of `rows` rows: instances are grouped in blocks of w (64
 // for the lane engine, 16 for the tile engine) and each block stores rows x w words contiguously,

@@ -107,19 +107,33 @@ __device__ __forceinline__ SPK_LDS GridBar *gridBar() {
     return (SPK_LDS GridBar *) &bar;
 }
 
-__device__ __forceinline__ unsigned *gridFlag(unsigned *mem, unsigned group) {
-    return mem + GRID_BAR_STEP * (GRID_GROUPS + 1 + group);
-}
+// Memory of the grid barrier (gridbar.hpp) on the device.  Relaxed accesses at agent scope act in the coherent
+// memory behind the XCDs' L2 caches; the fences write back and drop what a workgroup's caches hold.
+struct GridMem {
+    unsigned *words;
+    __device__ __forceinline__ unsigned add(unsigned w, unsigned k) {
+        return __hip_atomic_fetch_add(words + w, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + k;
+    }
+    __device__ __forceinline__ unsigned load(unsigned w) {
+        return __hip_atomic_load(words + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ void store(unsigned w, unsigned v) {
+        __hip_atomic_store(words + w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ void pause() { __builtin_amdgcn_s_sleep(1); }
+    __device__ __forceinline__ void release() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent"); }
+    __device__ __forceinline__ void acqRel() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent"); }
+    __device__ __forceinline__ void acquire() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
+};
 
 // Before a kernel's first barrier or reduction.
 __device__ __forceinline__ void startGrid(const Tc &c, unsigned *gbar) {
     if (c.ltid == 0) {
         *gridSeq() = 0;
         if (c.grid) {
+            GridMem mem{gbar};
             gridBar()->mem = (unsigned long long) gbar;
-            // no flag moves before this workgroup has arrived for the first time
-            gridBar()->passed = __hip_atomic_load(gridFlag(gbar, blockIdx.x % GRID_GROUPS), __ATOMIC_RELAXED,
-                                                  __HIP_MEMORY_SCOPE_AGENT);
+            gridBar()->passed = gridPassed(mem, blockIdx.x);
         }
     }
     __syncthreads();
@@ -129,35 +143,17 @@ __device__ __forceinline__ void startGrid(const Tc &c, unsigned *gbar) {
 // microseconds of work between two of them, so this is most of a large tree's time.  What bounds it are the trips
 // to memory and the accesses to one address, one after the other; workgroups therefore arrive in groups (by
 // index, so mostly of one XCD), the last of each group arrives at the root, and each group waits on a flag of
-// its own.  Counters are back at zero behind every barrier.  With 1,024 words written by each workgroup and
-// read by another: 32 / 128 / 256 workgroups 3.0 / 4.7 / 8.1 us; one counter that all add to and poll 2.7 / 7.2 /
-// 13.7; cooperative_groups' grid barrier 5.6 / 15.8 / 29.2.
+// its own.  With 1,024 words written by each workgroup and read by another: 32 / 128 / 256 workgroups 3.3 / 4.8 /
+// 7.9 us, 0.13 of them the fence at a group's last arrival; one counter that all add to and poll 2.7 / 7.2 / 13.7;
+// cooperative_groups' grid barrier 5.6 / 15.8 / 29.2.
 __device__ __noinline__ void gridBarrier() {
     // every wave's writes have left before the workgroup's first thread releases them to the other XCDs
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_s_waitcnt(0);
     __builtin_amdgcn_s_barrier();
     if (threadIdx.x == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        unsigned *mem = reinterpret_cast<unsigned *>(gridBar()->mem);
-        const unsigned next = gridBar()->passed + 1, n = gridDim.x, group = blockIdx.x % GRID_GROUPS;
-        const unsigned size = (n - group + GRID_GROUPS - 1) / GRID_GROUPS, groups = n < GRID_GROUPS ? n : GRID_GROUPS;
-        unsigned *count = mem + GRID_BAR_STEP * (1 + group), *flag = gridFlag(mem, group);
-        // Each workgroup has written its data back before it arrives and drops its caches after its flag, so what lies
-        // between only has to happen in order: every step waits for the value of the one before.
-        if (__hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == size) {
-            __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (__hip_atomic_fetch_add(mem, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == groups) {
-                __hip_atomic_store(mem, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                // the counters are at zero before anyone can arrive again
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent");
-                for (unsigned q = 0; q < groups; q++)
-                    __hip_atomic_store(gridFlag(mem, q), next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
-        while (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != next) __builtin_amdgcn_s_sleep(1);
-        gridBar()->passed = next;
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        GridMem mem{reinterpret_cast<unsigned *>(gridBar()->mem)};
+        gridBar()->passed = gridPass(mem, blockIdx.x, gridDim.x, gridBar()->passed);
     }
     __syncthreads();
 }
