@@ -41,7 +41,9 @@ SPK_BAR unsigned gridPassed(Mem &m, unsigned wg) {
 
 // The barrier behind release value `passed`, by workgroup wg of n; returns its own release value.  Workgroups
 // arrive in groups, the last of each group at the root, and the last there releases the flags.  Each of
-// them passes on what it has seen by a fence between the atomic it read and the one it writes.
+// them passes on what it has seen by a fence between the atomic it read and the one it writes.  All
+// flags move, also those of groups without a workgroup: a later launch of more workgroups starts from them, and
+// its groups have to agree on the next release value.
 template <typename Mem>
 SPK_BAR unsigned gridPass(Mem &m, unsigned wg, unsigned n, unsigned passed) {
     const unsigned next = passed + 1, group = wg % GRID_GROUPS;
@@ -51,7 +53,7 @@ SPK_BAR unsigned gridPass(Mem &m, unsigned wg, unsigned n, unsigned passed) {
         m.acqRel();
         if (m.add(GRID_BAR_ROOT, group == 0 ? GRID_BAR_ROUND - (groups - 1) : 1) % GRID_BAR_ROUND == 0) {
             m.acqRel();
-            for (unsigned q = 0; q < groups; q++) m.store(gridFlag(q), next);
+            for (unsigned q = 0; q < GRID_GROUPS; q++) m.store(gridFlag(q), next);
         }
     }
     while (m.load(gridFlag(group)) != next) m.pause();

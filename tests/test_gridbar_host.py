@@ -182,3 +182,13 @@ def test_one_count(model, n, late):
     """Launches of one count: arrivals at a barrier are not lost to stores of the one before."""
     for seed in range(20 if n < 30 else 3):
         run(model, seed, late, 6, [n, n])
+
+
+@pytest.mark.parametrize("late", [0, 1])
+@pytest.mark.parametrize("counts", [(4, 32), (32, 4, 32), (2, 3, 8, 256, 7, 9), (1, 5, 2, 64), (3, 9, 2, 32, 1024, 6, 12)],
+                         ids=lambda c: "-".join(map(str, c)))
+def test_counts_change(model, counts, late):
+    """Launches of different counts one after the other, from fewer workgroups than there are groups to more: every
+    workgroup starts from the same release value."""
+    for seed in range(20 if max(counts) < 100 else 1):
+        run(model, seed, late, 3, counts)
