@@ -200,9 +200,10 @@ class Cache {
 public:
     // Iterate sizes for which the automatic choice spreads one instance over kAutoGridWorkgroups
     // cooperating workgroups (grid mode): the range of the 229-node, 52,360-element problem this
-    // has been run and measured on (2.0 ms per outer iteration with 32 workgroups, 2.4 with 64,
-    // 8.9 with one).  Elsewhere one workgroup solves the instance unless workgroups(n) asks
-    // otherwise.
+    // has been run and measured on (first 50 iterations: 0.24 ms each with 32 workgroups, 0.23 with
+    // 64, 0.25 with 128; 1.14 with one over the first 25).  32 take half the compute units of the 5%
+    // faster 64 and leave them to others.  Elsewhere one workgroup solves the instance unless
+    // workgroups(n) asks otherwise.
     static constexpr size_t kAutoGridMin = 50000, kAutoGridMax = 100000;
     static constexpr int kAutoGridWorkgroups = 32;
 

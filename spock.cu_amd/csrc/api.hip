@@ -587,8 +587,8 @@ bool manyNodesPerWave(const spk_batch *b) {
 }
 
 // Threads per workgroup of a per-instance solve: the option, else the autotuned size, else 512 (in grid mode 256
-// or 512).  Measured on the 229-node problem (FP64, one instance and workgroup, the matrix-vector products lane per
-// row): 7.3 ms per outer iteration with 512 threads against 11.4 with 256.
+// or 512).  229-node problem, FP64, one workgroup, first 25 iterations: 1.14 ms each with 512 threads, 1.75 with 256,
+// 3.08 with 128.
 int solveBlock(const spk_options &o, const spk_batch *b = nullptr) {
     const bool grid = b && b->count == 1 && b->wgs > 1;
     const int bs = o.block_size > 0 ? o.block_size
@@ -1046,7 +1046,7 @@ void gatherLanes(spk_batch *b, int count, T *dst, long ld) {
 }
 
 // All accepted iterates of a batch of separate instances, gathered on the device instead of copied one by
-// one (256 FP32 instances, solved and read back: 12.0 ms a pass, now 10.3).
+// one and converted by one thread (256 FP32 instances, solved and read back: 11.8 ms a pass, now 8.1).
 template <typename T>
 void readIterates(spk_batch *b, double *z) {
     if (b->count == 1) {

@@ -1003,7 +1003,8 @@ __device__ __forceinline__ int teamSize(const Tc &c, int nodes, int children) {
 }
 
 // dynBackwardNode by member m of a team of g waves whose first is wave w0 of the workgroup: the same sums in the
-// same order.  With waves to spare (2 nc <= g) member nc + c takes the product with q of child c.  All waves
+// same order up to 64 states (beyond, a wave alone adds APB d to the first 64 columns of ABKTr q and then the others,
+// a team adds the columns first).  With waves to spare (2 nc <= g) member nc + c takes the product with q of child c.  All waves
 // of the workgroup come here together; i < 0: no node.
 template <typename T, int R, int V>
 __device__ __forceinline__ void dynBackwardTeam(IP<T> P, GP<T> cand, int i, int stage, unsigned row, int m, int g, int w0,
@@ -1223,7 +1224,10 @@ __device__ __noinline__ EllSums<T> reduceEllNodes(const Inst<T> *Pp, int grid, T
 
 // -2 gamma sum r_p . (L* r_d): as r_p . (L* r_d) = (L r_p) . r_d, this and |r|^2 (from the residual's
 // pass) make <r, M r>, the squared M-norm that SuperMann needs between the error checks, from one adjoint
-// instead of [L*; L] (229-node FP64 instance in one workgroup: 0.35 -> 0.17 ms an iteration).
+// instead of [L*; L] (229-node FP64 instance in one workgroup: 0.35 -> 0.17 ms an iteration).  No digits cancel:
+// <r, M r> is 0.63 to 1.07 of |r|^2 on residuals of 1 to 512 iterations of nine problems (31 to 229 nodes, 3 to
+// 100 states).  Error in FP32 against 64 bits on these 264: root mean square 5.0e-8, at most 2.0e-7; of [L*; L]
+// 6.5e-8 and 2.1e-7.
 template <typename T, int R, int V>
 __device__ __noinline__ T adjDotNodes(const Inst<T> *Pp, int grid, T *rIn) {
     IP<T> P = *cst(uniformPtr(Pp));
