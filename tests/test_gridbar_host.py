@@ -110,7 +110,14 @@ int main(int argc, char **argv) {
     W = &world;
     world.gen.seed(std::atoi(argv[1]));
     world.late = std::atoi(argv[2]);
-    for (int a = 4; a < argc; a++) {
+    if (std::atoi(argv[4])) {  // counters and flags about to overflow
+        for (unsigned q = 0; q < spk::GRID_GROUPS; q++) {
+            world.words[spk::gridCount(q)] = -spk::GRID_BAR_ROUND;
+            world.words[spk::gridFlag(q)] = -2u;
+        }
+        world.words[spk::GRID_BAR_ROOT] = -spk::GRID_BAR_ROUND;
+    }
+    for (int a = 5; a < argc; a++) {
         const unsigned n = std::atoi(argv[a]);
         const int barriers = std::atoi(argv[3]);
         world.data.assign(n, 0);
@@ -137,7 +144,7 @@ int main(int argc, char **argv) {
             }
             if (all) break;
             if (ready.empty()) {
-                if (holding.empty()) { std::printf("launch %d of %u workgroups never ends\n", a - 4, n); return 1; }
+                if (holding.empty()) { std::printf("launch %d of %u workgroups never ends\n", a - 5, n); return 1; }
                 holding[world.gen() % holding.size()]->landOne();
                 continue;
             }
@@ -170,9 +177,9 @@ def model(tmp_path_factory):
     return str(exe)
 
 
-def run(model, seed, late, barriers, counts):
-    r = subprocess.run([model, str(seed), str(late), str(barriers)] + [str(n) for n in counts], capture_output=True,
-                       text=True, timeout=100)
+def run(model, seed, late, barriers, counts, overflow=0):
+    r = subprocess.run([model, str(seed), str(late), str(barriers), str(overflow)] + [str(n) for n in counts],
+                       capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, (seed, late, counts, r.stdout)
 
 
@@ -192,3 +199,10 @@ def test_counts_change(model, counts, late):
     workgroup starts from the same release value."""
     for seed in range(20 if max(counts) < 100 else 1):
         run(model, seed, late, 3, counts)
+
+
+@pytest.mark.parametrize("late", [0, 1])
+def test_overflow(model, late):
+    """Counters and release values that pass 2^32."""
+    for seed in range(20):
+        run(model, seed, late, 5, (9, 4, 16), overflow=1)
