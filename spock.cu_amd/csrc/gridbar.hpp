@@ -61,4 +61,33 @@ SPK_BAR unsigned gridPass(Mem &m, unsigned wg, unsigned n, unsigned passed) {
     return next;
 }
 
+#if defined(__HIP__)
+// The policy on the device.  Relaxed accesses at agent scope act in the coherent memory behind the XCDs' L2
+// caches; the fences write back and drop what a workgroup's caches hold.  A write-back has to be waited for
+// explicitly: hipcc (ROCm 7.2) drops the wait that belongs to a release fence where no other access is under way, and
+// the next atomic could then overtake it.
+struct GridMem {
+    unsigned *words;
+    __device__ __forceinline__ unsigned add(unsigned w, unsigned k) {
+        return __hip_atomic_fetch_add(words + w, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + k;
+    }
+    __device__ __forceinline__ unsigned load(unsigned w) {
+        return __hip_atomic_load(words + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ void store(unsigned w, unsigned v) {
+        __hip_atomic_store(words + w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ void pause() { __builtin_amdgcn_s_sleep(1); }
+    __device__ __forceinline__ void release() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        __builtin_amdgcn_s_waitcnt(0);
+    }
+    __device__ __forceinline__ void acquire() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
+    __device__ __forceinline__ void acqRel() {
+        release();
+        acquire();
+    }
+};
+#endif
+
 }  // namespace spk

@@ -107,25 +107,6 @@ __device__ __forceinline__ SPK_LDS GridBar *gridBar() {
     return (SPK_LDS GridBar *) &bar;
 }
 
-// Memory of the grid barrier (gridbar.hpp) on the device.  Relaxed accesses at agent scope act in the coherent
-// memory behind the XCDs' L2 caches; the fences write back and drop what a workgroup's caches hold.
-struct GridMem {
-    unsigned *words;
-    __device__ __forceinline__ unsigned add(unsigned w, unsigned k) {
-        return __hip_atomic_fetch_add(words + w, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + k;
-    }
-    __device__ __forceinline__ unsigned load(unsigned w) {
-        return __hip_atomic_load(words + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __device__ __forceinline__ void store(unsigned w, unsigned v) {
-        __hip_atomic_store(words + w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __device__ __forceinline__ void pause() { __builtin_amdgcn_s_sleep(1); }
-    __device__ __forceinline__ void release() { __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent"); }
-    __device__ __forceinline__ void acqRel() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent"); }
-    __device__ __forceinline__ void acquire() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
-};
-
 // Before a kernel's first barrier or reduction.
 __device__ __forceinline__ void startGrid(const Tc &c, unsigned *gbar) {
     if (c.ltid == 0) {
@@ -143,9 +124,8 @@ __device__ __forceinline__ void startGrid(const Tc &c, unsigned *gbar) {
 // microseconds of work between two of them, so this is most of a large tree's time.  What bounds it are the trips
 // to memory and the accesses to one address, one after the other; workgroups therefore arrive in groups (by
 // index, so mostly of one XCD), the last of each group arrives at the root, and each group waits on a flag of
-// its own.  With 1,024 words written by each workgroup and read by another: 32 / 128 / 256 workgroups 3.3 / 4.8 /
-// 7.9 us, 0.13 of them the fence at a group's last arrival; one counter that all add to and poll 2.7 / 7.2 / 13.7;
-// cooperative_groups' grid barrier 5.6 / 15.8 / 29.2.
+// its own.  With 1,024 words written by each workgroup and read by another: 32 / 128 / 256 workgroups 3.4 / 4.9 /
+// 8.5 us; one counter that all add to and poll 2.7 / 7.2 / 13.7; cooperative_groups' grid barrier 5.6 / 15.8 / 29.2.
 __device__ __noinline__ void gridBarrier() {
     // every wave's writes have left before the workgroup's first thread releases them to the other XCDs
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");

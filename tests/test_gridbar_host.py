@@ -8,6 +8,7 @@ other on the same words, as the solves of one batch do, with the counts of workg
 fails a run in which every workgroup waits for good, one in which a workgroup leaves a barrier that
 another has not reached, and one in which it does not see what another wrote before the barrier."""
 import os
+import shutil
 import subprocess
 
 import pytest
@@ -206,3 +207,32 @@ def test_overflow(model, late):
     """Counters and release values that pass 2^32."""
     for seed in range(20):
         run(model, seed, late, 5, (9, 4, 16), overflow=1)
+
+
+DEVICE = r'''
+#include <hip/hip_runtime.h>
+#include "gridbar.hpp"
+__global__ void barrier(unsigned *words, unsigned *out, unsigned passed) {
+    spk::GridMem mem{words};
+    out[blockIdx.x] = spk::gridPass(mem, blockIdx.x, gridDim.x, passed);
+}
+'''
+HIPCC = "/opt/rocm/bin/hipcc"
+
+
+@pytest.mark.skipif(shutil.which(HIPCC) is None, reason="needs hipcc")
+def test_write_backs_are_waited_for(tmp_path):
+    """The compiled barrier waits behind every write-back of the cache, before the atomic or store that announces what
+    was written: the first instruction behind buffer_wbl2 that is not a scalar one is s_waitcnt vmcnt(0)."""
+    src, asm = tmp_path / "b.hip", tmp_path / "b.s"
+    src.write_text(DEVICE)
+    subprocess.run([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++20", "-Xclang", "-target-feature", "-Xclang",
+                    "-packed-fp32-ops", "-I", os.path.join(ROOT, "spock.cu_amd", "csrc"), "--cuda-device-only", "-S", "-o",
+                    str(asm), str(src)], check=True, capture_output=True, timeout=300)
+    lines = [l.split(";")[0].strip() for l in asm.read_text().splitlines()]
+    code = [l for l in lines if l and not l.startswith(".")]
+    backs = [i for i, l in enumerate(code) if l.startswith("buffer_wbl2")]
+    assert len(backs) == 3  # on arrival, at the group's last arrival, at the root's
+    for i in backs:
+        behind = next(l for l in code[i + 1:] if not l.startswith("s_") or l.startswith("s_waitcnt") and "vmcnt(0)" in l)
+        assert behind.startswith("s_waitcnt"), code[i:i + 12]
